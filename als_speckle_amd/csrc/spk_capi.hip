@@ -1758,21 +1758,39 @@ int spk_blur2d(spk_ctx* ctx, const float* in, float* out, int rows, int cols, fl
   return SPK_OK;
 }
 
+namespace {
+// PRTF (kind 0) or stack RFTF (kind 1) through the row transforms of the
+// estimates and one summing column pass.  The frames are split into groups so
+// that about 1024 workgroups (four per CU) run the column pass; a group keeps
+// at least 4 frames, so that the groups' FP64 sums stay the smaller traffic.
+int tf_stack(spk_plan* p, int kind, const float* stack, int frames, int rows, int cols,
+             const float* goal, float* out) {
+  const size_t nn = (size_t)p->nn();
+  const int want = std::max(1, std::min((frames + 3) / 4, 1024 / p->bands));
+  const int per = (frames + want - 1) / want, groups = (frames + per - 1) / per;
+  const size_t phi_bytes = frames * nn * sizeof(c32);
+  void* scr;
+  int rc = ctx_scratch(p->ctx, phi_bytes + (groups > 1 ? groups * nn * 2 * sizeof(double) : 0),
+                       &scr);
+  if (rc) return rc;
+  c32* phi = (c32*)scr;
+  double* part = (double*)((char*)scr + phi_bytes);
+  hipStream_t st = p->ctx->stream;
+  SPK_HIP(launch_rowfft_embed(p->n, p->tile, p->ept, (const c32*)stack, phi, rows, cols, p->tw,
+                              frames, st));
+  SPK_HIP(launch_tf_stack(p->n, p->tile, p->ept, kind, phi, goal, rows, frames, per, part, out,
+                          p->tw, st));
+  return SPK_OK;
+}
+}  // namespace
+
 int spk_prtf(spk_plan* p, const float* stack, int frames, int rows, int cols, float* out) {
   SPK_REQUIRE(p && stack && out && frames >= 1, SPK_EINVAL, "bad arguments");
   SPK_REQUIRE(rows >= 1 && cols >= 1 && rows <= p->n && cols <= p->n, SPK_EINVAL,
               "estimates larger than the plan's frame");
   int rc = set_device(p->ctx);
   if (rc) return rc;
-  const size_t nn = (size_t)p->nn();
-  void* scr;
-  if ((rc = ctx_scratch(p->ctx, 2 * frames * nn * sizeof(c32), &scr))) return rc;
-  c32* pad = (c32*)scr;
-  c32* F = pad + frames * nn;
-  SPK_HIP(launch_embed((const c32*)stack, pad, rows, cols, p->n, frames, p->ctx->stream));
-  if ((rc = spk_fft2(p, (const float*)pad, (float*)F, frames, 0))) return rc;
-  SPK_HIP(launch_prtf(F, frames, p->n, out, p->ctx->stream));
-  return SPK_OK;
+  return tf_stack(p, 0, stack, frames, rows, cols, nullptr, out);
 }
 
 namespace {
@@ -1827,6 +1845,7 @@ int spk_rftf_stack(spk_plan* p, const float* stack, int frames, int rows, int co
               "estimates larger than the goal modulus");
   int rc = set_device(p->ctx);
   if (rc) return rc;
+  if (!ipsf) return tf_stack(p, 1, stack, frames, rows, cols, goal, out);
   const size_t nn = (size_t)p->nn();
   void* scr;
   if ((rc = ctx_scratch(p->ctx, 2 * frames * nn * sizeof(c32), &scr))) return rc;
@@ -1834,7 +1853,7 @@ int spk_rftf_stack(spk_plan* p, const float* stack, int frames, int rows, int co
   c32* F = pad + frames * nn;
   SPK_HIP(launch_embed((const c32*)stack, pad, rows, cols, p->n, frames, p->ctx->stream));
   if ((rc = spk_fft2(p, (const float*)pad, (float*)F, frames, 0))) return rc;
-  if (ipsf && (rc = rftf_blur(p, F, frames, (const c32*)ipsf, 1, pad))) return rc;
+  if ((rc = rftf_blur(p, F, frames, (const c32*)ipsf, 1, pad))) return rc;
   SPK_HIP(launch_rftf_stack(F, goal, frames, p->n, out, p->ctx->stream));
   return SPK_OK;
 }

@@ -246,7 +246,16 @@ hipError_t launch_conv_axis(const float* in, float* out, int rows, int cols, int
 hipError_t launch_abs_c64(const c32* in, float* out, long long n, hipStream_t st);
 hipError_t launch_embed(const c32* in, c32* out, int r, int c, int n, int frames,
                         hipStream_t st);
-hipError_t launch_prtf(const c32* F, int frames, int n, float* out, hipStream_t st);
+// row transforms of (rows, cols) estimates zero-padded top-left into n x n
+// (bands of rows past the estimate are not written), and the transfer
+// function of their stack (kind 0 PRTF, 1 RFTF) from them: groups of `per`
+// frames summed in FP64 (part: 2 or 1 doubles per pixel and group, not used
+// for one group)
+hipError_t launch_rowfft_embed(int n, int tile, int ept, const c32* in, c32* out, int rows,
+                               int cols, const c32* tw, int frames, hipStream_t st);
+hipError_t launch_tf_stack(int n, int tile, int ept, int kind, const c32* phi, const float* goal,
+                           int rows, int frames, int per, double* part, float* out,
+                           const c32* tw, hipStream_t st);
 hipError_t launch_rftf_stack(const c32* F, const float* goal, int frames, int n, float* out,
                              hipStream_t st);
 hipError_t launch_rftf(const c32* F, const float* goal, int n, double* partial, int nblk,
