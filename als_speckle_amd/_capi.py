@@ -69,6 +69,7 @@ SIGNATURES = {
     "spk_iterate": (c_int, [c_void_p, POINTER(SpkStep), c_int, c_int, c_void_p]),
     "spk_shrinkwrap": (c_int, [c_void_p, c_int, c_float, c_float]),
     "spk_copy_roi": (c_int, [c_void_p, c_int, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int]),
+    "spk_copy_roi_all": (c_int, [c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int]),
     "spk_fft2": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int]),
     "spk_align_global_phase": (c_int, [c_void_p, c_void_p, c_int, c_int, c_int]),
     "spk_align_global_phase_noalloc": (c_int, [c_void_p, c_void_p, c_int, c_int, c_int]),

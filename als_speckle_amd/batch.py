@@ -107,8 +107,7 @@ class phasing_batch:
         """(trials, rows, cols) device tensor of every trial's ROI (the savebuffer)."""
         buf = torch.empty((self.trials, self.rows, self.cols), dtype=torch.complex64,
                           device=self.ctx.device)
-        for t in range(self.trials):
-            self._plan.copy_roi(t, buf, t, self.r0, self.c0, self.rows, self.cols)
+        self._plan.copy_roi_all(buf, 0, self.r0, self.c0, self.rows, self.cols)
         return buf
 
     def aligned_average(self):

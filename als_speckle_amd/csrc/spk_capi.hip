@@ -1601,22 +1601,34 @@ int spk_shrinkwrap(spk_plan* p, int frame, float sigma, float tau) {
   return do_shrinkwrap(p, f0, nf, sigma, tau);
 }
 
-int spk_copy_roi(spk_plan* p, int frame, float* dst, int slots, int slot, int r0, int c0,
-                 int rows, int cols) {
-  SPK_REQUIRE(p && dst, SPK_EINVAL, "null plan or destination");
+// frames [f0, f0 + nf) into savebuffer slots [slot, slot + nf)
+static int copy_roi_frames(spk_plan* p, int f0, int nf, float* dst, int slots, int slot, int r0,
+                           int c0, int rows, int cols) {
   int rc = set_device(p->ctx);
   if (rc) return rc;
-  SPK_REQUIRE(frame >= 0 && frame < p->batch, SPK_EINVAL, "frame out of range");
-  SPK_REQUIRE(slot >= 0 && slot < slots, SPK_EINVAL,
-              "savebuffer slot " + std::to_string(slot) + " out of range [0, " +
+  SPK_REQUIRE(f0 >= 0 && f0 < p->batch, SPK_EINVAL, "frame out of range");
+  SPK_REQUIRE(slot >= 0 && slot <= slots - nf, SPK_EINVAL,
+              "savebuffer slot " + std::to_string(slot + nf - 1) + " out of range [0, " +
                   std::to_string(slots) + ")");
   SPK_REQUIRE(rows > 0 && cols > 0 && r0 >= 0 && c0 >= 0 && r0 + rows <= p->n &&
                   c0 + cols <= p->n,
               SPK_EINVAL, "ROI outside the frame");
   c32* d = (c32*)dst + (size_t)slot * rows * cols;
-  SPK_HIP(launch_copy_roi(p->n, p->tile, p->psi + (size_t)frame * p->nn(), d, r0, c0, rows,
-                          cols, p->ctx->stream));
+  SPK_HIP(launch_copy_roi(p->n, p->tile, p->psi + (size_t)f0 * p->nn(), d, r0, c0, rows, cols, nf,
+                          p->ctx->stream));
   return SPK_OK;
+}
+
+int spk_copy_roi(spk_plan* p, int frame, float* dst, int slots, int slot, int r0, int c0,
+                 int rows, int cols) {
+  SPK_REQUIRE(p && dst, SPK_EINVAL, "null plan or destination");
+  return copy_roi_frames(p, frame, 1, dst, slots, slot, r0, c0, rows, cols);
+}
+
+int spk_copy_roi_all(spk_plan* p, float* dst, int slots, int slot, int r0, int c0, int rows,
+                     int cols) {
+  SPK_REQUIRE(p && dst, SPK_EINVAL, "null plan or destination");
+  return copy_roi_frames(p, 0, p->batch, dst, slots, slot, r0, c0, rows, cols);
 }
 
 int spk_fft2(spk_plan* p, const float* in, float* out, int count, int inverse) {

@@ -233,7 +233,8 @@ hipError_t launch_shrinkwrap(int n, int tile, const c32* psi, float* sup,
                              const int* fmap, int frame0, int frames, int rmax,
                              hipStream_t st);
 hipError_t launch_copy_roi(int n, int tile, const c32* psi, c32* dst, int r0,
-                           int c0, int rows, int cols, hipStream_t st);
+                           int c0, int rows, int cols, int frames, hipStream_t st);
+// nblk <= 64
 hipError_t launch_align(c32* data, int frames, long long per_frame,
                         double* partial, int nblk, hipStream_t st);
 hipError_t launch_stack_mean(const c32* data, long long per_frame, int frames,

@@ -1828,7 +1828,10 @@ static __global__ void __launch_bounds__(256) k_sw_threshold(float* sup, long lo
 }
 
 // ---------------------------------------------------------------------------
-// ROI copy (phasing_copy_to_buffer_f2.cl:6-19): dst[j*cols + i] = psi[r0+j, c0+i]
+// ROI copy (phasing_copy_to_buffer_f2.cl:6-19): dst[f][j*cols + i] =
+// psi_f[r0+j, c0+i], grid (pixels / 256, frames).  All frames of a plan go in
+// one launch: 64 trials of a 187^2 region took 64 launches of 3.2 us (4.5 us
+// apart), 206 us of kernels; one takes 13 us.
 // ---------------------------------------------------------------------------
 template <int TT>
 __global__ void __launch_bounds__(256) k_copy_roi(const c32* psi, c32* dst, int n, int r0,
@@ -1836,16 +1839,18 @@ __global__ void __launch_bounds__(256) k_copy_roi(const c32* psi, c32* dst, int 
   const int k = blockIdx.x * 256 + threadIdx.x;
   if (k >= rows * cols) return;
   const int j = k / cols, i = k % cols;
-  dst[k] = psi[tpos<TT>(n, r0 + j, c0 + i)];
+  dst[(size_t)blockIdx.y * rows * cols + k] =
+      psi[(size_t)blockIdx.y * n * n + tpos<TT>(n, r0 + j, c0 + i)];
 }
 
 // ---------------------------------------------------------------------------
 // align_global_phase, closed form (phasing.py:1355-1404): per frame the five
 // FP64 sums (Re^2, Im^2, Re*Im, Re, Im), then rotate by +-exp(i p*).
+// The five block sums go through one reduction (the order of block_sum each).
 // ---------------------------------------------------------------------------
 static __global__ void __launch_bounds__(256) k_align_partial(const c32* data, long long per_frame,
                                                        double* partial, int nblk) {
-  __shared__ double sh[256];
+  __shared__ double sh[5][4];
   const c32* d = data + (size_t)blockIdx.y * per_frame;
   double s[5] = {0, 0, 0, 0, 0};
   for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < per_frame;
@@ -1857,34 +1862,58 @@ static __global__ void __launch_bounds__(256) k_align_partial(const c32* data, l
     s[3] += re;
     s[4] += im;
   }
-  for (int q = 0; q < 5; ++q) {
-    const double v = block_sum(s[q], sh);
-    if (threadIdx.x == 0) partial[((size_t)blockIdx.y * 5 + q) * nblk + blockIdx.x] = v;
-    __syncthreads();
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) {
+#pragma unroll
+    for (int q = 0; q < 5; ++q) s[q] += __shfl_xor(s[q], o, 64);
+  }
+  if ((threadIdx.x & 63) == 0) {
+#pragma unroll
+    for (int q = 0; q < 5; ++q) sh[q][threadIdx.x >> 6] = s[q];
+  }
+  __syncthreads();
+  if (threadIdx.x < 5) {
+    const int q = threadIdx.x;
+    double v = 0.0;
+    for (int w = 0; w < 4; ++w) v += sh[q][w];
+    partial[((size_t)blockIdx.y * 5 + q) * nblk + blockIdx.x] = v;
   }
 }
 
+// Each block reduces the frame's partial sums through LDS, one thread per
+// sum, and one thread takes the angle.  With every thread summing all 5 x 64
+// partials from global memory itself this kernel took 127 us for 64 frames of
+// 187^2; now 16 us.
 static __global__ void __launch_bounds__(256) k_align_apply(c32* data, long long per_frame,
                                                      const double* partial, int nblk) {
+  __shared__ double pp[5 * 64];   // nblk <= 64
+  __shared__ double sum[5];
+  __shared__ float rot[2];
   const int f = blockIdx.y;
-  const double* pp = partial + (size_t)f * 5 * nblk;
-  const double a = kahan_sum(pp, nblk), bb = kahan_sum(pp + nblk, nblk);
-  const double c = kahan_sum(pp + 2 * nblk, nblk);
-  const double sre = kahan_sum(pp + 3 * nblk, nblk), sim = kahan_sum(pp + 4 * nblk, nblk);
-  // e(p) = (a+b)/2 + (b-a)/2 cos 2p + c sin 2p is smallest at
-  // 2p = atan2(c, (b-a)/2) + pi
-  const double p = 0.5 * (atan2(c, 0.5 * (bb - a)) + M_PI);
-  double cr = cos(p), ci = sin(p);
-  // sign rule of phasing.py:1396-1399: negate when sum Re(z e^{ip}) < 0
-  if (cr * sre - ci * sim < 0.0) {
-    cr = -cr;
-    ci = -ci;
+  for (int i = threadIdx.x; i < 5 * nblk; i += 256) pp[i] = partial[(size_t)f * 5 * nblk + i];
+  __syncthreads();
+  if (threadIdx.x < 5) sum[threadIdx.x] = kahan_sum(pp + threadIdx.x * nblk, nblk);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    const double a = sum[0], bb = sum[1], c = sum[2], sre = sum[3], sim = sum[4];
+    // e(p) = (a+b)/2 + (b-a)/2 cos 2p + c sin 2p is smallest at
+    // 2p = atan2(c, (b-a)/2) + pi
+    const double p = 0.5 * (atan2(c, 0.5 * (bb - a)) + M_PI);
+    double cr = cos(p), ci = sin(p);
+    // sign rule of phasing.py:1396-1399: negate when sum Re(z e^{ip}) < 0
+    if (cr * sre - ci * sim < 0.0) {
+      cr = -cr;
+      ci = -ci;
+    }
+    rot[0] = (float)cr;
+    rot[1] = (float)ci;
   }
-  const float fr = (float)cr, fi = (float)ci;
+  __syncthreads();
+  const c32 w{rot[0], rot[1]};
   c32* d = data + (size_t)f * per_frame;
   for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < per_frame;
        i += (long long)gridDim.x * 256) {
-    d[i] = mul(d[i], c32{fr, fi});
+    d[i] = mul(d[i], w);
   }
 }
 
@@ -2304,6 +2333,7 @@ static __global__ void __launch_bounds__(256) k_stack_mean(const c32* data, long
   for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < per_frame;
        i += (long long)gridDim.x * 256) {
     double re = 0.0, im = 0.0;
+#pragma unroll 8   // eight frames' loads in flight (17 -> 6 us for 64 x 187^2)
     for (int f = 0; f < frames; ++f) {
       const c32 v = data[(size_t)f * per_frame + i];
       re += v.x;
@@ -3010,9 +3040,9 @@ hipError_t launch_err_finalize(const double* errp, int nsteps, int frames, int b
 }
 
 hipError_t launch_copy_roi(int n, int tile, const c32* psi, c32* dst, int r0, int c0,
-                           int rows, int cols, hipStream_t st) {
+                           int rows, int cols, int frames, hipStream_t st) {
   const int total = rows * cols;
-  dim3 grid((total + 255) / 256);
+  dim3 grid((total + 255) / 256, frames);
   if (tile == 8)
     hipLaunchKernelGGL(k_copy_roi<8>, grid, dim3(256), 0, st, psi, dst, n, r0, c0, rows, cols);
   else if (tile == 2)
@@ -3026,7 +3056,9 @@ hipError_t launch_align(c32* data, int frames, long long per_frame, double* part
                         int nblk, hipStream_t st) {
   hipLaunchKernelGGL(k_align_partial, dim3(nblk, frames), dim3(256), 0, st, data, per_frame,
                      partial, nblk);
-  hipLaunchKernelGGL(k_align_apply, dim3(nblk, frames), dim3(256), 0, st, data, per_frame,
+  // about eight values per thread: each block first forms the frame's angle
+  const unsigned blocks = (unsigned)std::min<long long>(nblk, (per_frame + 2047) / 2048);
+  hipLaunchKernelGGL(k_align_apply, dim3(blocks, frames), dim3(256), 0, st, data, per_frame,
                      partial, nblk);
   return hipGetLastError();
 }

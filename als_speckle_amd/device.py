@@ -238,6 +238,15 @@ class Plan:
         check(self.lib.spk_copy_roi(self.handle, frame, _ptr(dst), dst.shape[0], slot,
                                     r0, c0, rows, cols))
 
+    def copy_roi_all(self, dst: torch.Tensor, slot: int, r0: int, c0: int,
+                     rows: int, cols: int) -> None:
+        """Every frame's ROI into slots slot, slot + 1, ... in one launch."""
+        if dst.dim() != 3 or tuple(dst.shape[1:]) != (rows, cols):
+            raise ValueError("dst must be (slots, rows, cols)")
+        _expect(dst, torch.complex64, tuple(dst.shape), self.ctx.device, "savebuffer")
+        check(self.lib.spk_copy_roi_all(self.handle, _ptr(dst), dst.shape[0], slot,
+                                        r0, c0, rows, cols))
+
     def fft2(self, x: torch.Tensor, inverse: bool = False, out: torch.Tensor | None = None):
         squeeze = x.dim() == 2
         xx = x.unsqueeze(0) if squeeze else x

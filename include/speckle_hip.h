@@ -237,6 +237,10 @@ int spk_shrinkwrap(spk_plan* plan, int frame, float sigma, float tau);
  * reference has none). */
 int spk_copy_roi(spk_plan* plan, int frame, float* dst_c64, int slots,
                  int slot, int r0, int c0, int rows, int cols);
+/* The same for every frame of the plan in one launch: frame f goes to slot
+ * slot + f (slot + batch <= slots).  The reference copies one trial at a time. */
+int spk_copy_roi_all(spk_plan* plan, float* dst_c64, int slots, int slot, int r0,
+                     int c0, int rows, int cols);
 
 /* -------------------------------------------------------------------------
  * HIP graphs.  spk_graph_begin starts stream capture on the plan's stream
