@@ -155,7 +155,10 @@ struct spk_plan {
   // resident single-frame launches (k_resident) and their exchange mode
   int resident = 0;
   int xm = 0;
-  unsigned* rsync = nullptr;   // barrier flags of the resident launches (a line per band)
+  // resident launches: the two exchange buffers of mode 3 (n*n values each),
+  // then the barrier flags (a 128-byte line per band)
+  c32* rll = nullptr;
+  bool rll_fill = true;   // new, or left unread by a launch that gave up
   unsigned polls = 1u << 18;   // polls of a grid-barrier wait before it gives up
   long long res_launches = 0, res_steps = 0;
   long long sw_fused_count = 0, sw_separate_count = 0;
@@ -568,6 +571,8 @@ int spk_plan_bytes(int n, int batch, int shared, int options, size_t* bytes) {
   if ((options & SPK_PB_DM) && (options & SPK_PB_SPECTRUM)) b += 2 * nn * batch * sizeof(float);
   if (options & SPK_PB_TRACE) b += 64 * (size_t)batch * bands * sizeof(double);
   b += 64 * 1024;                                      // step-table staging
+  if (batch == 1 && resident_supported(n, default_tile(n), default_ept(n, default_tile(n), 1)))
+    b += 2 * nn * sizeof(c32) + bands * 128;           // resident launches' exchange
   *bytes = b;
   return SPK_OK;
 }
@@ -598,13 +603,13 @@ int spk_plan_create(spk_ctx* ctx, int n, int batch, int shared, const spk_tune* 
   p->bands = n / tile;
   p->persist = (tune && tune->persist > 0) ? 1 : 0;
   p->phib_g.assign(batch, 0.0f);
-  // resident launches by default for one frame where they are built: 15-25 %
-  // fewer microseconds per iteration than one launch per pass at 256^2,
-  // 512^2 and 1024^2 on MI355X; the exchange of Phi by device-scope
-  // accesses without fences is the default (the fenced forms are slower)
+  // resident launches by default for one frame where they are built: half to
+  // two thirds of the time of one launch per pass from 64^2 to 1024^2 on
+  // MI355X; the exchange of Phi by polled values is the default (the barrier
+  // forms are slower, the fenced ones most)
   const int res_mode = tune ? tune->resident : 0;
   p->resident = (res_mode != 2 && batch == 1 && resident_supported(n, tile, ept)) ? 1 : 0;
-  p->xm = (tune && tune->exchange >= 1 && tune->exchange <= 3) ? tune->exchange - 1 : 2;
+  p->xm = (tune && tune->exchange >= 1 && tune->exchange <= 4) ? tune->exchange - 1 : 3;
   p->polls = (tune && tune->barrier_polls > 0) ? (unsigned)tune->barrier_polls : (1u << 18);
   p->sw_fuse = !(tune && tune->sw_separate > 0);
   const size_t nn = (size_t)n * n;
@@ -681,6 +686,7 @@ int spk_plan_check(spk_plan* p) {
   SPK_HIP(hipMemcpy(h, p->pbar, sizeof(h), hipMemcpyDeviceToHost));
   if (h[2]) {
     SPK_HIP(hipMemset(p->pbar + 2, 0, sizeof(unsigned)));
+    p->rll_fill = true;
     return fail(SPK_EHIP, "a grid barrier of a resident or persistent launch gave up "
                           "waiting; results of that launch are invalid");
   }
@@ -698,7 +704,7 @@ int spk_plan_destroy(spk_plan* p) {
   dfree(p->mod); dfree(p->sup);
   dfree(p->tw); dfree(p->summ2); dfree(p->sumpart); dfree(p->errp); dfree(p->pbar);
   dfree(p->ipsf); dfree(p->dbuf); dfree(p->dbufc);
-  dfree(p->dbuf2); dfree(p->dbufc2); dfree(p->imap2); dfree(p->dmap2); dfree(p->rsync);
+  dfree(p->dbuf2); dfree(p->dbufc2); dfree(p->imap2); dfree(p->dmap2); dfree(p->rll);
   dfree(p->spec); dfree(p->imap); dfree(p->dmap);
   dfree(p->coh_ac); dfree(p->coh_w); dfree(p->coh_cb); dfree(p->coh_m); dfree(p->coh_part);
   dfree(p->sw_tmp); dfree(p->sw_blur); dfree(p->sw_maxp); dfree(p->fftbuf);
@@ -1312,13 +1318,18 @@ int iter_step(IterRun& r, int k, int* next) {
   *next = k + 1;
   if (r.res_end[k]) {
     const int k1 = r.res_end[k];
-    if (!p->rsync && (rc = dalloc(&p->rsync, (size_t)p->bands * 32))) return rc;
+    // one allocation: the exchange buffers of mode 3, then the barrier flags
+    const size_t ll = p->xm == 3 ? 2 * (size_t)p->nn() : 0;
+    if (!p->rll && (rc = dalloc(&p->rll, ll + (size_t)p->bands * 16))) return rc;
+    const int fill = p->rll_fill;
+    p->rll_fill = false;
+    unsigned* rsync = reinterpret_cast<unsigned*>(p->rll + ll);
     if ((rc = prof_arm(p, 2))) return rc;
     PassArgs ra = base_args(p);
     ra.swr_tab = r.res_fused[k] ? (const SwParam*)r.dptr(r.res_sw_off[k]) : nullptr;
     SPK_HIP(launch_resident(p->n, p->tile, p->ept, p->xm, ra, (const RStep*)r.dptr(r.res_off[k]),
                             r.res_n[k], r.err_trace ? p->errp : nullptr, (long long)B * p->bands,
-                            p->rsync, (int*)(p->pbar + 1), st));
+                            rsync, (int*)(p->pbar + 1), p->rll, fill, st));
     p->res_launches++;
     p->res_steps += r.res_n[k];
     p->sw_fused_count += r.res_fused[k];

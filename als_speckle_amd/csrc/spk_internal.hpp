@@ -191,14 +191,16 @@ hipError_t launch_roll_sum(const c32* data, int frames, int rows, int cols, cons
 // resident single-frame iteration block: one cooperative launch of n/tile
 // workgroups runs nsteps steps with the frame's modulus, support and iterate
 // in registers (k_resident); xm: exchange mode of Phi (0 plain + fences,
-// 1 device-scope + fences, 2 device-scope, no fences); errp0[kidx *
+// 1 device-scope + fences, 2 device-scope, no fences, 3 values polled
+// themselves in the two n*n buffers of ll; fill: empty them first, a new
+// pair); errp0[kidx *
 // errp_step + band] gets the error partials of the steps with err set;
 // flags: n/tile * 32 words of barrier flags (zeroed by the launcher); flag:
 // this launch's give-up flag, then the sticky one
 bool resident_supported(int n, int tile, int ept);
 hipError_t launch_resident(int n, int tile, int ept, int xm, const PassArgs& a,
                            const RStep* steps, int nsteps, double* errp0, long long errp_step,
-                           unsigned* flags, int* flag, hipStream_t st);
+                           unsigned* flags, int* flag, c32* ll, int fill, hipStream_t st);
 // workgroups of the persistent kernel that fit on the current device at once
 hipError_t persist_grid(int n, int tile, int ept, int* out);
 // mode 0: out = rowFFT(in); 1: out = rowIFFT(in) (unscaled);

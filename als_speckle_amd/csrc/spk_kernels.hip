@@ -1066,53 +1066,67 @@ __global__ void __launch_bounds__((N / E) * TT)
 //   1  device-scope (sc1) loads and stores of Phi, and the fences of 0
 //   2  device-scope loads and stores of Phi; the barrier orders them without
 //      fences (each wave waits for its stores before the arrival)
+//   3  device-scope stores whose readers poll the values themselves, no
+//      barrier (LlWait, ll_take); the barrier's flags only for shrinkwrap maps
 // ---------------------------------------------------------------------------
+// Device-scope (sc1) 8- and 4-byte accesses at a 32-bit byte offset from a
+// workgroup-uniform base, as buffer instructions: the compiler gives the
+// atomic builtins 64-bit vector addresses instead, two registers per value,
+// which the resident kernel has to spill.  Volatile (bit 31): never hoisted
+// out of a polling loop.  Offsets stay below 2^31 (8 n^2 bytes, n <= 1024).
+constexpr int kDevScope = (int)0x80000010;
+using u32x2 = uint32_t __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t dev_rsrc(const void* base) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), (short)0, 0x7FFFFFFF, 0x00027000);
+}
+__device__ __forceinline__ u32x2 dev_ld(const c32* base, unsigned i) {
+  return __builtin_amdgcn_raw_buffer_load_b64(dev_rsrc(base), (int)(i * 8u), 0, kDevScope);
+}
+__device__ __forceinline__ void dev_st(c32* base, unsigned i, u32x2 v) {
+  __builtin_amdgcn_raw_buffer_store_b64(v, dev_rsrc(base), (int)(i * 8u), 0, kDevScope);
+}
 template <int XM>
 __device__ __forceinline__ c32 xld(const c32* base, unsigned i) {
   if constexpr (XM == 0) {
     return gld(base, i);
   } else {
-    const uint64_t v = __hip_atomic_load(reinterpret_cast<const uint64_t*>(base) + i,
-                                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    return c32{__uint_as_float((unsigned)v), __uint_as_float((unsigned)(v >> 32))};
+    const u32x2 v = dev_ld(base, i);
+    return c32{__uint_as_float(v.x), __uint_as_float(v.y)};
   }
 }
 template <int XM>
 __device__ __forceinline__ void xst(c32* base, unsigned i, const c32& v) {
-  if constexpr (XM == 0) {
-    gst(base, i, v);
-  } else {
-    const uint64_t w = (uint64_t)__float_as_uint(v.x) | ((uint64_t)__float_as_uint(v.y) << 32);
-    __hip_atomic_store(reinterpret_cast<uint64_t*>(base) + i, w, __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
-  }
+  if constexpr (XM == 0) gst(base, i, v);
+  else dev_st(base, i, u32x2{__float_as_uint(v.x), __float_as_uint(v.y)});
 }
 
 // Float exchange of the resident kernel's shrinkwrap maps, device scope in
 // the exchange modes without fences (as xld / xst)
 template <int XM>
 __device__ __forceinline__ float xldf(const float* p, unsigned i) {
-  if constexpr (XM != 2) return gld(p, i);
-  else return __hip_atomic_load(p + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if constexpr (XM < 2) return gld(p, i);
+  else return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(dev_rsrc(p), (int)(i * 4u), 0,
+                                                                   kDevScope));
 }
 template <int XM>
 __device__ __forceinline__ void xstf(float* p, unsigned i, float v) {
-  if constexpr (XM != 2) gst(p, i, v);
-  else __hip_atomic_store(p + i, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if constexpr (XM < 2) gst(p, i, v);
+  else __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), dev_rsrc(p), (int)(i * 4u), 0,
+                                             kDevScope);
 }
 // sw_store_staged for the resident kernel: float4 stores, or in the fenceless
-// exchange mode two device-scope 8-byte stores per group of four
+// exchange modes two device-scope 8-byte stores per group of four
 template <int N, int TT, int XM, class OFF>
 __device__ __forceinline__ void sw_store_staged_x(const float* stage, float* dst, OFF off) {
   for (int v = threadIdx.x; v < N * TT / 4; v += blockDim.x) {
-    if constexpr (XM != 2) {
+    if constexpr (XM < 2) {
       *reinterpret_cast<float4*>(dst + off(v)) =
           *reinterpret_cast<const float4*>(stage + sw_swz(4 * v));
     } else {
-      const uint64_t* s2 = reinterpret_cast<const uint64_t*>(stage + sw_swz(4 * v));
-      uint64_t* d2 = reinterpret_cast<uint64_t*>(dst + off(v));
-      __hip_atomic_store(d2, s2[0], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      __hip_atomic_store(d2 + 1, s2[1], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      const u32x2* s2 = reinterpret_cast<const u32x2*>(stage + sw_swz(4 * v));
+      const unsigned d2 = (unsigned)off(v) / 2;
+      dev_st(reinterpret_cast<c32*>(dst), d2, s2[0]);
+      dev_st(reinterpret_cast<c32*>(dst), d2 + 1, s2[1]);
     }
   }
 }
@@ -1131,19 +1145,22 @@ __device__ __forceinline__ void sw_store_staged_x(const float* stage, float* dst
 // flag, acquire after the wait).  Waits are bounded as in grid_sync: after
 // `limit` poll rounds flag[0] (this launch's) and flag[1] (sticky) are set
 // and every later wait of the launch passes.
-template <int XM, int K>
-__device__ __forceinline__ void resident_sync(unsigned* flags, unsigned epoch, int* flag,
-                                              unsigned limit) {
-  static_assert(K >= 1, "at least one flag per polling lane");
+template <int XM>
+__device__ __forceinline__ void resident_arrive(unsigned* flags, unsigned epoch) {
   constexpr int LINE = 32;   // unsigned words per 128-byte line
-  constexpr bool fence = XM != 2;
   __builtin_amdgcn_s_waitcnt(0x0F70);   // this wave's stores have completed
   __syncthreads();
   if (threadIdx.x == 0) {
-    if (fence) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+    if (XM < 2) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
     __hip_atomic_store(flags + blockIdx.x * LINE, epoch, __ATOMIC_RELAXED,
                        __HIP_MEMORY_SCOPE_AGENT);
   }
+}
+template <int XM, int K>
+__device__ __forceinline__ void resident_wait(unsigned* flags, unsigned epoch, int* flag,
+                                              unsigned limit) {
+  static_assert(K >= 1, "at least one flag per polling lane");
+  constexpr int LINE = 32;
   if (threadIdx.x < 64) {
     bool gave = __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
     unsigned polls = 0;
@@ -1167,16 +1184,302 @@ __device__ __forceinline__ void resident_sync(unsigned* flags, unsigned epoch, i
         gave = true;
       }
     }
-    if (fence) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    if (XM < 2) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
   }
   __syncthreads();
 }
+template <int XM, int K>
+__device__ __forceinline__ void resident_sync(unsigned* flags, unsigned epoch, int* flag,
+                                              unsigned limit) {
+  resident_arrive<XM>(flags, epoch);
+  resident_wait<XM, K>(flags, epoch, flag, limit);
+}
 
-// LDS of the resident kernel: the pass LDS, padded so that one workgroup
-// occupies a CU (the grid is one workgroup per band, at most one per CU)
+// Exchange mode 3: the data are their own flags.  Phi crosses in two buffers
+// (row phase -> column phase, column phase -> row phase) whose empty slots
+// hold kEmpty in the real part; a value is one 8-byte device-scope store, and
+// its reader polls the slot itself until it is not empty, then empties it.
+// That takes the store's completion, the barrier's flag, its polls and the
+// loads after them (four trips to the memory side) down to the store's and
+// the load's.
+//   - a slot is written by one thread and read by one other; aligned 8-byte
+//     accesses are single-copy atomic, so a value that is seen is whole, and
+//     nothing else is read on the strength of it;
+//   - a slot is written again only after its reader's workgroup has stored
+//     into the other buffer, which it does after all its emptying stores have
+//     completed (ll_emptied, then a workgroup barrier);
+//   - a real part of kEmpty's pattern (a NaN that only the caller's own data
+//     could hold) is stored as another NaN, so no value looks like an empty slot.
+// A poll is bounded as the barrier's waits are.  The emptying stores go out
+// after the phase's first transform, not with the take, where they delay the
+// other workgroups' loads (1024^2: 11.9 -> 10.5 us per step).
+// Measured per HIO step with the trace, this mode and the fenceless barrier
+// (mode 2): 1024^2 10.4 / 13.0 us, 512^2 6.2 / 7.6, 256^2 5.2 / 6.7.
+constexpr uint32_t kEmpty = 0xFFFFFFFFu;   // the real part of an empty slot
+struct LlWait {
+  int* flag;
+  unsigned limit;
+  bool gave;       // uniform over the wavefront
+};
+template <int DELAY, int E, class POS>
+__device__ __forceinline__ void ll_take(c32 (&x)[E], c32* buf, LlWait& w, POS pos) {
+  u32x2 v[E];
+  unsigned polls = 0;
+  __builtin_amdgcn_s_sleep(DELAY);
+  while (true) {
+#pragma unroll
+    for (int i = 0; i < E; ++i) v[i] = dev_ld(buf, pos(i));
+    bool full = true;
+#pragma unroll
+    for (int i = 0; i < E; ++i) full = full && v[i].x != kEmpty;
+    if (__all(full) || w.gave) break;
+    if (++polls >= w.limit) {
+      __hip_atomic_store(w.flag, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      __hip_atomic_store(w.flag + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      w.gave = true;
+    } else if ((polls & 63) == 0) {
+      w.gave = __hip_atomic_load(w.flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+    }
+    __builtin_amdgcn_s_sleep(1);
+  }
+#pragma unroll
+  for (int i = 0; i < E; ++i) x[i] = c32{__uint_as_float(v[i].x), __uint_as_float(v[i].y)};
+}
+// empty the slots that ll_take read
+template <int E, class POS>
+__device__ __forceinline__ void ll_empty(c32* buf, POS pos) {
+#pragma unroll
+  for (int i = 0; i < E; ++i) dev_st(buf, pos(i), u32x2{kEmpty, kEmpty});
+}
+template <int E, class POS>
+__device__ __forceinline__ void ll_give(const c32 (&x)[E], c32* buf, POS pos) {
+#pragma unroll
+  for (int i = 0; i < E; ++i) {
+    unsigned re = __float_as_uint(x[i].x);
+    if (re == kEmpty) re = 0x7FC00000u;
+    dev_st(buf, pos(i), u32x2{re, __float_as_uint(x[i].y)});
+  }
+}
+// this wave's emptying stores have completed
+__device__ __forceinline__ void ll_emptied() { __builtin_amdgcn_s_waitcnt(0x0F70); }
+
+// ---------------------------------------------------------------------------
+// Transforms of the resident kernel: T = N/8 threads per line, 8 values each,
+// two thread mappings.  In the coalesced mapping (line tid % TT, t = tid / TT)
+// a wavefront covers all lines of the band: the mapping of the Phi loads and
+// stores.  In the private mapping the threads of one line (N <= 512), or of
+// the even or the odd samples of one line (N = 1024: the first three stages
+// are two independent 512-point transforms, the last radix-2 stage combines
+// them), lie in one wavefront, so their LDS exchanges need no workgroup
+// barrier and the two wavefronts of a SIMD overlap one's exchanges with the
+// other's butterflies.  A phase loads coalesced, runs its first transform into
+// the private mapping, its pointwise work there, and its second transform back
+// into the coalesced one: 3 barriers at 1024 and 2 below instead of 6 and 4.
+// Butterflies, twiddles and their order are stage_butterflies', so values are
+// the pass kernels' bit for bit.  A thread's twiddles do not change during a
+// launch and stay in registers.
+// ---------------------------------------------------------------------------
+// orders a wavefront's LDS writes before its reads (the hardware keeps a
+// wavefront's LDS accesses in order)
+__device__ __forceinline__ void wave_lds_order() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+template <int N, int TT>
+struct LineFft {
+  static constexpr int E = 8, T = N / E;
+  static constexpr bool SPLIT = T > 64;              // even and odd samples apart
+  static constexpr int TW = SPLIT ? 64 : T;          // lanes of a sub-transform
+  static constexpr int M = E * TW;                   // its length
+  static constexpr int SUBS = N * TT / M;            // sub-transforms of a workgroup
+  using P = RadixPlan<M, E>;
+  static constexpr int S = P::kStages;               // 2 or 3: 8, 8[, 8 or less]
+  static_assert(T <= 128 && S >= 2 && S <= 3, "64 <= N <= 1024");
+  // LDS: a chunk of each region per sub-transform (c32 slots)
+  static constexpr int CHA = M + M / 8 + 2;          // e -> e + e / 8
+  static constexpr int CHB = S == 3 ? M + M / 8 : 0; // e -> e + 8 (e / 64)
+  static constexpr int HALF = M / 2 + 16;            // even, then odd values
+  static constexpr int CHC = SPLIT ? 2 * HALF : 0;
+  static constexpr int LDS = SUBS * (CHA + CHB + CHC);
+
+  int cb, ct;     // coalesced mapping: line, t
+  int pb, pt;     // private mapping: line, natural t (values pt + i T)
+  int l;          // lane in the sub-transform
+  c32* a0;        // coalesced thread's first slot of the first exchange
+  c32* a;         // private chunks
+  c32* b;
+  c32* c;
+  c32* cline;     // region C of this line
+  const c32* fa;  // coalesced thread's read base of the last exchange
+  c32 w1[7];                      // stage 1
+  c32 w2[S == 3 ? 7 : 1];         // stage 2 (entries by butterfly, then value)
+  c32 w3[SPLIT ? 4 : 1], w3c[SPLIT ? 4 : 1], w2c[(!SPLIT && S == 3) ? 7 : 1];
+  c32 w1c[S == 2 ? 7 : 1];
+
+  template <int ST>
+  static __device__ __forceinline__ void load_tw(c32* w, const c32* twl, int t) {
+    // entries of stage ST for the butterflies t + q T of a thread
+    constexpr int R = plan_radix(N, E, ST), NS = RadixPlan<N, E>::span(ST), Q = E / R;
+    constexpr int STEP = ST == RadixPlan<N, E>::kStages - 1 ? T : TW;
+#pragma unroll
+    for (int q = 0; q < Q; ++q)
+#pragma unroll
+      for (int r = 1; r < R; ++r)
+        w[q * (R - 1) + r - 1] =
+            twl[staged_tw_offset(N, E, ST) + ((t + q * STEP) & (NS - 1)) * (R - 1) + r - 1];
+  }
+  __device__ __forceinline__ void init(c32* lds, const c32* twl) {
+    const int tid = threadIdx.x;
+    cb = tid % TT;
+    ct = tid / TT;
+    const int sub = tid / TW;
+    l = tid % TW;
+    pb = SPLIT ? sub / 2 : sub;
+    pt = SPLIT ? 2 * l + (sub & 1) : l;
+    a = lds + sub * CHA;
+    b = lds + SUBS * CHA + sub * CHB;
+    c = lds + SUBS * (CHA + CHB) + sub * CHC;
+    cline = lds + SUBS * (CHA + CHB) + 2 * pb * CHC;
+    const int csub = SPLIT ? 2 * cb + (ct & 1) : cb, cl = SPLIT ? ct >> 1 : ct;
+    a0 = lds + csub * CHA + 9 * cl;
+    if constexpr (SPLIT) fa = lds + 2 * cb * CHA;
+    else if constexpr (S == 3) fa = lds + SUBS * CHA + cb * CHB;
+    else fa = lds + cb * CHA;
+    load_tw<1>(w1, twl, l);
+    if constexpr (S == 3) load_tw<2>(w2, twl, l);
+    if constexpr (SPLIT) {
+      load_tw<3>(w3, twl, pt);
+      load_tw<3>(w3c, twl, ct);
+    } else if constexpr (S == 3) {
+      load_tw<2>(w2c, twl, ct);
+    } else {
+      load_tw<1>(w1c, twl, ct);
+    }
+  }
+  // butterflies of a stage of radix R on the thread's registers
+  template <int R, bool INV>
+  static __device__ __forceinline__ void butterflies(c32 (&x)[E], const c32* w) {
+    constexpr int Q = E / R;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+      c32 v[R];
+#pragma unroll
+      for (int r = 0; r < R; ++r) v[r] = x[q + r * Q];
+      if (w) {
+#pragma unroll
+        for (int r = 1; r < R; ++r) v[r] = twiddle<INV>(v[r], w[q * (R - 1) + r - 1]);
+      }
+      dft<R, INV>(v);
+#pragma unroll
+      for (int r = 0; r < R; ++r) x[q + r * Q] = v[r];
+    }
+  }
+  __device__ __forceinline__ void put_a(const c32 (&x)[E], c32* p) const {
+#pragma unroll
+    for (int r = 0; r < E; ++r) p[r] = x[r];
+  }
+  __device__ __forceinline__ void get_a(c32 (&x)[E]) const {
+    const c32* p = a + l + (l >> 3);
+#pragma unroll
+    for (int q = 0; q < E; ++q) x[q] = p[q * (TW + TW / 8)];
+  }
+  // slot of value e = t + q step of a B chunk
+  static __device__ __forceinline__ int slot_b(int e) { return e + 8 * (e >> 6); }
+  __device__ __forceinline__ void put_b(const c32 (&x)[E]) const {
+    c32* p = b + 72 * (l >> 3) + (l & 7);   // (l / 8) 64 + l % 8 + 8 r
+#pragma unroll
+    for (int r = 0; r < E; ++r) p[8 * r] = x[r];
+  }
+  __device__ __forceinline__ void get_b(c32 (&x)[E]) const {
+#pragma unroll
+    for (int q = 0; q < E; ++q) x[q] = b[slot_b(l + q * TW)];
+  }
+  // stages 1 .. of the sub-transform in the private mapping, after the first
+  // exchange; last = false leaves out the final stage of the plan below 1024
+  template <bool INV>
+  __device__ __forceinline__ void middle(c32 (&x)[E]) {
+    get_a(x);
+    butterflies<8, INV>(x, w1);
+    if constexpr (S == 3) {
+      put_b(x);
+      wave_lds_order();
+      get_b(x);
+      butterflies<P::radix(2), INV>(x, w2);
+    }
+  }
+  // coalesced values ct + i T of line cb -> transform at pt + i T of line pb
+  template <bool INV>
+  __device__ __forceinline__ void to_private(c32 (&x)[E]) {
+    butterflies<8, INV>(x, nullptr);
+    put_a(x, a0);
+    __syncthreads();
+    middle<INV>(x);
+    if constexpr (SPLIT) {
+#pragma unroll
+      for (int r = 0; r < E; ++r) c[(l & 1) * HALF + (l >> 1) + 32 * r] = x[r];   // l + 64 r
+      __syncthreads();
+      const c32* p = cline + (pt & 1) * HALF + l;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        x[q] = p[64 * q];
+        x[q + 4] = p[CHC + 64 * q];
+      }
+      butterflies<2, INV>(x, w3);
+    }
+  }
+  // values pt + i T of line pb -> transform at ct + i T of line cb
+  template <bool INV, class HOOK>
+  __device__ __forceinline__ void to_coalesced(c32 (&x)[E], HOOK before_barrier) {
+    butterflies<8, INV>(x, nullptr);
+    put_a(x, a + 9 * l);
+    if constexpr (SPLIT) {
+      wave_lds_order();
+      middle<INV>(x);
+      c32* p = a + l + (l >> 3);
+#pragma unroll
+      for (int r = 0; r < E; ++r) p[72 * r] = x[r];   // l + 64 r
+      before_barrier();
+      __syncthreads();
+      const c32* g = fa + ct + (ct >> 3);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        x[q] = g[144 * q];
+        x[q + 4] = g[CHA + 144 * q];
+      }
+      butterflies<2, INV>(x, w3c);
+    } else if constexpr (S == 3) {
+      wave_lds_order();
+      get_a(x);
+      butterflies<8, INV>(x, w1);
+      put_b(x);
+      before_barrier();
+      __syncthreads();
+#pragma unroll
+      for (int q = 0; q < E; ++q) x[q] = fa[slot_b(ct + q * T)];
+      butterflies<P::radix(2), INV>(x, w2c);
+    } else {
+      before_barrier();
+      __syncthreads();
+      const c32* g = fa + ct + (ct >> 3);
+#pragma unroll
+      for (int q = 0; q < E; ++q) x[q] = g[q * (T + T / 8)];
+      butterflies<8, INV>(x, w1c);
+    }
+  }
+};
+
+// LDS of the resident kernel: the transforms' regions and the shrinkwrap lines,
+// padded so that one workgroup occupies a CU (the grid is one workgroup per
+// band, at most one per CU)
+template <int N, int TT>
+constexpr int resident_base() {   // c32 slots before the error sums
+  return LineFft<N, TT>::LDS + (sw_lds_floats<N, TT>() + 32 + 1) / 2;
+}
 template <int N, int TT>
 constexpr int resident_lds_elems() {
-  constexpr int base = LdsPlan<N, TT>::TOTAL;
+  constexpr int base = resident_base<N, TT>() + (N / 8 * TT > 64 ? N / 8 * TT : 64) + 16;
   constexpr int half = (kLdsBytes / 2) / 8 + 64;   // more than half a CU's LDS
   return base > half ? base : half;
 }
@@ -1184,80 +1487,113 @@ constexpr int resident_lds_elems() {
 template <int N, int TT, int E, int XM>
 __global__ void __launch_bounds__((N / E) * TT)
     k_resident(PassArgs a, const RStep* __restrict__ steps, int nsteps, double* errp0,
-               long long errp_step, unsigned* flags, int* flag) {
+               long long errp_step, unsigned* flags, int* flag, c32* ll) {
   constexpr int NT = (N / E) * TT;
   constexpr int NB = N / TT;
   constexpr int T = N / E;
-  using L = LdsPlan<N, TT>;
+  using LF = LineFft<N, TT>;
+  static_assert(E == LF::E && LdsPlan<N, TT>::FULL_TW, "8 values per thread, the whole table");
   __shared__ c32 lds[resident_lds_elems<N, TT>()];
-  // the shrinkwrap blur lines and staged outputs live after the twiddle
-  // table, which stays in LDS for the whole launch
-  static_assert(L::TOTAL * 8 + (sw_lds_floats<N, TT>() + 32) * 4 <=
-                    resident_lds_elems<N, TT>() * 8,
-                "resident LDS holds the pass LDS, the blur lines and weights");
-  float* swl = reinterpret_cast<float*>(lds + L::TOTAL);
+  static_assert(sizeof(lds) <= kLdsBytes, "resident kernel does not fit in LDS");
+  // the shrinkwrap blur lines, staged outputs and weights, the reductions'
+  // scratch (and the twiddle table until the threads have taken theirs)
+  float* swl = reinterpret_cast<float*>(lds + LF::LDS);
   float* swwl = swl + sw_lds_floats<N, TT>();   // blur weights
-  const int tid = threadIdx.x, b = tid % TT, t = tid / TT;
+  static_assert(sw_lds_floats<N, TT>() >= 2 * N, "the shrinkwrap area holds the table");
+  // the error partials by coalesced thread, then the wavefronts' sums
+  constexpr int NW = (NT + 63) / 64;
+  double* eord = reinterpret_cast<double*>(lds + resident_base<N, TT>());
+  double* ewave = eord + (NT > 64 ? NT : 64);
+  const int tid = threadIdx.x;
   const int cband = xcd_band<NB>(blockIdx.x);   // as k_colpass
   const int rband = blockIdx.x;                 // as k_rowpass
-  c32* twl = lds + L::NBUF * L::BUF;
+  LF tf;
   {
     TwStage<N, TT, NT> tws;
     tws.fetch(a.tw);
-    tws.put(twl);
+    tws.put(reinterpret_cast<c32*>(swl));
+    __syncthreads();
+    tf.init(lds, reinterpret_cast<const c32*>(swl));
   }
-  const auto tw = twiddle_view<N, TT>(twl);
-  // resident state: modulus of the column band, support and iterate of the row band
+  const int cb = tf.cb, ct = tf.ct, pb = tf.pb, pt = tf.pt;
+  // resident state, private mapping: modulus of the column band, support and
+  // iterate of the row band
   float m[E], sv[E];
   c32 pin[E];
 #pragma unroll
   for (int i = 0; i < E; ++i) {
-    m[i] = gld(a.mod, mcol_pos<N, TT, E>(cband, b, t, i));
-    sv[i] = gld(a.sup, row_pos<N, TT, E>(rband, b, t, i));
-    pin[i] = gld(a.psi, row_pos<N, TT, E>(rband, b, t, i));
+    m[i] = gld(a.mod, mcol_pos<N, TT, E>(cband, pb, pt, i));
+    sv[i] = gld(a.sup, row_pos<N, TT, E>(rband, pb, pt, i));
+    pin[i] = gld(a.psi, row_pos<N, TT, E>(rband, pb, pt, i));
   }
   c32* phi = a.phi;
+  constexpr bool LL = XM == 3;
+  constexpr int KF = (NB + 63) / 64;
+  c32* to_col = ll;                       // mode 3: row phase -> column phase
+  c32* to_row = ll + (size_t)N * N;       // column phase -> row phase
+  LlWait llw{flag, a.polls, false};
+  // s_sleep units (64 cycles) before the first poll: the other workgroups'
+  // 8 n^2 bytes of stores take that long to drain, and polls would compete
+  // with them (1024^2: 12.6 us per step with 0, 11.9 with 20, 12.8 with 60;
+  // 512^2 and 256^2: 2, more costs latency)
+  constexpr int DELAY = N >= 1024 ? 24 : 2;
+  bool given = false;   // mode 3: to_col holds the step's Phi (else phi does)
+  auto cpos = [&](int i) { return (unsigned)col_pos<N, TT, E>(cband, cb, ct, i); };
+  auto rpos = [&](int i) { return (unsigned)row_pos<N, TT, E>(rband, cb, ct, i); };
+  // whether step j has a column phase
+  auto has_col = [&](const RStep& q) {
+    return !(q.c.flags & kNoOut) || q.err || (q.c.flags & kSwFin);
+  };
   unsigned epoch = 0;
   bool sup_changed = false;
-  // the column phase's FP64 error partial of this thread; the workgroup sum
-  // is formed in the row phase while its Phi loads are in flight (off the
-  // path between the column stores and the barrier)
-  double err = 0.0;
   for (int k = 0; k < nsteps; ++k) {
     const RStep st = steps[k];
     const bool noout = (st.c.flags & kNoOut) != 0;
     const bool swrow = (st.c.flags & kSwRow) != 0;   // shrinkwrap after this step
     const bool swfin = (st.c.flags & kSwFin) != 0;   // ... after the previous one
-    const bool col = !noout || st.err || swfin;
+    const bool col = has_col(st);
+    const bool last = k + 1 == nsteps;
+    // mode 3: the new Phi is formed only where something reads it
+    const bool emit = !LL || last || has_col(steps[last ? k : k + 1]);
     const bool err_sum = col && st.err && errp0;
     c32 x[E];
     if (col) {
       // column phase (colpass_item MODE 0, MODE 10 for kNoOut, MODE 9's blur)
       __syncthreads();   // the LDS of the previous phase is free
+      if (LL && given) {
+        ll_take<DELAY>(x, to_col, llw, cpos);
+      } else {
 #pragma unroll
-      for (int i = 0; i < E; ++i) x[i] = xld<XM>(phi, col_pos<N, TT, E>(cband, b, t, i));
+        for (int i = 0; i < E; ++i) x[i] = xld<XM>(phi, cpos(i));
+      }
       // a fused shrinkwrap's column half: its weights, fetched with Phi
       float wcol = 0.0f;
-      int rcol = 0;
-      if (swfin) {
-        wcol = sw_weight_fetch(a.swr_tab[st.swf].w);
-        rcol = a.swr_tab[st.swf].w.radius;
-      }
-      err = 0.0;
-      fft_regs<N, E, TT, false, true>(x, t, b, lds, tw);
+      if (swfin) wcol = sw_weight_fetch(a.swr_tab[st.swf].w);
+      tf.template to_private<false>(x);
+      if (LL && given) ll_empty<E>(to_col, cpos);
+      // this thread's FP64 error partial goes to the thread that holds its
+      // values in the coalesced mapping; the workgroup's sum (colpass_item's,
+      // in its order) is formed in the row phase while Phi is on its way
+      double err = 0.0;
 #pragma unroll
       for (int i = 0; i < E; ++i) x[i] = project_modulus(x[i], m[i], err);
+      if (err_sum) eord[pt * TT + pb] = err;
       // the row-blurred |psi| of the band's columns, loaded under the inverse
       // transform (as colpass_item MODE 9)
       float rb[E];
       if (swfin) {
+        if (LL) resident_wait<XM, KF>(flags, epoch, flag, a.polls);
 #pragma unroll
-        for (int i = 0; i < E; ++i) rb[i] = xldf<XM>(a.sw_tmp, col_pos<N, TT, E>(cband, b, t, i));
+        for (int i = 0; i < E; ++i) rb[i] = xldf<XM>(a.sw_tmp, cpos(i));
       }
       if (!noout) {
-        fft_regs<N, E, TT, true, false>(x, t, b, lds, tw);
+        tf.template to_coalesced<true>(x, [&]() { if (LL) ll_emptied(); });
+        if constexpr (LL) {
+          ll_give(x, to_row, cpos);
+        } else {
 #pragma unroll
-        for (int i = 0; i < E; ++i) xst<XM>(phi, col_pos<N, TT, E>(cband, b, t, i), x[i]);
+          for (int i = 0; i < E; ++i) xst<XM>(phi, cpos(i), x[i]);
+        }
       }
       if (swfin) {
         // the column half of the previous step's shrinkwrap blur (as
@@ -1265,7 +1601,7 @@ __global__ void __launch_bounds__((N / E) * TT)
         // -> sw_blur (tiled) and the band maximum
         __syncthreads();
 #pragma unroll
-        for (int i = 0; i < E; ++i) swl[b * sw_line<N>() + blur_slot(t + i * T)] = rb[i];
+        for (int i = 0; i < E; ++i) swl[cb * sw_line<N>() + blur_slot(ct + i * T)] = rb[i];
         sw_weight_put(wcol, swwl);
         __syncthreads();
         float* stage = swl + sw_stage_off<N, TT>();
@@ -1280,25 +1616,45 @@ __global__ void __launch_bounds__((N / E) * TT)
         const float bm = block_max(mx, swl);
         if (tid == 0) xstf<XM>(a.sw_maxp, cband, bm);
       }
-      resident_sync<XM, (NB + 63) / 64>(flags, ++epoch, flag, a.polls);
+      // mode 3: a barrier only for the shrinkwrap maps, and where the row
+      // phase does not wait for this phase's Phi but overwrites its input
+      if (!LL) resident_sync<XM, KF>(flags, ++epoch, flag, a.polls);
+      else if (swfin || noout) resident_arrive<XM>(flags, ++epoch);
     }
     // row phase (rowpass_item; kNoOut skips Phi).  Every load is issued
     // first: Phi, the band maxima and blur of a fused shrinkwrap's threshold,
     // the weights of this step's shrinkwrap.
     __syncthreads();
-    if (!noout) {
+    // block_sum's wavefront half; its other half follows the next barrier
+    auto err_waves = [&]() {
+      if (!err_sum) return;
+      double v = eord[tid];
+      if constexpr (NT % 64 == 0) {
 #pragma unroll
-      for (int i = 0; i < E; ++i) x[i] = xld<XM>(phi, row_pos<N, TT, E>(rband, b, t, i));
+        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+        if ((tid & 63) == 0) ewave[tid >> 6] = v;
+      } else {
+        v = block_sum(v, eord);
+        if (tid == 0) ewave[0] = v;
+      }
+    };
+    if (!noout) {
+      if constexpr (LL) {
+        err_waves();
+        ll_take<DELAY>(x, to_row, llw, rpos);
+      } else {
+#pragma unroll
+        for (int i = 0; i < E; ++i) x[i] = xld<XM>(phi, rpos(i));
+      }
     }
+    if (!LL || noout) err_waves();
+    if (LL && swfin) resident_wait<XM, KF>(flags, epoch, flag, a.polls);
     float wrow = 0.0f;
-    int rrow = 0;
-    if (swrow) {
-      wrow = sw_weight_fetch(a.swr_tab[st.swr].w);
-      rrow = a.swr_tab[st.swr].w.radius;
-    }
+    if (swrow) wrow = sw_weight_fetch(a.swr_tab[st.swr].w);
     if (swfin) {
       // the previous step's threshold: s = 0 where blur <= tau * max, with
-      // the frame maximum from the column bands' maxima (FP64 threshold)
+      // the frame maximum from the column bands' maxima (FP64 threshold).
+      // The blur goes through LDS from the coalesced to the private mapping.
       constexpr int MPT = (NB + NT - 1) / NT;
       float mx = -INFINITY;
       float bl[E];
@@ -1308,40 +1664,54 @@ __global__ void __launch_bounds__((N / E) * TT)
         if (q < NB) mx = fmaxf(mx, xldf<XM>(a.sw_maxp, q));
       }
 #pragma unroll
-      for (int i = 0; i < E; ++i) bl[i] = xldf<XM>(a.sw_blur, row_pos<N, TT, E>(rband, b, t, i));
+      for (int i = 0; i < E; ++i) bl[i] = xldf<XM>(a.sw_blur, rpos(i));
       const double thr = (double)a.swr_tab[st.swf].tau * (double)block_max(mx, swl);
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < E; ++i) swl[cb * sw_line<N>() + blur_slot(ct + i * T)] = bl[i];
+      __syncthreads();
 #pragma unroll
       for (int i = 0; i < E; ++i)
-        if (!((double)bl[i] > thr)) sv[i] = 0.0f;
+        if (!((double)swl[pb * sw_line<N>() + blur_slot(pt + i * T)] > thr)) sv[i] = 0.0f;
       sup_changed = true;
       __syncthreads();
     }
-    if (err_sum) {
-      // the column phase's error partial (the same sum in the same order as
-      // colpass_item's); the reduction uses the shrinkwrap area of the LDS,
-      // which the transforms below do not touch
-      const double s = block_sum(err, reinterpret_cast<double*>(swl));
-      if (tid == 0) errp0[(size_t)st.kidx * errp_step + cband] = s;
+    if (!noout) {
+      tf.template to_private<true>(x);
+      if (LL) ll_empty<E>(to_row, rpos);
+    } else if (err_sum) {
+      __syncthreads();
     }
-    if (!noout) fft_regs<N, E, TT, true, true>(x, t, b, lds, tw);
-    float av[E];
+    if (err_sum && tid == 0) {
+      double s = 0.0;
+      for (int w = 0; w < NW; ++w) s += ewave[w];
+      errp0[(size_t)st.kidx * errp_step + cband] = s;
+    }
 #pragma unroll
     for (int i = 0; i < E; ++i) {
       const c32 pout = noout ? c32{0.0f, 0.0f} : scale(x[i], a.inv_nn);
-      const c32 nv = update_value<false>(st.c, pout, pin[i], sv[i], c32{0.0f, 0.0f});
-      pin[i] = nv;
-      x[i] = nv;
-      av[i] = sqrtf(nv.x * nv.x + nv.y * nv.y);
+      pin[i] = update_value<false>(st.c, pout, pin[i], sv[i], c32{0.0f, 0.0f});
+      x[i] = pin[i];
     }
-    fft_regs<N, E, TT, false, false>(x, t, b, lds, tw);
+    if (emit) {
+      tf.template to_coalesced<false>(x, [&]() { if (LL) ll_emptied(); });
+      if (LL && noout && col && !swfin) resident_wait<XM, KF>(flags, epoch, flag, a.polls);
+      if (LL && !last) {
+        ll_give(x, to_col, rpos);
+        given = true;
+      } else {
 #pragma unroll
-    for (int i = 0; i < E; ++i) xst<XM>(phi, row_pos<N, TT, E>(rband, b, t, i), x[i]);
+        for (int i = 0; i < E; ++i) xst<XM>(phi, rpos(i), x[i]);
+      }
+    }
     if (swrow) {
       // the row half of this step's shrinkwrap blur (as rowpass_item SW 1):
       // the band's rows of |new psi| -> sw_tmp
       __syncthreads();
 #pragma unroll
-      for (int i = 0; i < E; ++i) swl[b * sw_line<N>() + blur_slot(t + i * T)] = av[i];
+      for (int i = 0; i < E; ++i)
+        swl[pb * sw_line<N>() + blur_slot(pt + i * T)] =
+            sqrtf(pin[i].x * pin[i].x + pin[i].y * pin[i].y);
       sw_weight_put(wrow, swwl);
       __syncthreads();
       float* stage = swl + sw_stage_off<N, TT>();
@@ -1352,15 +1722,31 @@ __global__ void __launch_bounds__((N / E) * TT)
       sw_store_staged_x<N, TT, XM>(stage, a.sw_tmp + (size_t)rband * N * TT,
                                    [](int v) { return 4 * v; });
     }
-    if (k + 1 < nsteps) resident_sync<XM, (NB + 63) / 64>(flags, ++epoch, flag, a.polls);
+    if (!LL) {
+      if (!last) resident_sync<XM, KF>(flags, ++epoch, flag, a.polls);
+    } else if (swrow) {
+      resident_arrive<XM>(flags, ++epoch);
+    }
   }
 #pragma unroll
-  for (int i = 0; i < E; ++i) gst(a.psi, row_pos<N, TT, E>(rband, b, t, i), pin[i]);
+  for (int i = 0; i < E; ++i) gst(a.psi, row_pos<N, TT, E>(rband, pb, pt, i), pin[i]);
   if (sup_changed) {
     float* sup = const_cast<float*>(a.sup);
 #pragma unroll
-    for (int i = 0; i < E; ++i) gst(sup, row_pos<N, TT, E>(rband, b, t, i), sv[i]);
+    for (int i = 0; i < E; ++i) gst(sup, row_pos<N, TT, E>(rband, pb, pt, i), sv[i]);
   }
+}
+
+// before a resident launch: its barrier flags and give-up flag start at 0; the
+// exchange buffers of mode 3 are empty from the start and left empty by every
+// launch that did not give up (flag[1], sticky): filled when new or after that
+static __global__ void __launch_bounds__(256)
+    k_resident_begin(unsigned* flags, int words, int* flag, u32x2* ll, int count, int fill) {
+  const int i = blockIdx.x * 256 + threadIdx.x, n = gridDim.x * 256;
+  for (int j = i; j < words; j += n) flags[j] = 0u;
+  if (i == 0) flag[0] = 0;
+  if (fill || flag[1])
+    for (int j = i; j < count; j += n) ll[j] = u32x2{kEmpty, kEmpty};
 }
 
 static __global__ void k_zero_u32(unsigned* p, int n) {
@@ -2631,15 +3017,16 @@ static hipError_t tfcol_nt(int kind, const c32* phi, const float* goal, int rows
 template <int N, int TT, int E>
 static hipError_t resident_nt(int xm, const PassArgs& a, const RStep* steps, int nsteps,
                               double* errp0, long long errp_step, unsigned* flags, int* flag,
-                              hipStream_t st) {
-  // the workgroups' barrier flags and this launch's give-up flag start at 0
-  constexpr int words = (N / TT) * 32;
-  hipLaunchKernelGGL(k_zero_u32, dim3((words + 255) / 256), dim3(256), 0, st, flags, words);
-  hipLaunchKernelGGL(k_zero_u32, dim3(1), dim3(64), 0, st, reinterpret_cast<unsigned*>(flag), 1);
-  void* args[] = {(void*)&a, (void*)&steps, (void*)&nsteps, (void*)&errp0, (void*)&errp_step,
-                  (void*)&flags, (void*)&flag};
+                              c32* ll, int fill, hipStream_t st) {
+  const int words = (N / TT) * 32, count = xm == 3 ? 2 * N * N : 0;
+  const int blocks = fill && count ? 1024 : std::max(1, words / 256);
+  hipLaunchKernelGGL(k_resident_begin, dim3(blocks), dim3(256), 0, st, flags, words, flag,
+                     reinterpret_cast<u32x2*>(ll), count, fill);
+  void* args[] = {(void*)&a,     (void*)&steps, (void*)&nsteps, (void*)&errp0, (void*)&errp_step,
+                  (void*)&flags, (void*)&flag,  (void*)&ll};
   const void* fn = xm == 1   ? reinterpret_cast<const void*>(&k_resident<N, TT, E, 1>)
                    : xm == 2 ? reinterpret_cast<const void*>(&k_resident<N, TT, E, 2>)
+                   : xm == 3 ? reinterpret_cast<const void*>(&k_resident<N, TT, E, 3>)
                              : reinterpret_cast<const void*>(&k_resident<N, TT, E, 0>);
   if (g_launch_events[0]) {
     (void)hipEventRecord(g_launch_events[0], st);
@@ -2652,21 +3039,23 @@ static hipError_t resident_nt(int xm, const PassArgs& a, const RStep* steps, int
   return e;
 }
 
-// the resident form exists for one frame of 256^2 .. 1024^2 in tile 4 with
+// the resident form exists for one frame of 64^2 .. 1024^2 in tile 4 with
 // 8 values per thread (one workgroup of at most 512 threads per band, at
 // most 256 bands: one per CU), and for 256^2 and 512^2 also in tile 2 (128
 // and 256 bands: more CUs, half the lines per workgroup)
 template <int N>
 static hipError_t resident_dispatch(int tile, int ept, int xm, const PassArgs& a,
                                     const RStep* steps, int nsteps, double* errp0,
-                                    long long errp_step, unsigned* bar, int* flag,
-                                    hipStream_t st) {
-  if constexpr (N >= 256 && N <= 1024) {
+                                    long long errp_step, unsigned* bar, int* flag, c32* ll,
+                                    int fill, hipStream_t st) {
+  if constexpr (N >= 64 && N <= 1024) {
     if (tile == 4 && ept == 8)
-      return resident_nt<N, 4, 8>(xm, a, steps, nsteps, errp0, errp_step, bar, flag, st);
-    if constexpr (N <= 512) {
+      return resident_nt<N, 4, 8>(xm, a, steps, nsteps, errp0, errp_step, bar, flag, ll, fill,
+                                  st);
+    if constexpr (N >= 256 && N <= 512) {
       if (tile == 2 && ept == 8)
-        return resident_nt<N, 2, 8>(xm, a, steps, nsteps, errp0, errp_step, bar, flag, st);
+        return resident_nt<N, 2, 8>(xm, a, steps, nsteps, errp0, errp_step, bar, flag, ll, fill,
+                                    st);
     }
   }
   return hipErrorInvalidValue;
@@ -2736,7 +3125,7 @@ constexpr bool shape_ok() {
                        const c32* tw, hipStream_t st);                                      \
   hipError_t resident_##n(int tile, int ept, int xm, const PassArgs& a, const RStep* steps, \
                           int nsteps, double* errp0, long long errp_step, unsigned* bar,    \
-                          int* flag, hipStream_t st);
+                          int* flag, c32* ll, int fill, hipStream_t st);
 
 // a shape that is not built compiles to an error return, not a kernel
 #define SPK_CALL_COL(TT_, E_)                                                   \
@@ -2839,9 +3228,9 @@ constexpr bool shape_ok() {
   }                                                                                         \
   hipError_t resident_##n(int tile, int ept, int xm, const PassArgs& a, const RStep* steps, \
                           int nsteps, double* errp0, long long errp_step, unsigned* bar,    \
-                          int* flag, hipStream_t st) {                                      \
+                          int* flag, c32* ll, int fill, hipStream_t st) {                   \
     return resident_dispatch<n>(tile, ept, xm, a, steps, nsteps, errp0, errp_step, bar,     \
-                                flag, st);                                                  \
+                                flag, ll, fill, st);                                                  \
   }
 
 SPK_SIZES(SPK_SIZED_DECL)
@@ -2912,14 +3301,15 @@ hipError_t launch_rowpass(int n, int tile, int ept, bool use_t, bool emit_b, int
 }
 
 bool resident_supported(int n, int tile, int ept) {
-  return n >= 256 && n <= 1024 && (n & (n - 1)) == 0 && ept == 8 &&
-         (tile == 4 || (tile == 2 && n <= 512));
+  return n >= 64 && n <= 1024 && (n & (n - 1)) == 0 && ept == 8 &&
+         (tile == 4 || (tile == 2 && n >= 256 && n <= 512));
 }
 
 hipError_t launch_resident(int n, int tile, int ept, int xm, const PassArgs& a,
                            const RStep* steps, int nsteps, double* errp0, long long errp_step,
-                           unsigned* bar, int* flag, hipStream_t st) {
-  SPK_SIZE_SWITCH(resident, tile, ept, xm, a, steps, nsteps, errp0, errp_step, bar, flag, st)
+                           unsigned* bar, int* flag, c32* ll, int fill, hipStream_t st) {
+  SPK_SIZE_SWITCH(resident, tile, ept, xm, a, steps, nsteps, errp0, errp_step, bar, flag, ll, fill,
+                  st)
 }
 
 hipError_t launch_rowfft(int n, int tile, int ept, int mode, const c32* in, c32* out,

@@ -68,22 +68,24 @@ typedef struct spk_tune {
   int32_t sw_separate;/* 1: run each shrinkwrap as its own kernels (default:
                          fused into the passes of its step and the next
                          where the blur radius is <= 24 px, i.e. sigma <= 4) */
-  int32_t resident;   /* one frame of 256^2..1024^2 in tile 4 (256^2 and
+  int32_t resident;   /* one frame of 64^2..1024^2 in tile 4 (256^2 and
                          512^2 also in tile 2), 8 values per
                          thread: runs of non-DM steps run as one cooperative
                          resident launch each (the frame's modulus, support
-                         and iterate held on chip, Phi exchanged through a
-                         grid barrier, shrinkwraps inside the launch); 0 or
+                         and iterate held on chip, Phi exchanged between the
+                         workgroups, shrinkwraps inside the launch); 0 or
                          1: where built (the default), 2: never.  A resident
                          launch needs the whole device: no other cooperative
                          launch may run beside it (spk_plan_check reports a
-                         barrier that gave up waiting)                       */
-  int32_t exchange;   /* resident launches: how Phi crosses the barrier,
-                         1 plain + device-scope fences, 2 device-scope
-                         accesses + fences, 3 device-scope accesses without
-                         fences (the default); 0 = default                   */
+                         wait that gave up)                                  */
+  int32_t exchange;   /* resident launches: how Phi crosses between workgroups,
+                         1 plain + barrier with device-scope fences, 2
+                         device-scope accesses + fences, 3 device-scope
+                         accesses + barrier without fences, 4 device-scope
+                         values that their readers poll, no barrier (the
+                         default); 0 = default                               */
   int32_t barrier_polls; /* resident and persistent launches: poll rounds of
-                         a grid-barrier wait before it gives up (the launch
+                         a wait for other workgroups before it gives up (the launch
                          then drains without waiting and spk_plan_check
                          reports it); 0 = default, 262144.  Small values
                          exist to exercise the give-up path.                 */
