@@ -1082,7 +1082,7 @@ int iter_prepare(spk_plan* p, const spk_step* steps, int nsteps, int per_frame,
   emits.assign(nsteps, 0);
   for (int k = 0; k < nsteps; ++k)
     for (int f = 0; f < W; ++f) emits[k] |= (coefs[(size_t)k * W + f].flags & kEmitB) != 0;
-  // Resident blocks (k_resident, one frame): runs of steps with no DM work
+  // Resident blocks (one frame): runs of steps with no DM work
   // (no DM step, no emission).  A shrinkwrap after a step of the run runs
   // inside the block (row blur in that step's row phase, column blur in the
   // next active step's column phase, threshold in its row phase) when its
@@ -1098,8 +1098,11 @@ int iter_prepare(spk_plan* p, const spk_step* steps, int nsteps, int per_frame,
   r.res_off.assign(nsteps, 0);
   r.res_sw_off.assign(nsteps, 0);
   in_res.assign(nsteps, 0);
-  if (blocks && p->resident && B == 1 && !p->ipsf_on && !p->spec_on && !p->persist &&
-      !p->capturing) {
+  // With an ipsf the block is k_resident_ipsf's (tile 4, exchange mode 3), and
+  // ends at every shrinkwrap; with a spectrum there is none (the rescaled map
+  // is gathered from all over the frame).
+  if (blocks && p->resident && B == 1 && !p->spec_on && !p->persist && !p->capturing &&
+      (!p->ipsf_on || (p->xm == 3 && p->tile == 4))) {
     auto fits = [&](int j) { return !any_dm[j] && !emits[j]; };
     std::vector<RStep> rs;
     std::vector<SwParam> sp;
@@ -1123,7 +1126,7 @@ int iter_prepare(spk_plan* p, const spk_step* steps, int nsteps, int per_frame,
           int nx = j + 1;
           while (nx < nsteps && fits(nx) && !act[(size_t)nx * W]) ++nx;
           const bool goes_on = nx < nsteps && fits(nx);
-          if (!goes_on || sw_r[j] > kSwFuseRmax || !p->sw_fuse) {
+          if (!goes_on || sw_r[j] > kSwFuseRmax || !p->sw_fuse || p->ipsf_on) {
             rs.push_back(rsj);
             break;                        // stand-alone shrinkwrap after the block
           }
@@ -1327,9 +1330,16 @@ int iter_step(IterRun& r, int k, int* next) {
     if ((rc = prof_arm(p, 2))) return rc;
     PassArgs ra = base_args(p);
     ra.swr_tab = r.res_fused[k] ? (const SwParam*)r.dptr(r.res_sw_off[k]) : nullptr;
-    SPK_HIP(launch_resident(p->n, p->tile, p->ept, p->xm, ra, (const RStep*)r.dptr(r.res_off[k]),
-                            r.res_n[k], r.err_trace ? p->errp : nullptr, (long long)B * p->bands,
-                            rsync, (int*)(p->pbar + 1), p->rll, fill, st));
+    if (p->ipsf_on)
+      SPK_HIP(launch_resident_ipsf(p->n, p->tile, p->ept, ra, p->ipsf,
+                                   (const RStep*)r.dptr(r.res_off[k]), r.res_n[k],
+                                   r.err_trace ? p->errp : nullptr, (long long)B * p->bands,
+                                   (int*)(p->pbar + 1), p->rll, fill, st));
+    else
+      SPK_HIP(launch_resident(p->n, p->tile, p->ept, p->xm, ra,
+                              (const RStep*)r.dptr(r.res_off[k]), r.res_n[k],
+                              r.err_trace ? p->errp : nullptr, (long long)B * p->bands, rsync,
+                              (int*)(p->pbar + 1), p->rll, fill, st));
     p->res_launches++;
     p->res_steps += r.res_n[k];
     p->sw_fused_count += r.res_fused[k];

@@ -201,6 +201,12 @@ bool resident_supported(int n, int tile, int ept);
 hipError_t launch_resident(int n, int tile, int ept, int xm, const PassArgs& a,
                            const RStep* steps, int nsteps, double* errp0, long long errp_step,
                            unsigned* flags, int* flag, c32* ll, int fill, hipStream_t st);
+// the same with a partially coherent projection by the tiled ipsf, in tile 4
+// and exchange mode 3 (k_resident_ipsf); fused shrinkwraps are not part of it
+hipError_t launch_resident_ipsf(int n, int tile, int ept, const PassArgs& a, const c32* ipsf,
+                                const RStep* steps, int nsteps, double* errp0,
+                                long long errp_step, int* flag, c32* ll, int fill,
+                                hipStream_t st);
 // workgroups of the persistent kernel that fit on the current device at once
 hipError_t persist_grid(int n, int tile, int ept, int* out);
 // mode 0: out = rowFFT(in); 1: out = rowIFFT(in) (unscaled);

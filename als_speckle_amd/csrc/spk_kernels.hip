@@ -1470,6 +1470,35 @@ struct LineFft {
   }
 };
 
+// block_sum of the values in v[thread], in two halves: every wavefront's own
+// sum into part[], then (after a barrier) thread 0's sum of them in order.
+// v holds max(NT, 64) doubles; the caller's barrier precedes the first half.
+template <int NT>
+__device__ __forceinline__ void block_sum_waves(double* v, double* part) {
+  double s = v[threadIdx.x];
+  if constexpr (NT % 64 == 0) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = s;
+  } else {
+    s = block_sum(s, v);
+    if (threadIdx.x == 0) part[0] = s;
+  }
+}
+template <int NT>
+__device__ __forceinline__ double block_sum_rest(const double* part) {
+  double s = 0.0;
+  for (int w = 0; w < (NT + 63) / 64; ++w) s += part[w];
+  return s;
+}
+
+// s_sleep units (64 cycles) before the first poll of mode 3: the other
+// workgroups' 8 n^2 bytes of stores take that long to drain, and polls would
+// compete with them (1024^2: 12.6 us per step with 0, 11.9 with 20, 12.8 with
+// 60; 512^2 and 256^2: 2, more costs latency)
+template <int N>
+constexpr int ll_delay() { return N >= 1024 ? 24 : 2; }
+
 // LDS of the resident kernel: the transforms' regions and the shrinkwrap lines,
 // padded so that one workgroup occupies a CU (the grid is one workgroup per
 // band, at most one per CU)
@@ -1501,7 +1530,6 @@ __global__ void __launch_bounds__((N / E) * TT)
   float* swwl = swl + sw_lds_floats<N, TT>();   // blur weights
   static_assert(sw_lds_floats<N, TT>() >= 2 * N, "the shrinkwrap area holds the table");
   // the error partials by coalesced thread, then the wavefronts' sums
-  constexpr int NW = (NT + 63) / 64;
   double* eord = reinterpret_cast<double*>(lds + resident_base<N, TT>());
   double* ewave = eord + (NT > 64 ? NT : 64);
   const int tid = threadIdx.x;
@@ -1532,11 +1560,7 @@ __global__ void __launch_bounds__((N / E) * TT)
   c32* to_col = ll;                       // mode 3: row phase -> column phase
   c32* to_row = ll + (size_t)N * N;       // column phase -> row phase
   LlWait llw{flag, a.polls, false};
-  // s_sleep units (64 cycles) before the first poll: the other workgroups'
-  // 8 n^2 bytes of stores take that long to drain, and polls would compete
-  // with them (1024^2: 12.6 us per step with 0, 11.9 with 20, 12.8 with 60;
-  // 512^2 and 256^2: 2, more costs latency)
-  constexpr int DELAY = N >= 1024 ? 24 : 2;
+  constexpr int DELAY = ll_delay<N>();
   bool given = false;   // mode 3: to_col holds the step's Phi (else phi does)
   auto cpos = [&](int i) { return (unsigned)col_pos<N, TT, E>(cband, cb, ct, i); };
   auto rpos = [&](int i) { return (unsigned)row_pos<N, TT, E>(rband, cb, ct, i); };
@@ -1625,18 +1649,8 @@ __global__ void __launch_bounds__((N / E) * TT)
     // first: Phi, the band maxima and blur of a fused shrinkwrap's threshold,
     // the weights of this step's shrinkwrap.
     __syncthreads();
-    // block_sum's wavefront half; its other half follows the next barrier
     auto err_waves = [&]() {
-      if (!err_sum) return;
-      double v = eord[tid];
-      if constexpr (NT % 64 == 0) {
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-        if ((tid & 63) == 0) ewave[tid >> 6] = v;
-      } else {
-        v = block_sum(v, eord);
-        if (tid == 0) ewave[0] = v;
-      }
+      if (err_sum) block_sum_waves<NT>(eord, ewave);
     };
     if (!noout) {
       if constexpr (LL) {
@@ -1682,11 +1696,8 @@ __global__ void __launch_bounds__((N / E) * TT)
     } else if (err_sum) {
       __syncthreads();
     }
-    if (err_sum && tid == 0) {
-      double s = 0.0;
-      for (int w = 0; w < NW; ++w) s += ewave[w];
-      errp0[(size_t)st.kidx * errp_step + cband] = s;
-    }
+    if (err_sum && tid == 0)
+      errp0[(size_t)st.kidx * errp_step + cband] = block_sum_rest<NT>(ewave);
 #pragma unroll
     for (int i = 0; i < E; ++i) {
       const c32 pout = noout ? c32{0.0f, 0.0f} : scale(x[i], a.inv_nn);
@@ -1735,6 +1746,133 @@ __global__ void __launch_bounds__((N / E) * TT)
 #pragma unroll
     for (int i = 0; i < E; ++i) gst(sup, row_pos<N, TT, E>(rband, pb, pt, i), sv[i]);
   }
+}
+
+// ---------------------------------------------------------------------------
+// Resident block with a partially coherent projection (ipsf, no spectrum,
+// exchange mode 3): four phases per step, each a take, two transforms (one
+// each way) and a give, with the ipsf's rows and Psi kept in registers too:
+//   column  Psi = colFFT(Phi); colFFT(|Psi|^2)
+//   row     rowIFFT(ipsf * rowFFT(.))
+//   column  div = sqrt(|colIFFT(.)| / n^2); colIFFT(m Psi / div)
+//   row     rowIFFT, update, rowFFT
+// Arithmetic of colpass_ipsf_a, k_rowconv, colpass_div_b and rowpass_item,
+// except that Psi is not formed twice: bitwise the four launches' results.
+// Per step on MI355X, as four launches (each bound by its kernel boundary and one
+// pass over memory) and here: 1024^2 40.1 / 20.9 us, 512^2 24.3 / 12.9,
+// 256^2 18.7 / 10.8, 64^2 16.4 / 9.3.
+// ---------------------------------------------------------------------------
+template <int N, int TT, int E>
+__global__ void __launch_bounds__((N / E) * TT)
+    k_resident_ipsf(PassArgs a, const c32* __restrict__ ipsf, const RStep* __restrict__ steps,
+                    int nsteps, double* errp0, long long errp_step, int* flag, c32* ll) {
+  constexpr int NT = (N / E) * TT, NB = N / TT;
+  using LF = LineFft<N, TT>;
+  constexpr int TWF = N > 2 * NT ? N : 2 * NT;   // the table, then the error sums
+  constexpr int LDSN = LF::LDS + TWF + 64;
+  constexpr int HALF = (kLdsBytes / 2) / 8 + 64;
+  __shared__ c32 lds[LDSN > HALF ? LDSN : HALF];   // one workgroup per CU
+  static_assert(sizeof(lds) <= kLdsBytes, "resident kernel does not fit in LDS");
+  c32* area = lds + LF::LDS;
+  const int tid = threadIdx.x;
+  const int cband = xcd_band<NB>(blockIdx.x), rband = blockIdx.x;
+  LF tf;
+  {
+    TwStage<N, TT, NT> tws;
+    tws.fetch(a.tw);
+    tws.put(area);
+    __syncthreads();
+    tf.init(lds, area);
+    __syncthreads();
+  }
+  double* eord = reinterpret_cast<double*>(area);
+  double* ewave = eord + (NT > 64 ? NT : 64);
+  const int cb = tf.cb, ct = tf.ct, pb = tf.pb, pt = tf.pt;
+  float m[E], sv[E];
+  c32 pin[E], w[E], psi[E];
+#pragma unroll
+  for (int i = 0; i < E; ++i) {
+    m[i] = gld(a.mod, mcol_pos<N, TT, E>(cband, pb, pt, i));
+    sv[i] = gld(a.sup, row_pos<N, TT, E>(rband, pb, pt, i));
+    pin[i] = gld(a.psi, row_pos<N, TT, E>(rband, pb, pt, i));
+    w[i] = gld(ipsf, row_pos<N, TT, E>(rband, pb, pt, i));
+  }
+  c32* to_col = ll;
+  c32* to_row = ll + (size_t)N * N;
+  LlWait llw{flag, a.polls, false};
+  constexpr int DELAY = ll_delay<N>();
+  auto cpos = [&](int i) { return (unsigned)col_pos<N, TT, E>(cband, cb, ct, i); };
+  auto rpos = [&](int i) { return (unsigned)row_pos<N, TT, E>(rband, cb, ct, i); };
+  auto emptied = [&]() { ll_emptied(); };
+#pragma unroll 1
+  for (int k = 0; k < nsteps; ++k) {
+    const RStep st = steps[k];
+    const bool err_sum = st.err && errp0, last = k + 1 == nsteps;
+    c32 x[E];
+    __syncthreads();
+    if (k) {
+      ll_take<DELAY>(x, to_col, llw, cpos);
+    } else {
+#pragma unroll
+      for (int i = 0; i < E; ++i) x[i] = xld<3>(a.phi, cpos(i));
+    }
+    tf.template to_private<false>(x);
+    if (k) ll_empty<E>(to_col, cpos);
+#pragma unroll
+    for (int i = 0; i < E; ++i) {
+      psi[i] = x[i];
+      x[i] = c32{fmaf(x[i].x, x[i].x, x[i].y * x[i].y), 0.0f};
+    }
+    tf.template to_coalesced<false>(x, emptied);
+    ll_give(x, to_row, cpos);
+
+    __syncthreads();
+    ll_take<DELAY>(x, to_row, llw, rpos);
+    tf.template to_private<false>(x);
+    ll_empty<E>(to_row, rpos);
+#pragma unroll
+    for (int i = 0; i < E; ++i) x[i] = mul(x[i], w[i]);
+    tf.template to_coalesced<true>(x, emptied);
+    ll_give(x, to_col, rpos);
+
+    __syncthreads();
+    ll_take<DELAY>(x, to_col, llw, cpos);
+    tf.template to_private<true>(x);
+    ll_empty<E>(to_col, cpos);
+    double err = 0.0;
+#pragma unroll
+    for (int i = 0; i < E; ++i) {
+      const float div = sqrtf(sqrtf(fmaf(x[i].x, x[i].x, x[i].y * x[i].y)) * a.inv_nn);
+      const double dd = (double)div - (double)m[i];
+      err = fma(dd, dd, err);
+      x[i] = scale(psi[i], div > 0.0f ? m[i] / div : 0.0f);
+    }
+    if (err_sum) eord[pt * TT + pb] = err;
+    tf.template to_coalesced<true>(x, emptied);
+    ll_give(x, to_row, cpos);
+
+    __syncthreads();
+    if (err_sum) block_sum_waves<NT>(eord, ewave);
+    ll_take<DELAY>(x, to_row, llw, rpos);
+    tf.template to_private<true>(x);
+    ll_empty<E>(to_row, rpos);
+    if (err_sum && tid == 0)
+      errp0[(size_t)st.kidx * errp_step + cband] = block_sum_rest<NT>(ewave);
+#pragma unroll
+    for (int i = 0; i < E; ++i) {
+      pin[i] = update_value<false>(st.c, scale(x[i], a.inv_nn), pin[i], sv[i], c32{0.0f, 0.0f});
+      x[i] = pin[i];
+    }
+    tf.template to_coalesced<false>(x, emptied);
+    if (last) {
+#pragma unroll
+      for (int i = 0; i < E; ++i) xst<3>(a.phi, rpos(i), x[i]);
+    } else {
+      ll_give(x, to_col, rpos);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < E; ++i) gst(a.psi, row_pos<N, TT, E>(rband, pb, pt, i), pin[i]);
 }
 
 // before a resident launch: its barrier flags and give-up flag start at 0; the
@@ -3039,6 +3177,25 @@ static hipError_t resident_nt(int xm, const PassArgs& a, const RStep* steps, int
   return e;
 }
 
+template <int N, int TT, int E>
+static hipError_t resident_ipsf_nt(const PassArgs& a, const c32* ipsf, const RStep* steps,
+                                   int nsteps, double* errp0, long long errp_step, int* flag,
+                                   c32* ll, int fill, hipStream_t st) {
+  hipLaunchKernelGGL(k_resident_begin, dim3(fill ? 1024 : 1), dim3(256), 0, st, nullptr, 0, flag,
+                     reinterpret_cast<u32x2*>(ll), 2 * N * N, fill);
+  void* args[] = {(void*)&a,     (void*)&ipsf,      (void*)&steps, (void*)&nsteps,
+                  (void*)&errp0, (void*)&errp_step, (void*)&flag,  (void*)&ll};
+  if (g_launch_events[0]) (void)hipEventRecord(g_launch_events[0], st);
+  hipError_t e = hipLaunchCooperativeKernel(
+      reinterpret_cast<const void*>(&k_resident_ipsf<N, TT, E>), dim3(N / TT), dim3((N / E) * TT),
+      args, 0, st);
+  if (g_launch_events[0]) {
+    (void)hipEventRecord(g_launch_events[1], st);
+    g_launch_events[0] = g_launch_events[1] = nullptr;
+  }
+  return e;
+}
+
 // the resident form exists for one frame of 64^2 .. 1024^2 in tile 4 with
 // 8 values per thread (one workgroup of at most 512 threads per band, at
 // most 256 bands: one per CU), and for 256^2 and 512^2 also in tile 2 (128
@@ -3057,6 +3214,19 @@ static hipError_t resident_dispatch(int tile, int ept, int xm, const PassArgs& a
         return resident_nt<N, 2, 8>(xm, a, steps, nsteps, errp0, errp_step, bar, flag, ll, fill,
                                     st);
     }
+  }
+  return hipErrorInvalidValue;
+}
+
+template <int N>
+static hipError_t resident_ipsf_dispatch(int tile, int ept, const PassArgs& a, const c32* ipsf,
+                                         const RStep* steps, int nsteps, double* errp0,
+                                         long long errp_step, int* flag, c32* ll, int fill,
+                                         hipStream_t st) {
+  if constexpr (N >= 64 && N <= 1024) {
+    if (tile == 4 && ept == 8)
+      return resident_ipsf_nt<N, 4, 8>(a, ipsf, steps, nsteps, errp0, errp_step, flag, ll, fill,
+                                       st);
   }
   return hipErrorInvalidValue;
 }
@@ -3125,7 +3295,11 @@ constexpr bool shape_ok() {
                        const c32* tw, hipStream_t st);                                      \
   hipError_t resident_##n(int tile, int ept, int xm, const PassArgs& a, const RStep* steps, \
                           int nsteps, double* errp0, long long errp_step, unsigned* bar,    \
-                          int* flag, c32* ll, int fill, hipStream_t st);
+                          int* flag, c32* ll, int fill, hipStream_t st);                   \
+  hipError_t resident_ipsf_##n(int tile, int ept, const PassArgs& a, const c32* ipsf,       \
+                               const RStep* steps, int nsteps, double* errp0,               \
+                               long long errp_step, int* flag, c32* ll, int fill,           \
+                               hipStream_t st);
 
 // a shape that is not built compiles to an error return, not a kernel
 #define SPK_CALL_COL(TT_, E_)                                                   \
@@ -3230,7 +3404,14 @@ constexpr bool shape_ok() {
                           int nsteps, double* errp0, long long errp_step, unsigned* bar,    \
                           int* flag, c32* ll, int fill, hipStream_t st) {                   \
     return resident_dispatch<n>(tile, ept, xm, a, steps, nsteps, errp0, errp_step, bar,     \
-                                flag, ll, fill, st);                                                  \
+                                flag, ll, fill, st);                                        \
+  }                                                                                         \
+  hipError_t resident_ipsf_##n(int tile, int ept, const PassArgs& a, const c32* ipsf,       \
+                               const RStep* steps, int nsteps, double* errp0,               \
+                               long long errp_step, int* flag, c32* ll, int fill,           \
+                               hipStream_t st) {                                            \
+    return resident_ipsf_dispatch<n>(tile, ept, a, ipsf, steps, nsteps, errp0, errp_step,   \
+                                     flag, ll, fill, st);                                   \
   }
 
 SPK_SIZES(SPK_SIZED_DECL)
@@ -3310,6 +3491,14 @@ hipError_t launch_resident(int n, int tile, int ept, int xm, const PassArgs& a,
                            unsigned* bar, int* flag, c32* ll, int fill, hipStream_t st) {
   SPK_SIZE_SWITCH(resident, tile, ept, xm, a, steps, nsteps, errp0, errp_step, bar, flag, ll, fill,
                   st)
+}
+
+hipError_t launch_resident_ipsf(int n, int tile, int ept, const PassArgs& a, const c32* ipsf,
+                                const RStep* steps, int nsteps, double* errp0,
+                                long long errp_step, int* flag, c32* ll, int fill,
+                                hipStream_t st) {
+  SPK_SIZE_SWITCH(resident_ipsf, tile, ept, a, ipsf, steps, nsteps, errp0, errp_step, flag, ll,
+                  fill, st)
 }
 
 hipError_t launch_rowfft(int n, int tile, int ept, int mode, const c32* in, c32* out,
