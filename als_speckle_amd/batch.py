@@ -95,9 +95,10 @@ class phasing_batch:
         sem = _capi.SEM_CODES[semantics]
         steps = [(_capi.ALG_CODES[a], sem, beta, 0.0, 0.0)
                  for a in expand_order(order, iterations)]
+        before = self._plan.resident_counts()[0]
         self._trace = self._plan.iterate(steps, error_trace=error_trace) if steps else None
-        if self._plan.persist and steps:
-            self._plan.check()   # raises if a persistent block's grid barrier gave up
+        if steps and (self._plan.persist or self._plan.resident_counts()[0] != before):
+            self._plan.check()   # raises if a launch gave up waiting for its workgroups
 
     def get_error_trace(self):
         """(iterations, trials) FP64 modulus errors of the last ``iterate``."""

@@ -61,6 +61,24 @@ int default_ept(int n, int tile, int batch) {
   return (n / 8) * tile <= 1024 ? 8 : 16;
 }
 
+// Resident launches of several frames (uniform schedules): a launch holds
+// 2^20 / n^2 frames at once (2^19 at 64^2) and takes more in rounds.  They
+// pay up to three rounds; microseconds per step of all frames on MI355X, one
+// launch per pass / resident:
+//   64^2 x 128 14.7 / 6.0;  128^2 x 64 19.2 / 9.8, x 96 23.5 / 15.2;
+//   256^2 x 4 11.0 / 5.7, x 16 20.1 / 9.9, x 32 25.2 / 19.0, x 48 33.4 / 28.4,
+//   x 64 39.7 / 37.6;  512^2 x 2 14.9 / 6.9, x 4 21.0 / 10.8, x 8 26.8 / 21.3,
+//   x 12 34.3 / 31.8, x 16 40.5 / 42.2;  1024^2 x 2 29.6 / 20.6, x 3 36.6 / 30.8.
+constexpr int kResidentRounds = 3;
+// Steps from which a block runs resident by default: a cooperative launch
+// takes about 20 us more than a plain one and the frames' state goes in and
+// out once per round (4 / 8 steps of one 256^2 frame 49 / 89 us per pass, 60 /
+// 81 resident; of one 1024^2 frame 2 / 4 steps 57 / 100 and 70 / 92; 16 steps
+// of 40 x 256^2 479 and 461).
+int resident_min_steps(int n, int rounds) {
+  return rounds > 1 ? 16 * (rounds - 1) : n >= 1024 ? 3 : 6;
+}
+
 template <class T>
 int dalloc(T** p, size_t count) {
   *p = nullptr;
@@ -153,7 +171,8 @@ struct spk_plan {
   // shrinkwraps fused into the passes where possible (spk_tune.sw_separate = 0)
   bool sw_fuse = true;
   // resident single-frame launches (k_resident) and their exchange mode
-  int resident = 0;
+  int resident = 0;            // frames at once, 0: one launch per pass
+  int resident_min = 2;        // steps of a block that runs resident
   int xm = 0;
   // resident launches: the two exchange buffers of mode 3 (n*n values each),
   // then the barrier flags (a 128-byte line per band)
@@ -571,8 +590,11 @@ int spk_plan_bytes(int n, int batch, int shared, int options, size_t* bytes) {
   if ((options & SPK_PB_DM) && (options & SPK_PB_SPECTRUM)) b += 2 * nn * batch * sizeof(float);
   if (options & SPK_PB_TRACE) b += 64 * (size_t)batch * bands * sizeof(double);
   b += 64 * 1024;                                      // step-table staging
-  if (batch == 1 && resident_supported(n, default_tile(n), default_ept(n, default_tile(n), 1)))
-    b += 2 * nn * sizeof(c32) + bands * 128;           // resident launches' exchange
+  // resident launches' exchange, for the frames that a launch holds at once
+  const int tile = default_tile(n);
+  const size_t fit = std::max<size_t>(1, ((size_t)1 << 20) / nn);
+  if (resident_supported(n, tile, default_ept(n, tile, batch)) && batch <= kResidentRounds * fit)
+    b += std::min<size_t>(batch, fit) * (2 * nn * sizeof(c32) + bands * 128);
   *bytes = b;
   return SPK_OK;
 }
@@ -603,13 +625,27 @@ int spk_plan_create(spk_ctx* ctx, int n, int batch, int shared, const spk_tune* 
   p->bands = n / tile;
   p->persist = (tune && tune->persist > 0) ? 1 : 0;
   p->phib_g.assign(batch, 0.0f);
-  // resident launches by default for one frame where they are built: half to
-  // two thirds of the time of one launch per pass from 64^2 to 1024^2 on
-  // MI355X; the exchange of Phi by polled values is the default (the barrier
-  // forms are slower, the fenced ones most)
-  const int res_mode = tune ? tune->resident : 0;
-  p->resident = (res_mode != 2 && batch == 1 && resident_supported(n, tile, ept)) ? 1 : 0;
+  // resident launches by default where they are built and pay: one frame of
+  // 64^2 to 1024^2 takes about half the time of one launch per pass on
+  // MI355X, several see kResidentRounds; the exchange of Phi by polled values
+  // is the default (the barrier forms are slower, the fenced ones most)
   p->xm = (tune && tune->exchange >= 1 && tune->exchange <= 4) ? tune->exchange - 1 : 3;
+  const int res_mode = tune ? tune->resident : 0;
+  if (res_mode != 2 && resident_supported(n, tile, ept)) {
+    int fit = 1;
+    // (the occupancy query only where the answer can matter)
+    const bool few = batch <= kResidentRounds * std::max(1, (1 << 20) / (n * n));
+    if (batch > 1 && (p->xm != 3 || !(few || res_mode == 1) ||
+                      resident_frames(n, tile, ept, &fit) != hipSuccess))
+      fit = 0;
+    const int rounds = fit ? (batch + fit - 1) / fit : 0;
+    if (rounds && (rounds <= kResidentRounds || res_mode == 1)) {
+      p->resident = (batch + rounds - 1) / rounds;   // as even as they go
+      // a caller that asks for the form or its exchange gets it for any block
+      const bool asked = res_mode == 1 || (tune && tune->exchange > 0);
+      p->resident_min = asked ? 2 : resident_min_steps(n, rounds);
+    }
+  }
   p->polls = (tune && tune->barrier_polls > 0) ? (unsigned)tune->barrier_polls : (1u << 18);
   p->sw_fuse = !(tune && tune->sw_separate > 0);
   const size_t nn = (size_t)n * n;
@@ -1101,8 +1137,8 @@ int iter_prepare(spk_plan* p, const spk_step* steps, int nsteps, int per_frame,
   // With an ipsf the block is k_resident_ipsf's (tile 4, exchange mode 3), and
   // ends at every shrinkwrap; with a spectrum there is none (the rescaled map
   // is gathered from all over the frame).
-  if (blocks && p->resident && B == 1 && !p->spec_on && !p->persist && !p->capturing &&
-      (!p->ipsf_on || (p->xm == 3 && p->tile == 4))) {
+  if (blocks && p->resident && (B == 1 || !per_frame) && !p->spec_on && !p->persist &&
+      !p->capturing && (!p->ipsf_on || (B == 1 && p->xm == 3 && p->tile == 4))) {
     auto fits = [&](int j) { return !any_dm[j] && !emits[j]; };
     std::vector<RStep> rs;
     std::vector<SwParam> sp;
@@ -1126,7 +1162,7 @@ int iter_prepare(spk_plan* p, const spk_step* steps, int nsteps, int per_frame,
           int nx = j + 1;
           while (nx < nsteps && fits(nx) && !act[(size_t)nx * W]) ++nx;
           const bool goes_on = nx < nsteps && fits(nx);
-          if (!goes_on || sw_r[j] > kSwFuseRmax || !p->sw_fuse || p->ipsf_on) {
+          if (!goes_on || sw_r[j] > kSwFuseRmax || !p->sw_fuse || p->ipsf_on || B > 1) {
             rs.push_back(rsj);
             break;                        // stand-alone shrinkwrap after the block
           }
@@ -1138,7 +1174,8 @@ int iter_prepare(spk_plan* p, const spk_step* steps, int nsteps, int per_frame,
         }
         rs.push_back(rsj);
       }
-      if (rs.size() >= 2) {
+      // an ipsf step saves more: four launches per pass, from 16 us at 64^2
+      if ((int)rs.size() >= (p->ipsf_on ? 2 : p->resident_min)) {
         res_end[k] = k1;
         r.res_n[k] = (int)rs.size();
         r.res_fused[k] = fused;
@@ -1321,25 +1358,27 @@ int iter_step(IterRun& r, int k, int* next) {
   *next = k + 1;
   if (r.res_end[k]) {
     const int k1 = r.res_end[k];
-    // one allocation: the exchange buffers of mode 3, then the barrier flags
-    const size_t ll = p->xm == 3 ? 2 * (size_t)p->nn() : 0;
-    if (!p->rll && (rc = dalloc(&p->rll, ll + (size_t)p->bands * 16))) return rc;
-    const int fill = p->rll_fill;
-    p->rll_fill = false;
+    // one allocation: the exchange buffers of mode 3, then the barrier flags,
+    // for the frames that a launch runs at once
+    const int g = p->resident;
+    const size_t ll = p->xm == 3 ? (size_t)g * 2 * p->nn() : 0;
+    if (!p->rll && (rc = dalloc(&p->rll, ll + (size_t)g * p->bands * 16))) return rc;
     unsigned* rsync = reinterpret_cast<unsigned*>(p->rll + ll);
-    if ((rc = prof_arm(p, 2))) return rc;
     PassArgs ra = base_args(p);
     ra.swr_tab = r.res_fused[k] ? (const SwParam*)r.dptr(r.res_sw_off[k]) : nullptr;
+    const int fill = p->rll_fill;
+    p->rll_fill = false;
+    if ((rc = prof_arm(p, 2))) return rc;
+    double* errp = r.err_trace ? p->errp : nullptr;
+    const RStep* tab = (const RStep*)r.dptr(r.res_off[k]);
     if (p->ipsf_on)
-      SPK_HIP(launch_resident_ipsf(p->n, p->tile, p->ept, ra, p->ipsf,
-                                   (const RStep*)r.dptr(r.res_off[k]), r.res_n[k],
-                                   r.err_trace ? p->errp : nullptr, (long long)B * p->bands,
-                                   (int*)(p->pbar + 1), p->rll, fill, st));
+      SPK_HIP(launch_resident_ipsf(p->n, p->tile, p->ept, ra, p->ipsf, tab, r.res_n[k], errp,
+                                   (long long)B * p->bands, (int*)(p->pbar + 1), p->rll, fill,
+                                   st));
     else
-      SPK_HIP(launch_resident(p->n, p->tile, p->ept, p->xm, ra,
-                              (const RStep*)r.dptr(r.res_off[k]), r.res_n[k],
-                              r.err_trace ? p->errp : nullptr, (long long)B * p->bands, rsync,
-                              (int*)(p->pbar + 1), p->rll, fill, st));
+      SPK_HIP(launch_resident(p->n, p->tile, p->ept, p->xm, ra, tab, r.res_n[k], errp,
+                              (long long)B * p->bands, rsync, (int*)(p->pbar + 1), p->rll, fill,
+                              B, g, st));
     p->res_launches++;
     p->res_steps += r.res_n[k];
     p->sw_fused_count += r.res_fused[k];

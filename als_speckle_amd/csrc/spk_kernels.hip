@@ -1146,21 +1146,19 @@ __device__ __forceinline__ void sw_store_staged_x(const float* stage, float* dst
 // `limit` poll rounds flag[0] (this launch's) and flag[1] (sticky) are set
 // and every later wait of the launch passes.
 template <int XM>
-__device__ __forceinline__ void resident_arrive(unsigned* flags, unsigned epoch) {
+__device__ __forceinline__ void resident_arrive(unsigned* flags, int self, unsigned epoch) {
   constexpr int LINE = 32;   // unsigned words per 128-byte line
   __builtin_amdgcn_s_waitcnt(0x0F70);   // this wave's stores have completed
   __syncthreads();
   if (threadIdx.x == 0) {
     if (XM < 2) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
-    __hip_atomic_store(flags + blockIdx.x * LINE, epoch, __ATOMIC_RELAXED,
-                       __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(flags + self * LINE, epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
-template <int XM, int K>
+template <int XM, int NB>
 __device__ __forceinline__ void resident_wait(unsigned* flags, unsigned epoch, int* flag,
                                               unsigned limit) {
-  static_assert(K >= 1, "at least one flag per polling lane");
-  constexpr int LINE = 32;
+  constexpr int LINE = 32, K = (NB + 63) / 64;
   if (threadIdx.x < 64) {
     bool gave = __hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
     unsigned polls = 0;
@@ -1170,7 +1168,7 @@ __device__ __forceinline__ void resident_wait(unsigned* flags, unsigned epoch, i
       unsigned v[K];
 #pragma unroll
       for (int q = 0; q < K; ++q) {
-        const unsigned j = min(threadIdx.x + q * 64u, gridDim.x - 1u);
+        const unsigned j = min(threadIdx.x + q * 64u, NB - 1u);
         v[q] = __hip_atomic_load(flags + j * LINE, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
       bool done = true;
@@ -1188,11 +1186,11 @@ __device__ __forceinline__ void resident_wait(unsigned* flags, unsigned epoch, i
   }
   __syncthreads();
 }
-template <int XM, int K>
-__device__ __forceinline__ void resident_sync(unsigned* flags, unsigned epoch, int* flag,
+template <int XM, int NB>
+__device__ __forceinline__ void resident_sync(unsigned* flags, int self, unsigned epoch, int* flag,
                                               unsigned limit) {
-  resident_arrive<XM>(flags, epoch);
-  resident_wait<XM, K>(flags, epoch, flag, limit);
+  resident_arrive<XM>(flags, self, epoch);
+  resident_wait<XM, NB>(flags, epoch, flag, limit);
 }
 
 // Exchange mode 3: the data are their own flags.  Phi crosses in two buffers
@@ -1500,29 +1498,33 @@ template <int N>
 constexpr int ll_delay() { return N >= 1024 ? 24 : 2; }
 
 // LDS of the resident kernel: the transforms' regions and the shrinkwrap lines,
-// padded so that one workgroup occupies a CU (the grid is one workgroup per
-// band, at most one per CU)
+// for one frame padded so that one workgroup occupies a CU (the grid is one
+// workgroup per band, at most one per CU)
 template <int N, int TT>
 constexpr int resident_base() {   // c32 slots before the error sums
   return LineFft<N, TT>::LDS + (sw_lds_floats<N, TT>() + 32 + 1) / 2;
 }
 template <int N, int TT>
+constexpr int resident_used() {
+  return resident_base<N, TT>() + (N / 8 * TT > 64 ? N / 8 * TT : 64) + 16;
+}
+template <int N, int TT>
 constexpr int resident_lds_elems() {
-  constexpr int base = resident_base<N, TT>() + (N / 8 * TT > 64 ? N / 8 * TT : 64) + 16;
+  constexpr int base = resident_used<N, TT>();
   constexpr int half = (kLdsBytes / 2) / 8 + 64;   // more than half a CU's LDS
   return base > half ? base : half;
 }
 
-template <int N, int TT, int E, int XM>
-__global__ void __launch_bounds__((N / E) * TT)
+template <int N, int TT, int E, int XM, bool MANY>
+__global__ void __launch_bounds__((N / E) * TT, 2)
     k_resident(PassArgs a, const RStep* __restrict__ steps, int nsteps, double* errp0,
-               long long errp_step, unsigned* flags, int* flag, c32* ll) {
+               long long errp_step, unsigned* flags, int* flag, c32* ll, int nframes) {
   constexpr int NT = (N / E) * TT;
   constexpr int NB = N / TT;
   constexpr int T = N / E;
   using LF = LineFft<N, TT>;
   static_assert(E == LF::E && LdsPlan<N, TT>::FULL_TW, "8 values per thread, the whole table");
-  __shared__ c32 lds[resident_lds_elems<N, TT>()];
+  __shared__ c32 lds[MANY ? resident_used<N, TT>() : resident_lds_elems<N, TT>()];
   static_assert(sizeof(lds) <= kLdsBytes, "resident kernel does not fit in LDS");
   // the shrinkwrap blur lines, staged outputs and weights, the reductions'
   // scratch (and the twiddle table until the threads have taken theirs)
@@ -1533,8 +1535,13 @@ __global__ void __launch_bounds__((N / E) * TT)
   double* eord = reinterpret_cast<double*>(lds + resident_base<N, TT>());
   double* ewave = eord + (NT > 64 ? NT : 64);
   const int tid = threadIdx.x;
-  const int cband = xcd_band<NB>(blockIdx.x);   // as k_colpass
-  const int rband = blockIdx.x;                 // as k_rowpass
+  const int fl = MANY ? blockIdx.x / NB : 0;    // frame of the launch
+  const int rband = MANY ? blockIdx.x % NB : blockIdx.x;   // as k_rowpass
+  const int cband = xcd_band<NB>(rband);        // as k_colpass
+  if constexpr (MANY) {
+    flags += fl * NB * 32;
+    ll += (size_t)fl * 2 * N * N;
+  }
   LF tf;
   {
     TwStage<N, TT, NT> tws;
@@ -1544,22 +1551,34 @@ __global__ void __launch_bounds__((N / E) * TT)
     tf.init(lds, reinterpret_cast<const c32*>(swl));
   }
   const int cb = tf.cb, ct = tf.ct, pb = tf.pb, pt = tf.pt;
+  // several frames: NB workgroups per frame at a time, each group its frames
+  // fl, fl + groups, ... one after the other
+  unsigned epoch = 0;
+  LlWait llw{flag, a.polls, false};
+#pragma unroll 1
+  for (int f = fl; f < (MANY ? nframes : 1); f += MANY ? gridDim.x / NB : 1) {
+  const float* mod = a.mod + (MANY ? (size_t)f * a.mstride : 0);
+  float* sup = const_cast<float*>(a.sup) + (MANY ? (size_t)f * a.sstride : 0);
+  const size_t fo = MANY ? (size_t)f * N * N : 0;
+  c32* phi = a.phi + fo;
+  c32* psi = a.psi + fo;
+  float* sw_tmp = a.sw_tmp + fo;
+  float* sw_blur = a.sw_blur + fo;
+  float* sw_maxp = a.sw_maxp + (MANY ? (size_t)f * NB : 0);
+  double* errp = errp0 ? errp0 + (MANY ? (size_t)f * NB : 0) : nullptr;
   // resident state, private mapping: modulus of the column band, support and
   // iterate of the row band
   float m[E], sv[E];
   c32 pin[E];
 #pragma unroll
   for (int i = 0; i < E; ++i) {
-    m[i] = gld(a.mod, mcol_pos<N, TT, E>(cband, pb, pt, i));
-    sv[i] = gld(a.sup, row_pos<N, TT, E>(rband, pb, pt, i));
-    pin[i] = gld(a.psi, row_pos<N, TT, E>(rband, pb, pt, i));
+    m[i] = gld(mod, mcol_pos<N, TT, E>(cband, pb, pt, i));
+    sv[i] = gld(sup, row_pos<N, TT, E>(rband, pb, pt, i));
+    pin[i] = gld(psi, row_pos<N, TT, E>(rband, pb, pt, i));
   }
-  c32* phi = a.phi;
   constexpr bool LL = XM == 3;
-  constexpr int KF = (NB + 63) / 64;
   c32* to_col = ll;                       // mode 3: row phase -> column phase
   c32* to_row = ll + (size_t)N * N;       // column phase -> row phase
-  LlWait llw{flag, a.polls, false};
   constexpr int DELAY = ll_delay<N>();
   bool given = false;   // mode 3: to_col holds the step's Phi (else phi does)
   auto cpos = [&](int i) { return (unsigned)col_pos<N, TT, E>(cband, cb, ct, i); };
@@ -1568,18 +1587,18 @@ __global__ void __launch_bounds__((N / E) * TT)
   auto has_col = [&](const RStep& q) {
     return !(q.c.flags & kNoOut) || q.err || (q.c.flags & kSwFin);
   };
-  unsigned epoch = 0;
   bool sup_changed = false;
   for (int k = 0; k < nsteps; ++k) {
     const RStep st = steps[k];
     const bool noout = (st.c.flags & kNoOut) != 0;
-    const bool swrow = (st.c.flags & kSwRow) != 0;   // shrinkwrap after this step
-    const bool swfin = (st.c.flags & kSwFin) != 0;   // ... after the previous one
+    // a fused shrinkwrap after this step, after the previous one (one frame)
+    const bool swrow = !MANY && (st.c.flags & kSwRow) != 0;
+    const bool swfin = !MANY && (st.c.flags & kSwFin) != 0;
     const bool col = has_col(st);
     const bool last = k + 1 == nsteps;
     // mode 3: the new Phi is formed only where something reads it
     const bool emit = !LL || last || has_col(steps[last ? k : k + 1]);
-    const bool err_sum = col && st.err && errp0;
+    const bool err_sum = col && st.err && errp;
     c32 x[E];
     if (col) {
       // column phase (colpass_item MODE 0, MODE 10 for kNoOut, MODE 9's blur)
@@ -1606,9 +1625,9 @@ __global__ void __launch_bounds__((N / E) * TT)
       // transform (as colpass_item MODE 9)
       float rb[E];
       if (swfin) {
-        if (LL) resident_wait<XM, KF>(flags, epoch, flag, a.polls);
+        if (LL) resident_wait<XM, NB>(flags, epoch, flag, a.polls);
 #pragma unroll
-        for (int i = 0; i < E; ++i) rb[i] = xldf<XM>(a.sw_tmp, cpos(i));
+        for (int i = 0; i < E; ++i) rb[i] = xldf<XM>(sw_tmp, cpos(i));
       }
       if (!noout) {
         tf.template to_coalesced<true>(x, [&]() { if (LL) ll_emptied(); });
@@ -1633,17 +1652,17 @@ __global__ void __launch_bounds__((N / E) * TT)
           stage[sw_swz((row / TT) * (TT * TT) + (row % TT) * TT + l)] = v;
         });
         __syncthreads();
-        sw_store_staged_x<N, TT, XM>(stage, a.sw_blur, [&](int v) {
+        sw_store_staged_x<N, TT, XM>(stage, sw_blur, [&](int v) {
           const int q = (4 * v) / (TT * TT), within = (4 * v) % (TT * TT);
           return (q * NB + cband) * (TT * TT) + within;
         });
         const float bm = block_max(mx, swl);
-        if (tid == 0) xstf<XM>(a.sw_maxp, cband, bm);
+        if (tid == 0) xstf<XM>(sw_maxp, cband, bm);
       }
       // mode 3: a barrier only for the shrinkwrap maps, and where the row
       // phase does not wait for this phase's Phi but overwrites its input
-      if (!LL) resident_sync<XM, KF>(flags, ++epoch, flag, a.polls);
-      else if (swfin || noout) resident_arrive<XM>(flags, ++epoch);
+      if (!LL) resident_sync<XM, NB>(flags, rband, ++epoch, flag, a.polls);
+      else if (swfin || noout) resident_arrive<XM>(flags, rband, ++epoch);
     }
     // row phase (rowpass_item; kNoOut skips Phi).  Every load is issued
     // first: Phi, the band maxima and blur of a fused shrinkwrap's threshold,
@@ -1662,7 +1681,7 @@ __global__ void __launch_bounds__((N / E) * TT)
       }
     }
     if (!LL || noout) err_waves();
-    if (LL && swfin) resident_wait<XM, KF>(flags, epoch, flag, a.polls);
+    if (LL && swfin) resident_wait<XM, NB>(flags, epoch, flag, a.polls);
     float wrow = 0.0f;
     if (swrow) wrow = sw_weight_fetch(a.swr_tab[st.swr].w);
     if (swfin) {
@@ -1675,10 +1694,10 @@ __global__ void __launch_bounds__((N / E) * TT)
 #pragma unroll
       for (int j = 0; j < MPT; ++j) {
         const int q = tid + j * NT;
-        if (q < NB) mx = fmaxf(mx, xldf<XM>(a.sw_maxp, q));
+        if (q < NB) mx = fmaxf(mx, xldf<XM>(sw_maxp, q));
       }
 #pragma unroll
-      for (int i = 0; i < E; ++i) bl[i] = xldf<XM>(a.sw_blur, rpos(i));
+      for (int i = 0; i < E; ++i) bl[i] = xldf<XM>(sw_blur, rpos(i));
       const double thr = (double)a.swr_tab[st.swf].tau * (double)block_max(mx, swl);
       __syncthreads();
 #pragma unroll
@@ -1697,7 +1716,7 @@ __global__ void __launch_bounds__((N / E) * TT)
       __syncthreads();
     }
     if (err_sum && tid == 0)
-      errp0[(size_t)st.kidx * errp_step + cband] = block_sum_rest<NT>(ewave);
+      errp[(size_t)st.kidx * errp_step + cband] = block_sum_rest<NT>(ewave);
 #pragma unroll
     for (int i = 0; i < E; ++i) {
       const c32 pout = noout ? c32{0.0f, 0.0f} : scale(x[i], a.inv_nn);
@@ -1706,7 +1725,7 @@ __global__ void __launch_bounds__((N / E) * TT)
     }
     if (emit) {
       tf.template to_coalesced<false>(x, [&]() { if (LL) ll_emptied(); });
-      if (LL && noout && col && !swfin) resident_wait<XM, KF>(flags, epoch, flag, a.polls);
+      if (LL && noout && col && !swfin) resident_wait<XM, NB>(flags, epoch, flag, a.polls);
       if (LL && !last) {
         ll_give(x, to_col, rpos);
         given = true;
@@ -1730,21 +1749,24 @@ __global__ void __launch_bounds__((N / E) * TT)
         stage[sw_swz((c / TT) * (TT * TT) + l * TT + (c % TT))] = v;
       });
       __syncthreads();
-      sw_store_staged_x<N, TT, XM>(stage, a.sw_tmp + (size_t)rband * N * TT,
+      sw_store_staged_x<N, TT, XM>(stage, sw_tmp + (size_t)rband * N * TT,
                                    [](int v) { return 4 * v; });
     }
     if (!LL) {
-      if (!last) resident_sync<XM, KF>(flags, ++epoch, flag, a.polls);
+      if (!last) resident_sync<XM, NB>(flags, rband, ++epoch, flag, a.polls);
     } else if (swrow) {
-      resident_arrive<XM>(flags, ++epoch);
+      resident_arrive<XM>(flags, rband, ++epoch);
     }
   }
 #pragma unroll
-  for (int i = 0; i < E; ++i) gst(a.psi, row_pos<N, TT, E>(rband, pb, pt, i), pin[i]);
+  for (int i = 0; i < E; ++i) gst(psi, row_pos<N, TT, E>(rband, pb, pt, i), pin[i]);
   if (sup_changed) {
-    float* sup = const_cast<float*>(a.sup);
 #pragma unroll
     for (int i = 0; i < E; ++i) gst(sup, row_pos<N, TT, E>(rband, pb, pt, i), sv[i]);
+  }
+  // the group's exchange buffers, flags and LDS are free for its next frame
+  // once every workgroup of the group is here
+  if constexpr (MANY) resident_sync<XM, NB>(flags, rband, ++epoch, flag, a.polls);
   }
 }
 
@@ -3155,25 +3177,40 @@ static hipError_t tfcol_nt(int kind, const c32* phi, const float* goal, int rows
 template <int N, int TT, int E>
 static hipError_t resident_nt(int xm, const PassArgs& a, const RStep* steps, int nsteps,
                               double* errp0, long long errp_step, unsigned* flags, int* flag,
-                              c32* ll, int fill, hipStream_t st) {
-  const int words = (N / TT) * 32, count = xm == 3 ? 2 * N * N : 0;
+                              c32* ll, int fill, int frames, int at_once, hipStream_t st) {
+  const int words = at_once * (N / TT) * 32, count = xm == 3 ? at_once * 2 * N * N : 0;
   const int blocks = fill && count ? 1024 : std::max(1, words / 256);
   hipLaunchKernelGGL(k_resident_begin, dim3(blocks), dim3(256), 0, st, flags, words, flag,
                      reinterpret_cast<u32x2*>(ll), count, fill);
   void* args[] = {(void*)&a,     (void*)&steps, (void*)&nsteps, (void*)&errp0, (void*)&errp_step,
-                  (void*)&flags, (void*)&flag,  (void*)&ll};
-  const void* fn = xm == 1   ? reinterpret_cast<const void*>(&k_resident<N, TT, E, 1>)
-                   : xm == 2 ? reinterpret_cast<const void*>(&k_resident<N, TT, E, 2>)
-                   : xm == 3 ? reinterpret_cast<const void*>(&k_resident<N, TT, E, 3>)
-                             : reinterpret_cast<const void*>(&k_resident<N, TT, E, 0>);
+                  (void*)&flags, (void*)&flag,  (void*)&ll,     (void*)&frames};
+  const void* fn = frames > 1 ? reinterpret_cast<const void*>(&k_resident<N, TT, E, 3, true>)
+                   : xm == 1 ? reinterpret_cast<const void*>(&k_resident<N, TT, E, 1, false>)
+                   : xm == 2 ? reinterpret_cast<const void*>(&k_resident<N, TT, E, 2, false>)
+                   : xm == 3 ? reinterpret_cast<const void*>(&k_resident<N, TT, E, 3, false>)
+                             : reinterpret_cast<const void*>(&k_resident<N, TT, E, 0, false>);
   if (g_launch_events[0]) {
     (void)hipEventRecord(g_launch_events[0], st);
   }
-  hipError_t e = hipLaunchCooperativeKernel(fn, dim3(N / TT), dim3((N / E) * TT), args, 0, st);
+  hipError_t e =
+      hipLaunchCooperativeKernel(fn, dim3(at_once * (N / TT)), dim3((N / E) * TT), args, 0, st);
   if (g_launch_events[0]) {
     (void)hipEventRecord(g_launch_events[1], st);
     g_launch_events[0] = g_launch_events[1] = nullptr;
   }
+  return e;
+}
+
+// frames that one launch of several holds at once on the current device
+template <int N, int TT, int E>
+static hipError_t resident_frames_nt(int* out) {
+  int occ = 0, dev = 0, cus = 0;
+  hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
+      &occ, reinterpret_cast<const void*>(&k_resident<N, TT, E, 3, true>), (N / E) * TT, 0);
+  if (e == hipSuccess) e = hipGetDevice(&dev);
+  if (e == hipSuccess)
+    e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+  if (e == hipSuccess) *out = occ * cus / (N / TT);
   return e;
 }
 
@@ -3204,15 +3241,26 @@ template <int N>
 static hipError_t resident_dispatch(int tile, int ept, int xm, const PassArgs& a,
                                     const RStep* steps, int nsteps, double* errp0,
                                     long long errp_step, unsigned* bar, int* flag, c32* ll,
-                                    int fill, hipStream_t st) {
+                                    int fill, int frames, int at_once, hipStream_t st) {
   if constexpr (N >= 64 && N <= 1024) {
     if (tile == 4 && ept == 8)
       return resident_nt<N, 4, 8>(xm, a, steps, nsteps, errp0, errp_step, bar, flag, ll, fill,
-                                  st);
+                                  frames, at_once, st);
     if constexpr (N >= 256 && N <= 512) {
       if (tile == 2 && ept == 8)
         return resident_nt<N, 2, 8>(xm, a, steps, nsteps, errp0, errp_step, bar, flag, ll, fill,
-                                    st);
+                                    frames, at_once, st);
+    }
+  }
+  return hipErrorInvalidValue;
+}
+
+template <int N>
+static hipError_t resident_frames_dispatch(int tile, int ept, int* out) {
+  if constexpr (N >= 64 && N <= 1024) {
+    if (tile == 4 && ept == 8) return resident_frames_nt<N, 4, 8>(out);
+    if constexpr (N >= 256 && N <= 512) {
+      if (tile == 2 && ept == 8) return resident_frames_nt<N, 2, 8>(out);
     }
   }
   return hipErrorInvalidValue;
@@ -3295,7 +3343,9 @@ constexpr bool shape_ok() {
                        const c32* tw, hipStream_t st);                                      \
   hipError_t resident_##n(int tile, int ept, int xm, const PassArgs& a, const RStep* steps, \
                           int nsteps, double* errp0, long long errp_step, unsigned* bar,    \
-                          int* flag, c32* ll, int fill, hipStream_t st);                   \
+                          int* flag, c32* ll, int fill, int frames, int at_once,                 \
+                          hipStream_t st);                                                  \
+  hipError_t resident_frames_##n(int tile, int ept, int* out);                              \
   hipError_t resident_ipsf_##n(int tile, int ept, const PassArgs& a, const c32* ipsf,       \
                                const RStep* steps, int nsteps, double* errp0,               \
                                long long errp_step, int* flag, c32* ll, int fill,           \
@@ -3402,9 +3452,13 @@ constexpr bool shape_ok() {
   }                                                                                         \
   hipError_t resident_##n(int tile, int ept, int xm, const PassArgs& a, const RStep* steps, \
                           int nsteps, double* errp0, long long errp_step, unsigned* bar,    \
-                          int* flag, c32* ll, int fill, hipStream_t st) {                   \
+                          int* flag, c32* ll, int fill, int frames, int at_once,                 \
+                          hipStream_t st) {                                                 \
     return resident_dispatch<n>(tile, ept, xm, a, steps, nsteps, errp0, errp_step, bar,     \
-                                flag, ll, fill, st);                                        \
+                                flag, ll, fill, frames, at_once, st);                            \
+  }                                                                                         \
+  hipError_t resident_frames_##n(int tile, int ept, int* out) {                             \
+    return resident_frames_dispatch<n>(tile, ept, out);                                     \
   }                                                                                         \
   hipError_t resident_ipsf_##n(int tile, int ept, const PassArgs& a, const c32* ipsf,       \
                                const RStep* steps, int nsteps, double* errp0,               \
@@ -3488,9 +3542,14 @@ bool resident_supported(int n, int tile, int ept) {
 
 hipError_t launch_resident(int n, int tile, int ept, int xm, const PassArgs& a,
                            const RStep* steps, int nsteps, double* errp0, long long errp_step,
-                           unsigned* bar, int* flag, c32* ll, int fill, hipStream_t st) {
+                           unsigned* bar, int* flag, c32* ll, int fill, int frames, int at_once,
+                           hipStream_t st) {
   SPK_SIZE_SWITCH(resident, tile, ept, xm, a, steps, nsteps, errp0, errp_step, bar, flag, ll, fill,
-                  st)
+                  frames, at_once, st)
+}
+
+hipError_t resident_frames(int n, int tile, int ept, int* out) {
+  SPK_SIZE_SWITCH(resident_frames, tile, ept, out)
 }
 
 hipError_t launch_resident_ipsf(int n, int tile, int ept, const PassArgs& a, const c32* ipsf,

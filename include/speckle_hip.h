@@ -73,11 +73,14 @@ typedef struct spk_tune {
                          thread: runs of non-DM steps run as one cooperative
                          resident launch each (the frame's modulus, support
                          and iterate held on chip, Phi exchanged between the
-                         workgroups, shrinkwraps inside the launch); 0 or
-                         1: where built (the default), 2: never.  A resident
-                         launch needs the whole device: no other cooperative
-                         launch may run beside it (spk_plan_check reports a
-                         wait that gave up)                                  */
+                         workgroups, shrinkwraps of a single frame inside the
+                         launch); plans of several frames with per_frame = 0
+                         too, a few at a time, up to three rounds.  0: where
+                         it pays (the default: not for blocks of a few steps,
+                         many frames), 1: where built, 2: never.  The
+                         workgroups of a launch wait for each other: it is a
+                         cooperative launch (spk_plan_check reports a wait
+                         that gave up)                                       */
   int32_t exchange;   /* resident launches: how Phi crosses between workgroups,
                          1 plain + barrier with device-scope fences, 2
                          device-scope accesses + fences, 3 device-scope

@@ -69,7 +69,7 @@ def test_values_that_look_empty(gpu_ctx, n):
     """A guess full of the empty slot's pattern (a NaN) still ends every wait."""
     f, g = case(n)
     g.view(np.uint32)[...] = 0xFFFFFFFF
-    out, counts = run(gpu_ctx, f, g, [[HIO] * 4, [ER] * 3 + [HIO]], True)
+    out, counts = run(gpu_ctx, f, g, [[HIO] * 4, [ER] * 3 + [HIO]], True, exchange=4)
     assert counts[0] == 2 and np.isnan(out[0]).all() and np.isnan(out[2]).all()
 
 
@@ -80,7 +80,7 @@ def test_same_plan_after_a_launch_that_gave_up(gpu_ctx):
     n = 256
     f, g = case(n)
     want, _ = run(gpu_ctx, f, g, [[HIO] * 3], True, resident=2)
-    p = Plan(gpu_ctx, n, barrier_polls=1)
+    p = Plan(gpu_ctx, n, barrier_polls=1, exchange=4)
     p.set_modulus(torch.from_numpy(f.modulus).cuda())
     ok = 0
     for _ in range(3):
@@ -95,5 +95,5 @@ def test_same_plan_after_a_launch_that_gave_up(gpu_ctx):
         ok += 1
         assert np.array_equal(p.get_psi().cpu().numpy(), want[0])
     p.close()
-    again, _ = run(gpu_ctx, f, g, [[HIO] * 3], True)
+    again, _ = run(gpu_ctx, f, g, [[HIO] * 3], True, exchange=4)
     assert np.array_equal(again[0], want[0])
