@@ -173,6 +173,7 @@ struct spk_plan {
   // resident single-frame launches (k_resident) and their exchange mode
   int resident = 0;            // frames at once, 0: one launch per pass
   int resident_min = 2;        // steps of a block that runs resident
+  bool res_allowed = true;     // spk_tune.resident != 2
   int xm = 0;
   // resident launches: the two exchange buffers of mode 3 (n*n values each),
   // then the barrier flags (a 128-byte line per band)
@@ -631,6 +632,7 @@ int spk_plan_create(spk_ctx* ctx, int n, int batch, int shared, const spk_tune* 
   // is the default (the barrier forms are slower, the fenced ones most)
   p->xm = (tune && tune->exchange >= 1 && tune->exchange <= 4) ? tune->exchange - 1 : 3;
   const int res_mode = tune ? tune->resident : 0;
+  p->res_allowed = res_mode != 2;
   if (res_mode != 2 && resident_supported(n, tile, ept)) {
     int fit = 1;
     // (the occupancy query only where the answer can matter)
@@ -2003,7 +2005,14 @@ int spk_coherence_rl(spk_plan* p, const float* est, int rows, int cols, const fl
   // u = the start Gaussian of widths n/4 (phasing.py:818)
   const double w0 = (double)(n / 4);
   SPK_HIP(launch_coh(7, n, tile, nullptr, nullptr, u, nullptr, nullptr, nullptr, 0, 0, w0, w0, st));
-  for (int it = 0; it < iterations; ++it) {
+  // the updates in one launch where the resident form is built (W and w hold
+  // its exchange), otherwise as launches
+  const bool one = iterations > 0 && p->res_allowed && p->xm == 3 && tile == 4 && !p->capturing &&
+                   resident_supported(n, tile, p->ept);
+  if (one)
+    SPK_HIP(launch_resident_rl(n, tile, p->ept, p->tw, u, d, P, Ph, iterations, inv_nn, p->polls,
+                               (int*)(p->pbar + 1), W, st));
+  for (int it = 0; it < iterations && !one; ++it) {
     // blur = ifft2(fft2(u) P); w = d / blur; w = ifft2(fft2(w) Ph); u *= w
     // (phasing.py:700-736); the inverse transforms are unnormalised, 1/n^2
     // is applied in the elementwise steps

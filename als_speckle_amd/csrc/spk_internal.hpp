@@ -212,6 +212,12 @@ hipError_t launch_resident_ipsf(int n, int tile, int ept, const PassArgs& a, con
                                 const RStep* steps, int nsteps, double* errp0,
                                 long long errp_step, int* flag, c32* ll, int fill,
                                 hipStream_t st);
+// `iterations` Richardson-Lucy updates of u (tiled; d, P, Ph tiled) in one
+// cooperative launch (k_resident_rl; tile 4, 8 values per thread, 64 <= n <=
+// 1024); ll: two n*n exchange buffers, emptied first; flag as launch_resident's
+hipError_t launch_resident_rl(int n, int tile, int ept, const c32* tw, c32* u, const float* d,
+                              const c32* P, const c32* Ph, int iterations, float inv_nn,
+                              unsigned polls, int* flag, c32* ll, hipStream_t st);
 // workgroups of the persistent kernel that fit on the current device at once
 hipError_t persist_grid(int n, int tile, int ept, int* out);
 // mode 0: out = rowFFT(in); 1: out = rowIFFT(in) (unscaled);

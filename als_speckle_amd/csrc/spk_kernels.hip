@@ -21,6 +21,7 @@
 
 #include <algorithm>
 #include <stdint.h>
+#include <type_traits>
 
 #include "spk_internal.hpp"
 
@@ -344,7 +345,7 @@ __device__ __forceinline__ float sw_blur_lines_win(const float* line, const floa
     const float w0 = wl[0];
 #pragma unroll
     for (int k = 0; k < K; ++k) acc[k] = w0 * ln[blur_slot((j0 + k) & (N - 1))];
-#pragma unroll
+#pragma unroll 1   // unrolled, the 1024^2 resident kernel spills (0.4 us more per step)
     for (int a = 1; a <= kSwFuseRmax; a += C) {
       // x[j0 + k - d] = lo[k - d + a + C - 1], x[j0 + k + d] = hi[k + d - a]
       float lo[K + C - 1], hi[K + C - 1];
@@ -1304,7 +1305,7 @@ struct LineFft {
 
   int cb, ct;     // coalesced mapping: line, t
   int pb, pt;     // private mapping: line, natural t (values pt + i T)
-  int l;          // lane in the sub-transform
+  int sub, l;     // sub-transform and lane in it
   c32* a0;        // coalesced thread's first slot of the first exchange
   c32* a;         // private chunks
   c32* b;
@@ -1332,7 +1333,7 @@ struct LineFft {
     const int tid = threadIdx.x;
     cb = tid % TT;
     ct = tid / TT;
-    const int sub = tid / TW;
+    sub = tid / TW;
     l = tid % TW;
     pb = SPLIT ? sub / 2 : sub;
     pt = SPLIT ? 2 * l + (sub & 1) : l;
@@ -1426,6 +1427,21 @@ struct LineFft {
       }
       butterflies<2, INV>(x, w3);
     }
+  }
+  // values pt + i T of line pb -> the same values at ct + i T of line cb
+  template <class HOOK>
+  __device__ __forceinline__ void spread(c32 (&x)[E], HOOK before_barrier) {
+    // slot of value v of a line: its chunks of region A one after the other
+    auto slot = [](int line, int v) {
+      return (SPLIT ? 2 * line + v / M : line) * CHA + v % M + (v % M) / 8;
+    };
+    c32* base = a - sub * CHA;
+#pragma unroll
+    for (int i = 0; i < E; ++i) base[slot(pb, pt + i * T)] = x[i];
+    before_barrier();
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < E; ++i) x[i] = base[slot(cb, ct + i * T)];
   }
   // values pt + i T of line pb -> transform at ct + i T of line cb
   template <bool INV, class HOOK>
@@ -1895,6 +1911,100 @@ __global__ void __launch_bounds__((N / E) * TT)
   }
 #pragma unroll
   for (int i = 0; i < E; ++i) gst(a.psi, row_pos<N, TT, E>(rband, pb, pt, i), pin[i]);
+}
+
+// ---------------------------------------------------------------------------
+// Richardson-Lucy updates of the coherence function (phasing.py:700-736) in one
+// cooperative launch, exchange mode 3: per update two convolutions,
+//   u' = u * ifft2(fft2(d / ifft2(fft2(u) P)) Ph),
+// as eight phases of one transform each (rows, columns, rows, ... in the order
+// of the stand-alone transforms), u, d, P and Ph of the column band in
+// registers.  Twelve launches per update (four 2-D transforms and their
+// elementwise steps) take 85 us at 1024^2 on MI355X, 39 us here (512^2 42 / 22,
+// 256^2 38 / 17, 64^2 41 / 13), with
+// the same roundings: bitwise the same u.
+// ---------------------------------------------------------------------------
+__device__ __forceinline__ c32 rl_quotient(float d, c32 w, float sc) {
+  const c32 v = scale(w, sc);
+  const float den = fmaf(v.x, v.x, v.y * v.y);
+  return c32{d * v.x / den, -d * v.y / den};
+}
+
+template <int N, int TT, int E>
+__global__ void __launch_bounds__((N / E) * TT, 2)
+    k_resident_rl(const c32* __restrict__ tw, c32* u, const float* __restrict__ d,
+                  const c32* __restrict__ P, const c32* __restrict__ Ph, int iterations,
+                  float inv_nn, unsigned polls, int* flag, c32* ll) {
+  constexpr int NT = (N / E) * TT, NB = N / TT;
+  using LF = LineFft<N, TT>;
+  constexpr int LDSN = LF::LDS + N, HALF = (kLdsBytes / 2) / 8 + 64;
+  __shared__ c32 lds[LDSN > HALF ? LDSN : HALF];   // one workgroup per CU
+  static_assert(sizeof(lds) <= kLdsBytes, "resident kernel does not fit in LDS");
+  const int cband = xcd_band<NB>(blockIdx.x), rband = blockIdx.x;
+  LF tf;
+  {
+    TwStage<N, TT, NT> tws;
+    tws.fetch(tw);
+    tws.put(lds + LF::LDS);
+    __syncthreads();
+    tf.init(lds, lds + LF::LDS);
+  }
+  const int cb = tf.cb, ct = tf.ct, pb = tf.pb, pt = tf.pt;
+  c32 uu[E], p[E], ph[E];
+  float dd[E];
+#pragma unroll
+  for (int i = 0; i < E; ++i) {
+    const unsigned o = col_pos<N, TT, E>(cband, pb, pt, i);
+    uu[i] = gld(u, o);
+    p[i] = gld(P, o);
+    ph[i] = gld(Ph, o);
+    dd[i] = gld(d, o);
+  }
+  c32* to_col = ll;
+  c32* to_row = ll + (size_t)N * N;
+  LlWait llw{flag, polls, false};
+  constexpr int DELAY = ll_delay<N>();
+  auto cpos = [&](int i) { return (unsigned)col_pos<N, TT, E>(cband, cb, ct, i); };
+  auto rpos = [&](int i) { return (unsigned)row_pos<N, TT, E>(rband, cb, ct, i); };
+  auto emptied = [&]() { ll_emptied(); };
+  c32 x[E];
+  // the columns' values to the rows, the rows' transforms back to the columns,
+  // and their column transform in the private mapping
+  auto transform = [&](auto inv) {
+    constexpr bool INV = decltype(inv)::value;
+    tf.spread(x, emptied);
+    ll_give(x, to_row, cpos);
+    __syncthreads();
+    ll_take<DELAY>(x, to_row, llw, rpos);
+    tf.template to_private<INV>(x);
+    ll_empty<E>(to_row, rpos);
+    tf.spread(x, emptied);
+    ll_give(x, to_col, rpos);
+    __syncthreads();
+    ll_take<DELAY>(x, to_col, llw, cpos);
+    tf.template to_private<INV>(x);
+    ll_empty<E>(to_col, cpos);
+  };
+#pragma unroll 1
+  for (int it = 0; it < iterations; ++it) {
+#pragma unroll
+    for (int i = 0; i < E; ++i) x[i] = uu[i];
+    __syncthreads();
+    transform(std::false_type{});
+#pragma unroll
+    for (int i = 0; i < E; ++i) x[i] = mul(x[i], p[i]);
+    transform(std::true_type{});
+#pragma unroll
+    for (int i = 0; i < E; ++i) x[i] = rl_quotient(dd[i], x[i], inv_nn);
+    transform(std::false_type{});
+#pragma unroll
+    for (int i = 0; i < E; ++i) x[i] = mul(x[i], ph[i]);
+    transform(std::true_type{});
+#pragma unroll
+    for (int i = 0; i < E; ++i) uu[i] = mul(uu[i], scale(x[i], inv_nn));
+  }
+#pragma unroll
+  for (int i = 0; i < E; ++i) gst(u, col_pos<N, TT, E>(cband, pb, pt, i), uu[i]);
 }
 
 // before a resident launch: its barrier flags and give-up flag start at 0; the
@@ -2704,9 +2814,7 @@ static __global__ void __launch_bounds__(256) k_rl_divide(const float* d, const 
                                                           long long nn, float sc) {
   for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < nn;
        i += (long long)gridDim.x * 256) {
-    const c32 v = scale(w[i], sc);
-    const float den = fmaf(v.x, v.x, v.y * v.y);
-    out[i] = c32{d[i] * v.x / den, -d[i] * v.y / den};
+    out[i] = rl_quotient(d[i], w[i], sc);
   }
 }
 
@@ -2732,12 +2840,22 @@ static __global__ void __launch_bounds__(256) k_abs2_sum(c32* x, long long nn, d
   if (threadIdx.x == 0) partial[blockIdx.x] = s;
 }
 
-// x /= sum of the nblk partials (each thread adds them in order: deterministic)
+// x /= sum of the nblk (<= 256) partials, added in order by one thread of each
+// block from LDS (9 us at 1024^2; by every thread from global memory 42 us)
 static __global__ void __launch_bounds__(256) k_div_by_partials(c32* x, float* xr, long long nn,
                                                                 const double* partial, int nblk) {
-  double s = 0.0;
-  for (int b = 0; b < nblk; ++b) s += partial[b];
-  const float inv = (float)(1.0 / s);
+  __shared__ double part[256];
+  __shared__ float scale_by;
+  if ((int)threadIdx.x < nblk) part[threadIdx.x] = partial[threadIdx.x];
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    double s = 0.0;
+#pragma unroll 16
+    for (int b = 0; b < nblk; ++b) s += part[b];
+    scale_by = (float)(1.0 / s);
+  }
+  __syncthreads();
+  const float inv = scale_by;
   for (long long i = (long long)blockIdx.x * 256 + threadIdx.x; i < nn;
        i += (long long)gridDim.x * 256) {
     if (x) x[i] = scale(x[i], inv);
@@ -3201,6 +3319,22 @@ static hipError_t resident_nt(int xm, const PassArgs& a, const RStep* steps, int
   return e;
 }
 
+template <int N>
+static hipError_t resident_rl_dispatch(int tile, int ept, const c32* tw, c32* u, const float* d,
+                                       const c32* P, const c32* Ph, int iterations, float inv_nn,
+                                       unsigned polls, int* flag, c32* ll, hipStream_t st) {
+  if constexpr (N >= 64 && N <= 1024) {
+    if (tile != 4 || ept != 8) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(k_resident_begin, dim3(1024), dim3(256), 0, st, nullptr, 0, flag,
+                       reinterpret_cast<u32x2*>(ll), 2 * N * N, 1);
+    void* args[] = {(void*)&tw,     (void*)&u,     (void*)&d,    (void*)&P,  (void*)&Ph,
+                    (void*)&iterations, (void*)&inv_nn, (void*)&polls, (void*)&flag, (void*)&ll};
+    return hipLaunchCooperativeKernel(reinterpret_cast<const void*>(&k_resident_rl<N, 4, 8>),
+                                      dim3(N / 4), dim3((N / 8) * 4), args, 0, st);
+  }
+  return hipErrorInvalidValue;
+}
+
 // frames that one launch of several holds at once on the current device
 template <int N, int TT, int E>
 static hipError_t resident_frames_nt(int* out) {
@@ -3346,6 +3480,9 @@ constexpr bool shape_ok() {
                           int* flag, c32* ll, int fill, int frames, int at_once,                 \
                           hipStream_t st);                                                  \
   hipError_t resident_frames_##n(int tile, int ept, int* out);                              \
+  hipError_t resident_rl_##n(int tile, int ept, const c32* tw, c32* u, const float* d,      \
+                             const c32* P, const c32* Ph, int iterations, float inv_nn,     \
+                             unsigned polls, int* flag, c32* ll, hipStream_t st);           \
   hipError_t resident_ipsf_##n(int tile, int ept, const PassArgs& a, const c32* ipsf,       \
                                const RStep* steps, int nsteps, double* errp0,               \
                                long long errp_step, int* flag, c32* ll, int fill,           \
@@ -3460,6 +3597,12 @@ constexpr bool shape_ok() {
   hipError_t resident_frames_##n(int tile, int ept, int* out) {                             \
     return resident_frames_dispatch<n>(tile, ept, out);                                     \
   }                                                                                         \
+  hipError_t resident_rl_##n(int tile, int ept, const c32* tw, c32* u, const float* d,      \
+                             const c32* P, const c32* Ph, int iterations, float inv_nn,     \
+                             unsigned polls, int* flag, c32* ll, hipStream_t st) {          \
+    return resident_rl_dispatch<n>(tile, ept, tw, u, d, P, Ph, iterations, inv_nn, polls,   \
+                                   flag, ll, st);                                           \
+  }                                                                                         \
   hipError_t resident_ipsf_##n(int tile, int ept, const PassArgs& a, const c32* ipsf,       \
                                const RStep* steps, int nsteps, double* errp0,               \
                                long long errp_step, int* flag, c32* ll, int fill,           \
@@ -3546,6 +3689,12 @@ hipError_t launch_resident(int n, int tile, int ept, int xm, const PassArgs& a,
                            hipStream_t st) {
   SPK_SIZE_SWITCH(resident, tile, ept, xm, a, steps, nsteps, errp0, errp_step, bar, flag, ll, fill,
                   frames, at_once, st)
+}
+
+hipError_t launch_resident_rl(int n, int tile, int ept, const c32* tw, c32* u, const float* d,
+                              const c32* P, const c32* Ph, int iterations, float inv_nn,
+                              unsigned polls, int* flag, c32* ll, hipStream_t st) {
+  SPK_SIZE_SWITCH(resident_rl, tile, ept, tw, u, d, P, Ph, iterations, inv_nn, polls, flag, ll, st)
 }
 
 hipError_t resident_frames(int n, int tile, int ept, int* out) {

@@ -524,6 +524,7 @@ class phasing:
             frame = to_device(est[-1].astype(np.complex64), self.ctx.device, torch.complex64)
             ipsf = plan.coherence_rl(frame, m_dev, int(iterations), semantics, is_fourier)
             out = ipsf.cpu().numpy()
+            plan.check()    # raises if the updates' launch gave up waiting
             if load:
                 self.load(ipsf=out)
             return np.fft.fftshift(out)
