@@ -287,9 +287,9 @@ SPK_HD int col_pos(int band, int b, int t, int i) {
 //  - single layout (n <= 2048): Phi stays tiled; the row pass reads and
 //    writes whole contiguous row bands, the column pass reads and writes
 //    TT x TT tiles in place;
-//  - dual layout (n = 4096): the row pass writes Phi column-band-major and
-//    the column pass writes it back tiled, so every pass *reads* contiguous
-//    memory (at 4096 the tile stride of the single layout is 128 KB).
+//  - dual layout (n = 4096): the row pass writes Phi column-band-major
+//    (dual_row_pos) and the column pass writes it back tiled, so every pass
+//    *reads* contiguous memory (at 4096 the tile stride of the single layout is 128 KB).
 // Measured on MI355X: strided writes cost more than strided reads up to
 // 2048, so the dual layout only pays at 4096.
 #ifndef SPK_DUAL_MIN
@@ -317,6 +317,23 @@ SPK_HD int cbrow_pos(int band, int b, int t, int i) {
   constexpr int T = N / E;
   const int col = t + i * T;
   return (col / TT) * N * TT + (band * TT + b) * TT + (col % TT);
+}
+
+// Phi's column-band-major copy in the dual layout: bands of at least four
+// columns, so that the row pass of two rows writes 64-byte pieces (4096^2: row
+// pass 158 -> 127 us with 64-byte instead of 32-byte pieces; the column pass of
+// two columns reads half of each piece and its neighbour, on the same XCD, the
+// other half from the L2).  Row pass: row b of row-band `band`, column t + i T.
+template <int N, int TT, int E = ept<N, TT>()>
+SPK_HD int dual_row_pos(int band, int b, int t, int i) {
+  constexpr int T = N / E, W = TT > 4 ? TT : 4;
+  return mcb_pos<W>(N, band * TT + b, t + i * T);
+}
+// column pass: column b of column-band `band`, row t + i T
+template <int N, int TT, int E = ept<N, TT>()>
+SPK_HD int dual_col_pos(int band, int b, int t, int i) {
+  constexpr int T = N / E, W = TT > 4 ? TT : 4;
+  return mcb_pos<W>(N, t + i * T, band * TT + b);
 }
 
 // LDS slot of element p of transform b (TT transforms per workgroup,

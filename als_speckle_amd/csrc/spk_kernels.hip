@@ -448,7 +448,7 @@ __device__ __forceinline__ void colpass_item(const PassArgs& a, int f, int band,
   c32 x[E];
 #pragma unroll
   for (int i = 0; i < E; ++i) {
-    if constexpr (DUAL) x[i] = gld_nt(src, mcol_pos<N, TT, E>(band, b, t, i));
+    if constexpr (DUAL) x[i] = gld(src, dual_col_pos<N, TT, E>(band, b, t, i));
     else x[i] = gld(src, col_pos<N, TT, E>(band, b, t, i));
   }
   // the modulus is loaded with the data where registers allow, otherwise
@@ -563,7 +563,8 @@ __device__ __forceinline__ void colpass_ipsf_a(const PassArgs& a, int f, int ban
   c32 x[E];
 #pragma unroll
   for (int i = 0; i < E; ++i)
-    x[i] = gld(src, DUAL ? mcol_pos<N, TT, E>(band, b, t, i) : col_pos<N, TT, E>(band, b, t, i));
+    x[i] = gld(src, DUAL ? dual_col_pos<N, TT, E>(band, b, t, i)
+                         : col_pos<N, TT, E>(band, b, t, i));
   c32* twl = lds + L::NBUF * L::BUF;
   tws.put(twl);
   const auto tw = twiddle_view<N, TT, kColDbWgs>(twl);
@@ -595,7 +596,8 @@ __device__ __forceinline__ void colpass_intensity(const PassArgs& a, int f, int 
   c32 x[E];
 #pragma unroll
   for (int i = 0; i < E; ++i)
-    x[i] = gld(src, DUAL ? mcol_pos<N, TT, E>(band, b, t, i) : col_pos<N, TT, E>(band, b, t, i));
+    x[i] = gld(src, DUAL ? dual_col_pos<N, TT, E>(band, b, t, i)
+                         : col_pos<N, TT, E>(band, b, t, i));
   c32* twl = lds + L::NBUF * L::BUF;
   tws.put(twl);
   fft_regs<N, E, TT, MODE == 7, true, kColDbWgs>(x, t, b, lds, twiddle_view<N, TT, kColDbWgs>(twl));
@@ -634,7 +636,8 @@ __device__ __forceinline__ void colpass_div_b(const PassArgs& a, int f, int band
     const c32* dsrc = (z ? (DUAL ? a.dbufc2 : a.dbuf2) : (DUAL ? a.dbufc : a.dbuf)) + fo;
 #pragma unroll
     for (int i = 0; i < E; ++i)
-      d[i] = gld(dsrc, DUAL ? mcol_pos<N, TT, E>(band, b, t, i) : col_pos<N, TT, E>(band, b, t, i));
+      d[i] = gld(dsrc, DUAL ? dual_col_pos<N, TT, E>(band, b, t, i)
+                            : col_pos<N, TT, E>(band, b, t, i));
   } else {
 #pragma unroll
     for (int i = 0; i < E; ++i) div[i] = gld((z ? a.dmap2 : a.dmap) + fo, mcol_pos<N, TT, E>(band, b, t, i));
@@ -642,7 +645,8 @@ __device__ __forceinline__ void colpass_div_b(const PassArgs& a, int f, int band
   c32 x[E];
 #pragma unroll
   for (int i = 0; i < E; ++i)
-    x[i] = gld(src, DUAL ? mcol_pos<N, TT, E>(band, b, t, i) : col_pos<N, TT, E>(band, b, t, i));
+    x[i] = gld(src, DUAL ? dual_col_pos<N, TT, E>(band, b, t, i)
+                         : col_pos<N, TT, E>(band, b, t, i));
   const float* __restrict__ mod = a.mod + (size_t)f * a.mstride;
   float m[E];
 #pragma unroll
@@ -863,14 +867,14 @@ __device__ __forceinline__ void rowpass_item(const PassArgs& a, int f, int band,
     fft_regs<N, E, TT, false, false>(y, t, b, lds, tw);
 #pragma unroll
     for (int i = 0; i < E; ++i) {
-      if constexpr (DUAL) gst(a.phibc + fo, cbrow_pos<N, TT, E>(band, b, t, i), y[i]);
+      if constexpr (DUAL) gst(a.phibc + fo, dual_row_pos<N, TT, E>(band, b, t, i), y[i]);
       else gst(a.phib + fo, SPK_RPOS(i), y[i]);
     }
   }
   fft_regs<N, E, TT, false, false>(x, t, b, lds, tw);
 #pragma unroll
   for (int i = 0; i < E; ++i) {
-    if constexpr (DUAL) gst(a.phic + fo, cbrow_pos<N, TT, E>(band, b, t, i), x[i]);
+    if constexpr (DUAL) gst(a.phic + fo, dual_row_pos<N, TT, E>(band, b, t, i), x[i]);
     else if (a.nt_store) gst_nt(phi, SPK_RPOS(i), x[i]);
     else gst(phi, SPK_RPOS(i), x[i]);
   }
@@ -948,7 +952,7 @@ __global__ void __launch_bounds__((N / E) * TT)
   fft_regs<N, E, TT, true, false>(x, t, b, lds, tv);
 #pragma unroll
   for (int i = 0; i < E; ++i) {
-    if constexpr (dual_layout<N>()) gst(out + fo, cbrow_pos<N, TT, E>(band, b, t, i), x[i]);
+    if constexpr (dual_layout<N>()) gst(out + fo, dual_row_pos<N, TT, E>(band, b, t, i), x[i]);
     else gst(out + fo, row_pos<N, TT, E>(band, b, t, i), x[i]);
   }
 }
@@ -2061,7 +2065,7 @@ __global__ void __launch_bounds__((N / E) * TT)
   c32* dst = out + fo;
 #pragma unroll
   for (int i = 0; i < E; ++i) {
-    if constexpr (dual_layout<N>()) gst(dst, cbrow_pos<N, TT, E>(band, b, t, i), x[i]);
+    if constexpr (dual_layout<N>()) gst(dst, dual_row_pos<N, TT, E>(band, b, t, i), x[i]);
     else gst(dst, row_pos<N, TT, E>(band, b, t, i), x[i]);
   }
 }
@@ -2107,7 +2111,7 @@ __global__ void __launch_bounds__((N / E) * TT)
   c32* dst = out + (size_t)f * N * N;
 #pragma unroll
   for (int i = 0; i < E; ++i) {
-    if constexpr (dual_layout<N>()) gst(dst, cbrow_pos<N, TT, E>(band, b, t, i), x[i]);
+    if constexpr (dual_layout<N>()) gst(dst, dual_row_pos<N, TT, E>(band, b, t, i), x[i]);
     else gst(dst, row_pos<N, TT, E>(band, b, t, i), x[i]);
   }
 }
@@ -2174,7 +2178,7 @@ __global__ void __launch_bounds__((N / E) * TT)
 #pragma unroll
     for (int i = 0; i < E; ++i) {
       if (t + i * T < used)
-        v[i] = gld(src, dual_layout<N>() ? mcol_pos<N, TT, E>(band, b, t, i)
+        v[i] = gld(src, dual_layout<N>() ? dual_col_pos<N, TT, E>(band, b, t, i)
                                          : col_pos<N, TT, E>(band, b, t, i));
       else
         v[i] = c32{0.0f, 0.0f};
