@@ -707,6 +707,91 @@ __global__ void __launch_bounds__((N / E) * TT) k_colpass(PassArgs a) {
 }
 
 // ---------------------------------------------------------------------------
+// Column pass in tile 2, four columns per workgroup (MODE 0; z = 1: phib, no
+// error): the columns of two bands, two at a time through the transforms, so
+// that a thread loads and stores 16 bytes (columns 2b and 2b + 1 of a row) and
+// the tiles of a row pair are 64 contiguous bytes instead of 32.  Bound by
+// those scattered pieces: with 32 bytes the 4096^2 pass took 113 us, 57 of them
+// without its stores and loads, 89 with contiguous stores; 64 bytes 90 us.
+// 2048^2: one frame 23.3 -> 22.8 us, four 78 -> 69, ten 203 -> 185.  1024^2 in
+// tile 2: no gain (16 frames 61.9 / 64.5).  Values, error sums and their order
+// are colpass_item's.  grid (n/4, frames, z)
+// ---------------------------------------------------------------------------
+template <int N, int E>
+__global__ void __launch_bounds__((N / E) * 2) k_colpass_pair(PassArgs a) {
+  constexpr int TT = 2, T = N / E, NT = T * TT, NB = N / TT, NW = NT / 64;
+  static_assert(NT % 64 == 0, "whole wavefronts");
+  using L = LdsPlan<N, TT, kColDbWgs>;
+  using V4 = float __attribute__((ext_vector_type(4)));
+  using V2 = float __attribute__((ext_vector_type(2)));
+  __shared__ c32 lds[L::TOTAL];
+  const int q = xcd_band<NB / 2>(blockIdx.x);
+  const int f = a.fmap ? a.fmap[blockIdx.y] : blockIdx.y, z = blockIdx.z;
+  const Coef c = a.tab ? a.tab[f] : a.c;
+  if (!(c.flags & kActive)) return;
+  if (z && !(c.flags & kUseT)) return;
+  const size_t fo = (size_t)f * N * N;
+  const int tid = threadIdx.x, b = tid % TT, t = tid / TT;
+  TwStage<N, TT, NT, kColDbWgs> tws;
+  tws.fetch(a.tw);
+  constexpr bool DUAL = dual_layout<N>();
+  // columns 2b and 2b + 1 of row r: in a row of the tile of band 2q + b, or of
+  // the four-column band of the dual layout's column-band-major copy
+  auto tile = [&](int r) { return ((r / 2) * NB + 2 * q + b) * 2 + r % 2; };
+  const V4* src = reinterpret_cast<const V4*>(
+      (z ? (DUAL ? a.phibc : a.phib) : (DUAL ? a.phic : a.phi)) + fo);
+  const V2* mod = reinterpret_cast<const V2*>(a.mod + (size_t)f * a.mstride);
+  c32 x0[E], x1[E];
+  V2 m[E];
+#pragma unroll
+  for (int i = 0; i < E; ++i) {
+    const V4 v = gld(src, DUAL ? (q * N + t + i * T) * 2 + b : tile(t + i * T));
+    x0[i] = c32{v.x, v.y};
+    x1[i] = c32{v.z, v.w};
+  }
+#pragma unroll
+  for (int i = 0; i < E; ++i)
+    m[i] = DUAL ? __builtin_nontemporal_load(mod + (2 * q + b) * N + t + i * T)
+                : gld(mod, (2 * q + b) * N + t + i * T);
+  c32* twl = lds + L::NBUF * L::BUF;
+  tws.put(twl);
+  const auto tw = twiddle_view<N, TT, kColDbWgs>(twl);
+  double e0 = 0.0, e1 = 0.0;
+  fft_regs<N, E, TT, false, true, kColDbWgs>(x0, t, b, lds, tw);
+#pragma unroll
+  for (int i = 0; i < E; ++i) x0[i] = project_modulus(x0[i], m[i].x, e0);
+  fft_regs<N, E, TT, true, false, kColDbWgs>(x0, t, b, lds, tw);
+  fft_regs<N, E, TT, false, false, kColDbWgs>(x1, t, b, lds, tw);
+#pragma unroll
+  for (int i = 0; i < E; ++i) x1[i] = project_modulus(x1[i], m[i].y, e1);
+  fft_regs<N, E, TT, true, false, kColDbWgs>(x1, t, b, lds, tw);
+  V4* dst = reinterpret_cast<V4*>((z ? a.phib : a.phi) + fo);
+#pragma unroll
+  for (int i = 0; i < E; ++i) {
+    gst(dst, tile(t + i * T), V4{x0[i].x, x0[i].y, x1[i].x, x1[i].y});
+  }
+  if (z == 0 && a.errp) {
+    // band 2q + b holds the columns of the threads with this b: block_sum's
+    // wavefront sums over t for either column, then the two columns, then the
+    // wavefronts in order
+    double* sh = reinterpret_cast<double*>(lds);
+#pragma unroll
+    for (int o = 32; o > 1; o >>= 1) {
+      e0 += __shfl_xor(e0, o, 64);
+      e1 += __shfl_xor(e1, o, 64);
+    }
+    __syncthreads();
+    if ((tid & 63) < 2) sh[(tid & 1) * NW + (tid >> 6)] = e0 + e1;
+    __syncthreads();
+    if (tid < 2) {
+      double s = 0.0;
+      for (int w = 0; w < NW; ++w) s += sh[tid * NW + w];
+      a.errp[(size_t)f * NB + 2 * q + tid] = s;
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // Row pass: row IFFT of phi (and phib for DM) -> update -> psi; row FFT of the
 // new psi -> phi (and of dm1(psi) -> phib when the next step is DM).
 // One item = one band of TT rows of frame f with coefficients c.
@@ -3184,6 +3269,12 @@ template <int N, int TT, int E>
 static hipError_t colpass_nt(int mode, const PassArgs& a, int frames, int zdim,
                              hipStream_t st) {
   dim3 grid(N / TT, frames, zdim), block((N / E) * TT);
+  if constexpr (N >= 2048 && TT == 2 && E == 16) {
+    if (mode == 0) {
+      launch_pass(k_colpass_pair<N, E>, dim3(N / 4, frames, zdim), block, st, a);
+      return hipGetLastError();
+    }
+  }
   switch (mode) {
     case 0: launch_pass(k_colpass<N, TT, E, 0>, grid, block, st, a); break;
     case 2: launch_pass(k_colpass<N, TT, E, 2>, grid, block, st, a); break;
