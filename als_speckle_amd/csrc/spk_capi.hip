@@ -61,22 +61,31 @@ int default_ept(int n, int tile, int batch) {
   return (n / 8) * tile <= 1024 ? 8 : 16;
 }
 
-// Resident launches of several frames (uniform schedules): a launch holds
-// 2^20 / n^2 frames at once (2^19 at 64^2) and takes more in rounds.  They
-// pay up to three rounds; microseconds per step of all frames on MI355X, one
-// launch per pass / resident:
-//   64^2 x 128 14.7 / 6.0;  128^2 x 64 19.2 / 9.8, x 96 23.5 / 15.2;
-//   256^2 x 4 11.0 / 5.7, x 16 20.1 / 9.9, x 32 25.2 / 19.0, x 48 33.4 / 28.4,
-//   x 64 39.7 / 37.6;  512^2 x 2 14.9 / 6.9, x 4 21.0 / 10.8, x 8 26.8 / 21.3,
-//   x 12 34.3 / 31.8, x 16 40.5 / 42.2;  1024^2 x 2 29.6 / 20.6, x 3 36.6 / 30.8.
-constexpr int kResidentRounds = 3;
+// Resident launches of several frames (uniform schedules): in exchange mode 3
+// a launch holds 2^20 / n^2 frames at once (2^19 at 64^2); where those are not
+// all and n <= kResidentLeanMax, the lean form holds twice as many (k_resident)
+// and takes the rest in rounds.  They pay up to four rounds, three from 512 up;
+// microseconds per step of all frames on MI355X, one launch per pass / resident:
+//   64^2 x 128 14.4 / 6.4, x 512 29.5 / 19.1;  128^2 x 64 19.3 / 9.8, x 128
+//   26.1 / 15.0, x 192 31.8 / 23.0;  256^2 x 4 11.1 / 6.2, x 16 20.1 / 10.3,
+//   x 32 25.0 / 15.5, x 64 39.3 / 29.6, x 96 53.6 / 43.5, x 128 67.7 / 57.3;
+//   512^2 x 2 15.0 / 7.4, x 4 21.0 / 10.1, x 8 26.8 / 16.5, x 9 28.0 / 22.4, x 16
+//   40.6 / 32.3, x 24 54.4 / 47.7, x 28 61.6 / 60.0 (four rounds of 7), x 40
+//   82.7 / 78.6, x 64 125 / 128;  1024^2 x 2 30.1 / 21.5, x 3 36.6 / 32.1.
+int resident_rounds(int n) { return n <= 256 ? 4 : 3; }
+// frames at once by the sizes alone (a 256-CU device): mode 3, lean
+int resident_fit(int n) { return std::max(1, (1 << 20) / (n * n)); }
 // Steps from which a block runs resident by default: a cooperative launch
 // takes about 20 us more than a plain one and the frames' state goes in and
-// out once per round (4 / 8 steps of one 256^2 frame 49 / 89 us per pass, 60 /
-// 81 resident; of one 1024^2 frame 2 / 4 steps 57 / 100 and 70 / 92; 16 steps
-// of 40 x 256^2 479 and 461).
+// out once per round.  Microseconds of a block, per pass / resident: 4 / 8
+// steps of one 256^2 frame 49 / 89 and 60 / 81; 2 / 4 steps of one 1024^2 frame
+// 57 / 100 and 70 / 92; 6 steps of 32 x 256^2 185 / 153; two rounds, 8 / 12 steps
+// of 33 x 256^2 251 / 358 and 218 / 291, of 9 x 512^2 257 / 377 and 246 / 333;
+// three, 12 / 16 steps of 17 x 512^2 539 / 717 and 536 / 692; four, 16 steps of
+// 97 x 256^2 899 / 825.
 int resident_min_steps(int n, int rounds) {
-  return rounds > 1 ? 16 * (rounds - 1) : n >= 1024 ? 3 : 6;
+  if (n >= 1024) return rounds > 1 ? 16 * (rounds - 1) : 3;
+  return 6 * rounds;
 }
 
 template <class T>
@@ -175,6 +184,7 @@ struct spk_plan {
   int resident_min = 2;        // steps of a block that runs resident
   bool res_allowed = true;     // spk_tune.resident != 2
   int xm = 0;
+  int res_xm = 0;              // that of this plan's launches (several frames: 3 or 2)
   // resident launches: the two exchange buffers of mode 3 (n*n values each),
   // then the barrier flags (a 128-byte line per band)
   c32* rll = nullptr;
@@ -593,9 +603,13 @@ int spk_plan_bytes(int n, int batch, int shared, int options, size_t* bytes) {
   b += 64 * 1024;                                      // step-table staging
   // resident launches' exchange, for the frames that a launch holds at once
   const int tile = default_tile(n);
-  const size_t fit = std::max<size_t>(1, ((size_t)1 << 20) / nn);
-  if (resident_supported(n, tile, default_ept(n, tile, batch)) && batch <= kResidentRounds * fit)
-    b += std::min<size_t>(batch, fit) * (2 * nn * sizeof(c32) + bands * 128);
+  const size_t fit = resident_fit(n);
+  if (resident_supported(n, tile, default_ept(n, tile, batch))) {
+    if ((size_t)batch <= fit || (n > kResidentLeanMax && batch <= resident_rounds(n) * fit))
+      b += std::min<size_t>(batch, fit) * (2 * nn * sizeof(c32) + bands * 128);
+    else if (n <= kResidentLeanMax && batch <= resident_rounds(n) * 2 * fit)
+      b += std::min<size_t>(batch, 2 * fit) * bands * 128;
+  }
   *bytes = b;
   return SPK_OK;
 }
@@ -628,7 +642,7 @@ int spk_plan_create(spk_ctx* ctx, int n, int batch, int shared, const spk_tune* 
   p->phib_g.assign(batch, 0.0f);
   // resident launches by default where they are built and pay: one frame of
   // 64^2 to 1024^2 takes about half the time of one launch per pass on
-  // MI355X, several see kResidentRounds; the exchange of Phi by polled values
+  // MI355X, several see resident_rounds; the exchange of Phi by polled values
   // is the default (the barrier forms are slower, the fenced ones most)
   p->xm = (tune && tune->exchange >= 1 && tune->exchange <= 4) ? tune->exchange - 1 : 3;
   const int res_mode = tune ? tune->resident : 0;
@@ -636,12 +650,20 @@ int spk_plan_create(spk_ctx* ctx, int n, int batch, int shared, const spk_tune* 
   if (res_mode != 2 && resident_supported(n, tile, ept)) {
     int fit = 1;
     // (the occupancy query only where the answer can matter)
-    const bool few = batch <= kResidentRounds * std::max(1, (1 << 20) / (n * n));
-    if (batch > 1 && (p->xm != 3 || !(few || res_mode == 1) ||
-                      resident_frames(n, tile, ept, &fit) != hipSuccess))
-      fit = 0;
+    const bool few = batch <= resident_rounds(n) * 2 * resident_fit(n);
+    p->res_xm = p->xm;
+    if (batch > 1) {
+      if (p->xm != 3 || !(few || res_mode == 1) ||
+          resident_frames(n, tile, ept, 3, &fit) != hipSuccess)
+        fit = 0;
+      // more than one round of mode 3: the lean form's
+      if (fit && batch > fit && n <= kResidentLeanMax) {
+        p->res_xm = 2;
+        if (resident_frames(n, tile, ept, 2, &fit) != hipSuccess) fit = 0;
+      }
+    }
     const int rounds = fit ? (batch + fit - 1) / fit : 0;
-    if (rounds && (rounds <= kResidentRounds || res_mode == 1)) {
+    if (rounds && (rounds <= resident_rounds(n) || res_mode == 1)) {
       p->resident = (batch + rounds - 1) / rounds;   // as even as they go
       // a caller that asks for the form or its exchange gets it for any block
       const bool asked = res_mode == 1 || (tune && tune->exchange > 0);
@@ -1363,7 +1385,7 @@ int iter_step(IterRun& r, int k, int* next) {
     // one allocation: the exchange buffers of mode 3, then the barrier flags,
     // for the frames that a launch runs at once
     const int g = p->resident;
-    const size_t ll = p->xm == 3 ? (size_t)g * 2 * p->nn() : 0;
+    const size_t ll = p->res_xm == 3 ? (size_t)g * 2 * p->nn() : 0;
     if (!p->rll && (rc = dalloc(&p->rll, ll + (size_t)g * p->bands * 16))) return rc;
     unsigned* rsync = reinterpret_cast<unsigned*>(p->rll + ll);
     PassArgs ra = base_args(p);
@@ -1378,7 +1400,7 @@ int iter_step(IterRun& r, int k, int* next) {
                                    (long long)B * p->bands, (int*)(p->pbar + 1), p->rll, fill,
                                    st));
     else
-      SPK_HIP(launch_resident(p->n, p->tile, p->ept, p->xm, ra, tab, r.res_n[k], errp,
+      SPK_HIP(launch_resident(p->n, p->tile, p->ept, p->res_xm, ra, tab, r.res_n[k], errp,
                               (long long)B * p->bands, rsync, (int*)(p->pbar + 1), p->rll, fill,
                               B, g, st));
     p->res_launches++;

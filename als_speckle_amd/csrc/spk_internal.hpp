@@ -194,7 +194,8 @@ hipError_t launch_roll_sum(const c32* data, int frames, int rows, int cols, cons
 // 1 device-scope + fences, 2 device-scope, no fences, 3 values polled
 // themselves in the two n*n buffers of ll; fill: empty them first, a new
 // pair); `frames` frames of the plan, `at_once` of them at a time (one frame:
-// any exchange mode; several: mode 3, flags and ll for each of at_once);
+// any exchange mode; several: mode 3, or 2 up to kResidentLeanMax; flags and,
+// in mode 3, ll for each of at_once);
 // errp0[kidx *
 // errp_step + band] gets the error partials of the steps with err set;
 // flags: n/tile * 32 words of barrier flags (zeroed by the launcher); flag:
@@ -204,8 +205,10 @@ hipError_t launch_resident(int n, int tile, int ept, int xm, const PassArgs& a,
                            const RStep* steps, int nsteps, double* errp0, long long errp_step,
                            unsigned* flags, int* flag, c32* ll, int fill, int frames, int at_once,
                            hipStream_t st);
-// frames that one launch holds at once on the current device (exchange mode 3)
-hipError_t resident_frames(int n, int tile, int ept, int* out);
+// frames that one launch of several holds at once on the current device, in
+// exchange mode 3 or (n <= kResidentLeanMax) 2
+constexpr int kResidentLeanMax = 512;
+hipError_t resident_frames(int n, int tile, int ept, int xm, int* out);
 // the same with a partially coherent projection by the tiled ipsf, in tile 4
 // and exchange mode 3 (k_resident_ipsf); fused shrinkwraps are not part of it
 hipError_t launch_resident_ipsf(int n, int tile, int ept, const PassArgs& a, const c32* ipsf,

@@ -1175,19 +1175,26 @@ __device__ __forceinline__ u32x2 dev_ld(const c32* base, unsigned i) {
 __device__ __forceinline__ void dev_st(c32* base, unsigned i, u32x2 v) {
   __builtin_amdgcn_raw_buffer_store_b64(v, dev_rsrc(base), (int)(i * 8u), 0, kDevScope);
 }
+// element i + s with a uniform s: one vector offset serves all of a thread's values
+__device__ __forceinline__ u32x2 dev_ld(const c32* base, unsigned i, unsigned s) {
+  return __builtin_amdgcn_raw_buffer_load_b64(dev_rsrc(base), (int)(i * 8u), (int)(s * 8u), kDevScope);
+}
+__device__ __forceinline__ void dev_st(c32* base, unsigned i, unsigned s, u32x2 v) {
+  __builtin_amdgcn_raw_buffer_store_b64(v, dev_rsrc(base), (int)(i * 8u), (int)(s * 8u), kDevScope);
+}
 template <int XM>
-__device__ __forceinline__ c32 xld(const c32* base, unsigned i) {
+__device__ __forceinline__ c32 xld(const c32* base, unsigned i, unsigned s = 0) {
   if constexpr (XM == 0) {
-    return gld(base, i);
+    return gld(base, i + s);
   } else {
-    const u32x2 v = dev_ld(base, i);
+    const u32x2 v = dev_ld(base, i, s);
     return c32{__uint_as_float(v.x), __uint_as_float(v.y)};
   }
 }
 template <int XM>
-__device__ __forceinline__ void xst(c32* base, unsigned i, const c32& v) {
-  if constexpr (XM == 0) gst(base, i, v);
-  else dev_st(base, i, u32x2{__float_as_uint(v.x), __float_as_uint(v.y)});
+__device__ __forceinline__ void xst(c32* base, unsigned i, unsigned s, const c32& v) {
+  if constexpr (XM == 0) gst(base, i + s, v);
+  else dev_st(base, i, s, u32x2{__float_as_uint(v.x), __float_as_uint(v.y)});
 }
 
 // Float exchange of the resident kernel's shrinkwrap maps, device scope in
@@ -1365,7 +1372,9 @@ __device__ __forceinline__ void ll_emptied() { __builtin_amdgcn_s_waitcnt(0x0F70
 // into the coalesced one: 3 barriers at 1024 and 2 below instead of 6 and 4.
 // Butterflies, twiddles and their order are stage_butterflies', so values are
 // the pass kernels' bit for bit.  A thread's twiddles do not change during a
-// launch and stay in registers.
+// launch and stay in registers.  LEAN (128 registers per thread, four
+// wavefronts per SIMD) reads them from the table in LDS at each stage and
+// makes both private exchanges in one region.
 // ---------------------------------------------------------------------------
 // orders a wavefront's LDS writes before its reads (the hardware keeps a
 // wavefront's LDS accesses in order)
@@ -1375,7 +1384,7 @@ __device__ __forceinline__ void wave_lds_order() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-template <int N, int TT>
+template <int N, int TT, bool LEAN = false>
 struct LineFft {
   static constexpr int E = 8, T = N / E;
   static constexpr bool SPLIT = T > 64;              // even and odd samples apart
@@ -1387,7 +1396,7 @@ struct LineFft {
   static_assert(T <= 128 && S >= 2 && S <= 3, "64 <= N <= 1024");
   // LDS: a chunk of each region per sub-transform (c32 slots)
   static constexpr int CHA = M + M / 8 + 2;          // e -> e + e / 8
-  static constexpr int CHB = S == 3 ? M + M / 8 : 0; // e -> e + 8 (e / 64)
+  static constexpr int CHB = S == 3 && !LEAN ? M + M / 8 : 0;   // e -> e + 8 (e / 64)
   static constexpr int HALF = M / 2 + 16;            // even, then odd values
   static constexpr int CHC = SPLIT ? 2 * HALF : 0;
   static constexpr int LDS = SUBS * (CHA + CHB + CHC);
@@ -1401,10 +1410,12 @@ struct LineFft {
   c32* c;
   c32* cline;     // region C of this line
   const c32* fa;  // coalesced thread's read base of the last exchange
-  c32 w1[7];                      // stage 1
-  c32 w2[S == 3 ? 7 : 1];         // stage 2 (entries by butterfly, then value)
-  c32 w3[SPLIT ? 4 : 1], w3c[SPLIT ? 4 : 1], w2c[(!SPLIT && S == 3) ? 7 : 1];
-  c32 w1c[S == 2 ? 7 : 1];
+  const c32* table;               // the staged twiddle table
+  static constexpr int REG = LEAN ? 0 : 1;
+  c32 w1[REG ? 7 : 1];                      // stage 1
+  c32 w2[REG && S == 3 ? 7 : 1];            // stage 2 (entries by butterfly, then value)
+  c32 w3[REG && SPLIT ? 4 : 1], w3c[REG && SPLIT ? 4 : 1], w2c[REG && !SPLIT && S == 3 ? 7 : 1];
+  c32 w1c[REG && S == 2 ? 7 : 1];
 
   template <int ST>
   static __device__ __forceinline__ void load_tw(c32* w, const c32* twl, int t) {
@@ -1418,6 +1429,18 @@ struct LineFft {
         w[q * (R - 1) + r - 1] =
             twl[staged_tw_offset(N, E, ST) + ((t + q * STEP) & (NS - 1)) * (R - 1) + r - 1];
   }
+  // stage ST with its twiddles: those of registers w, or the table's for t
+  template <int ST, bool INV>
+  __device__ __forceinline__ void stage(c32 (&x)[E], const c32* w, int t) const {
+    constexpr int R = plan_radix(N, E, ST);
+    if constexpr (LEAN) {
+      c32 u[(E / R) * (R - 1)];
+      load_tw<ST>(u, table, t);
+      butterflies<R, INV>(x, u);
+    } else {
+      butterflies<R, INV>(x, w);
+    }
+  }
   __device__ __forceinline__ void init(c32* lds, const c32* twl) {
     const int tid = threadIdx.x;
     cb = tid % TT;
@@ -1427,14 +1450,16 @@ struct LineFft {
     pb = SPLIT ? sub / 2 : sub;
     pt = SPLIT ? 2 * l + (sub & 1) : l;
     a = lds + sub * CHA;
-    b = lds + SUBS * CHA + sub * CHB;
+    table = twl;
+    b = LEAN ? a : lds + SUBS * CHA + sub * CHB;
     c = lds + SUBS * (CHA + CHB) + sub * CHC;
     cline = lds + SUBS * (CHA + CHB) + 2 * pb * CHC;
     const int csub = SPLIT ? 2 * cb + (ct & 1) : cb, cl = SPLIT ? ct >> 1 : ct;
     a0 = lds + csub * CHA + 9 * cl;
     if constexpr (SPLIT) fa = lds + 2 * cb * CHA;
-    else if constexpr (S == 3) fa = lds + SUBS * CHA + cb * CHB;
+    else if constexpr (S == 3) fa = LEAN ? lds + cb * CHA : lds + SUBS * CHA + cb * CHB;
     else fa = lds + cb * CHA;
+    if constexpr (LEAN) return;
     load_tw<1>(w1, twl, l);
     if constexpr (S == 3) load_tw<2>(w2, twl, l);
     if constexpr (SPLIT) {
@@ -1489,12 +1514,13 @@ struct LineFft {
   template <bool INV>
   __device__ __forceinline__ void middle(c32 (&x)[E]) {
     get_a(x);
-    butterflies<8, INV>(x, w1);
+    stage<1, INV>(x, w1, l);
     if constexpr (S == 3) {
+      if constexpr (LEAN) wave_lds_order();   // a chunk is read before it is written
       put_b(x);
       wave_lds_order();
       get_b(x);
-      butterflies<P::radix(2), INV>(x, w2);
+      stage<2, INV>(x, w2, l);
     }
   }
   // coalesced values ct + i T of line cb -> transform at pt + i T of line pb
@@ -1514,7 +1540,7 @@ struct LineFft {
         x[q] = p[64 * q];
         x[q + 4] = p[CHC + 64 * q];
       }
-      butterflies<2, INV>(x, w3);
+      stage<3, INV>(x, w3, pt);
     }
   }
   // values pt + i T of line pb -> the same values at ct + i T of line cb
@@ -1551,24 +1577,25 @@ struct LineFft {
         x[q] = g[144 * q];
         x[q + 4] = g[CHA + 144 * q];
       }
-      butterflies<2, INV>(x, w3c);
+      stage<3, INV>(x, w3c, ct);
     } else if constexpr (S == 3) {
       wave_lds_order();
       get_a(x);
-      butterflies<8, INV>(x, w1);
+      stage<1, INV>(x, w1, l);
+      if constexpr (LEAN) wave_lds_order();   // a chunk is read before it is written
       put_b(x);
       before_barrier();
       __syncthreads();
 #pragma unroll
       for (int q = 0; q < E; ++q) x[q] = fa[slot_b(ct + q * T)];
-      butterflies<P::radix(2), INV>(x, w2c);
+      stage<2, INV>(x, w2c, ct);
     } else {
       before_barrier();
       __syncthreads();
       const c32* g = fa + ct + (ct >> 3);
 #pragma unroll
       for (int q = 0; q < E; ++q) x[q] = g[q * (T + T / 8)];
-      butterflies<8, INV>(x, w1c);
+      stage<1, INV>(x, w1c, ct);
     }
   }
 };
@@ -1613,6 +1640,13 @@ template <int N, int TT>
 constexpr int resident_used() {
   return resident_base<N, TT>() + (N / 8 * TT > 64 ? N / 8 * TT : 64) + 16;
 }
+// the lean form's: transforms, twiddle table, error sums
+template <int N, int TT>
+constexpr int resident_lean_base() { return LineFft<N, TT, true>::LDS + N; }
+template <int N, int TT>
+constexpr int resident_lean_used() {
+  return resident_lean_base<N, TT>() + (N / 8 * TT > 64 ? N / 8 * TT : 64) + 16;
+}
 template <int N, int TT>
 constexpr int resident_lds_elems() {
   constexpr int base = resident_used<N, TT>();
@@ -1620,16 +1654,26 @@ constexpr int resident_lds_elems() {
   return base > half ? base : half;
 }
 
+// MANY: several frames, in exchange mode 3 (two wavefronts per SIMD) or, in
+// mode 2, lean (four; twice the frames at once, n <= 512).  With one round of
+// frames mode 3's shorter exchange wins; in rounds the SIMDs' occupancy does:
+// one frame's barriers run under another's transforms.  Its registers are
+// those of 32 spilled values at 512^2; reading modulus and support again in
+// every step instead frees them and takes 4 % longer.  Microseconds per step,
+// mode 3 / lean: 512^2 x 4 10.1 / 11.5, x 8 19.0 / 16.5, x 16 36.7 / 32.3;
+// 256^2 x 16 10.3 / 10.3, x 32 19.5 / 15.5, x 64 38.5 / 29.6; 1024^2 x 2 21.5 / 28.9.
 template <int N, int TT, int E, int XM, bool MANY>
-__global__ void __launch_bounds__((N / E) * TT, 2)
+__global__ void __launch_bounds__((N / E) * TT, MANY && XM == 2 ? 4 : 2)
     k_resident(PassArgs a, const RStep* __restrict__ steps, int nsteps, double* errp0,
                long long errp_step, unsigned* flags, int* flag, c32* ll, int nframes) {
   constexpr int NT = (N / E) * TT;
   constexpr int NB = N / TT;
   constexpr int T = N / E;
-  using LF = LineFft<N, TT>;
+  constexpr bool LEAN = MANY && XM == 2;
+  using LF = LineFft<N, TT, LEAN>;
   static_assert(E == LF::E && LdsPlan<N, TT>::FULL_TW, "8 values per thread, the whole table");
-  __shared__ c32 lds[MANY ? resident_used<N, TT>() : resident_lds_elems<N, TT>()];
+  __shared__ c32 lds[LEAN ? resident_lean_used<N, TT>()
+                          : MANY ? resident_used<N, TT>() : resident_lds_elems<N, TT>()];
   static_assert(sizeof(lds) <= kLdsBytes, "resident kernel does not fit in LDS");
   // the shrinkwrap blur lines, staged outputs and weights, the reductions'
   // scratch (and the twiddle table until the threads have taken theirs)
@@ -1637,7 +1681,8 @@ __global__ void __launch_bounds__((N / E) * TT, 2)
   float* swwl = swl + sw_lds_floats<N, TT>();   // blur weights
   static_assert(sw_lds_floats<N, TT>() >= 2 * N, "the shrinkwrap area holds the table");
   // the error partials by coalesced thread, then the wavefronts' sums
-  double* eord = reinterpret_cast<double*>(lds + resident_base<N, TT>());
+  double* eord = reinterpret_cast<double*>(
+      lds + (LEAN ? resident_lean_base<N, TT>() : resident_base<N, TT>()));
   double* ewave = eord + (NT > 64 ? NT : 64);
   const int tid = threadIdx.x;
   const int fl = MANY ? blockIdx.x / NB : 0;    // frame of the launch
@@ -1688,6 +1733,9 @@ __global__ void __launch_bounds__((N / E) * TT, 2)
   bool given = false;   // mode 3: to_col holds the step's Phi (else phi does)
   auto cpos = [&](int i) { return (unsigned)col_pos<N, TT, E>(cband, cb, ct, i); };
   auto rpos = [&](int i) { return (unsigned)row_pos<N, TT, E>(rband, cb, ct, i); };
+  // distance of a thread's consecutive values in either direction
+  const unsigned CS = (unsigned)(col_pos<N, TT, E>(0, 0, 0, 1) - col_pos<N, TT, E>(0, 0, 0, 0));
+  const unsigned RS = (unsigned)(row_pos<N, TT, E>(0, 0, 0, 1) - row_pos<N, TT, E>(0, 0, 0, 0));
   // whether step j has a column phase
   auto has_col = [&](const RStep& q) {
     return !(q.c.flags & kNoOut) || q.err || (q.c.flags & kSwFin);
@@ -1712,7 +1760,7 @@ __global__ void __launch_bounds__((N / E) * TT, 2)
         ll_take<DELAY>(x, to_col, llw, cpos);
       } else {
 #pragma unroll
-        for (int i = 0; i < E; ++i) x[i] = xld<XM>(phi, cpos(i));
+        for (int i = 0; i < E; ++i) x[i] = xld<XM>(phi, cpos(0), i * CS);
       }
       // a fused shrinkwrap's column half: its weights, fetched with Phi
       float wcol = 0.0f;
@@ -1740,7 +1788,7 @@ __global__ void __launch_bounds__((N / E) * TT, 2)
           ll_give(x, to_row, cpos);
         } else {
 #pragma unroll
-          for (int i = 0; i < E; ++i) xst<XM>(phi, cpos(i), x[i]);
+          for (int i = 0; i < E; ++i) xst<XM>(phi, cpos(0), i * CS, x[i]);
         }
       }
       if (swfin) {
@@ -1782,7 +1830,7 @@ __global__ void __launch_bounds__((N / E) * TT, 2)
         ll_take<DELAY>(x, to_row, llw, rpos);
       } else {
 #pragma unroll
-        for (int i = 0; i < E; ++i) x[i] = xld<XM>(phi, rpos(i));
+        for (int i = 0; i < E; ++i) x[i] = xld<XM>(phi, rpos(0), i * RS);
       }
     }
     if (!LL || noout) err_waves();
@@ -1836,7 +1884,7 @@ __global__ void __launch_bounds__((N / E) * TT, 2)
         given = true;
       } else {
 #pragma unroll
-        for (int i = 0; i < E; ++i) xst<XM>(phi, rpos(i), x[i]);
+        for (int i = 0; i < E; ++i) xst<XM>(phi, rpos(0), i * RS, x[i]);
       }
     }
     if (swrow) {
@@ -1993,7 +2041,7 @@ __global__ void __launch_bounds__((N / E) * TT)
     tf.template to_coalesced<false>(x, emptied);
     if (last) {
 #pragma unroll
-      for (int i = 0; i < E; ++i) xst<3>(a.phi, rpos(i), x[i]);
+      for (int i = 0; i < E; ++i) xst<3>(a.phi, rpos(i), 0, x[i]);
     } else {
       ll_give(x, to_col, rpos);
     }
@@ -3387,6 +3435,15 @@ static hipError_t tfcol_nt(int kind, const c32* phi, const float* goal, int rows
   return hipGetLastError();
 }
 
+// k_resident for several frames: exchange mode 3, or 2 (lean)
+template <int N, int TT, int E>
+static const void* resident_many(int xm) {
+  if constexpr (N <= kResidentLeanMax) {
+    if (xm == 2) return reinterpret_cast<const void*>(&k_resident<N, TT, E, 2, true>);
+  }
+  return reinterpret_cast<const void*>(&k_resident<N, TT, E, 3, true>);
+}
+
 template <int N, int TT, int E>
 static hipError_t resident_nt(int xm, const PassArgs& a, const RStep* steps, int nsteps,
                               double* errp0, long long errp_step, unsigned* flags, int* flag,
@@ -3397,7 +3454,8 @@ static hipError_t resident_nt(int xm, const PassArgs& a, const RStep* steps, int
                      reinterpret_cast<u32x2*>(ll), count, fill);
   void* args[] = {(void*)&a,     (void*)&steps, (void*)&nsteps, (void*)&errp0, (void*)&errp_step,
                   (void*)&flags, (void*)&flag,  (void*)&ll,     (void*)&frames};
-  const void* fn = frames > 1 ? reinterpret_cast<const void*>(&k_resident<N, TT, E, 3, true>)
+  if (frames > 1 && xm != 3 && !(xm == 2 && N <= kResidentLeanMax)) return hipErrorInvalidValue;
+  const void* fn = frames > 1 ? resident_many<N, TT, E>(xm)
                    : xm == 1 ? reinterpret_cast<const void*>(&k_resident<N, TT, E, 1, false>)
                    : xm == 2 ? reinterpret_cast<const void*>(&k_resident<N, TT, E, 2, false>)
                    : xm == 3 ? reinterpret_cast<const void*>(&k_resident<N, TT, E, 3, false>)
@@ -3432,10 +3490,10 @@ static hipError_t resident_rl_dispatch(int tile, int ept, const c32* tw, c32* u,
 
 // frames that one launch of several holds at once on the current device
 template <int N, int TT, int E>
-static hipError_t resident_frames_nt(int* out) {
+static hipError_t resident_frames_nt(int xm, int* out) {
   int occ = 0, dev = 0, cus = 0;
   hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-      &occ, reinterpret_cast<const void*>(&k_resident<N, TT, E, 3, true>), (N / E) * TT, 0);
+      &occ, resident_many<N, TT, E>(xm), (N / E) * TT, 0);
   if (e == hipSuccess) e = hipGetDevice(&dev);
   if (e == hipSuccess)
     e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
@@ -3485,11 +3543,11 @@ static hipError_t resident_dispatch(int tile, int ept, int xm, const PassArgs& a
 }
 
 template <int N>
-static hipError_t resident_frames_dispatch(int tile, int ept, int* out) {
+static hipError_t resident_frames_dispatch(int tile, int ept, int xm, int* out) {
   if constexpr (N >= 64 && N <= 1024) {
-    if (tile == 4 && ept == 8) return resident_frames_nt<N, 4, 8>(out);
+    if (tile == 4 && ept == 8) return resident_frames_nt<N, 4, 8>(xm, out);
     if constexpr (N >= 256 && N <= 512) {
-      if (tile == 2 && ept == 8) return resident_frames_nt<N, 2, 8>(out);
+      if (tile == 2 && ept == 8) return resident_frames_nt<N, 2, 8>(xm, out);
     }
   }
   return hipErrorInvalidValue;
@@ -3574,7 +3632,7 @@ constexpr bool shape_ok() {
                           int nsteps, double* errp0, long long errp_step, unsigned* bar,    \
                           int* flag, c32* ll, int fill, int frames, int at_once,                 \
                           hipStream_t st);                                                  \
-  hipError_t resident_frames_##n(int tile, int ept, int* out);                              \
+  hipError_t resident_frames_##n(int tile, int ept, int xm, int* out);                              \
   hipError_t resident_rl_##n(int tile, int ept, const c32* tw, c32* u, const float* d,      \
                              const c32* P, const c32* Ph, int iterations, float inv_nn,     \
                              unsigned polls, int* flag, c32* ll, hipStream_t st);           \
@@ -3689,8 +3747,8 @@ constexpr bool shape_ok() {
     return resident_dispatch<n>(tile, ept, xm, a, steps, nsteps, errp0, errp_step, bar,     \
                                 flag, ll, fill, frames, at_once, st);                            \
   }                                                                                         \
-  hipError_t resident_frames_##n(int tile, int ept, int* out) {                             \
-    return resident_frames_dispatch<n>(tile, ept, out);                                     \
+  hipError_t resident_frames_##n(int tile, int ept, int xm, int* out) {                             \
+    return resident_frames_dispatch<n>(tile, ept, xm, out);                                     \
   }                                                                                         \
   hipError_t resident_rl_##n(int tile, int ept, const c32* tw, c32* u, const float* d,      \
                              const c32* P, const c32* Ph, int iterations, float inv_nn,     \
@@ -3792,8 +3850,8 @@ hipError_t launch_resident_rl(int n, int tile, int ept, const c32* tw, c32* u, c
   SPK_SIZE_SWITCH(resident_rl, tile, ept, tw, u, d, P, Ph, iterations, inv_nn, polls, flag, ll, st)
 }
 
-hipError_t resident_frames(int n, int tile, int ept, int* out) {
-  SPK_SIZE_SWITCH(resident_frames, tile, ept, out)
+hipError_t resident_frames(int n, int tile, int ept, int xm, int* out) {
+  SPK_SIZE_SWITCH(resident_frames, tile, ept, xm, out)
 }
 
 hipError_t launch_resident_ipsf(int n, int tile, int ept, const PassArgs& a, const c32* ipsf,

@@ -75,7 +75,7 @@ typedef struct spk_tune {
                          and iterate held on chip, Phi exchanged between the
                          workgroups, shrinkwraps of a single frame inside the
                          launch); plans of several frames with per_frame = 0
-                         too, a few at a time, up to three rounds.  0: where
+                         too, some at a time, up to four rounds.  0: where
                          it pays (the default: not for blocks of a few steps,
                          many frames), 1: where built, 2: never.  The
                          workgroups of a launch wait for each other: it is a

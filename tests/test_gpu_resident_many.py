@@ -36,11 +36,14 @@ def run(ctx, n, batch, shared, calls, trace, **kw):
     return out, counts
 
 
-# one round full and partial, a remainder, three rounds; workgroups of half a
-# wavefront to eight
+# polled values: one round full and partial; the lean form: the first batch that
+# takes it, a full round, remainders, more rounds; 1024^2 in rounds of polled
+# values; workgroups of half a wavefront to eight
 @pytest.mark.parametrize("n,batch,shared,tile,trace", [
     (64, 2, True, 0, True), (64, 129, False, 0, False), (128, 65, True, 0, True),
     (256, 16, False, 0, True), (256, 17, True, 0, False), (256, 5, True, 2, True),
+    (64, 257, True, 0, True), (128, 130, False, 0, True), (256, 33, False, 0, True),
+    (256, 35, True, 2, True), (512, 8, False, 0, False), (512, 17, True, 2, True),
     (512, 3, False, 0, True), (512, 9, True, 0, True), (1024, 2, True, 0, True),
     (1024, 3, False, 0, False)])
 def test_resident_frames_equal_per_pass(gpu_ctx, n, batch, shared, tile, trace):
@@ -58,7 +61,7 @@ def test_resident_frames_equal_per_pass(gpu_ctx, n, batch, shared, tile, trace):
 
 @pytest.mark.parametrize("n,batch,steps,resident", [
     (256, 1, 5, False), (256, 1, 6, True), (1024, 1, 2, False), (1024, 1, 3, True),
-    (256, 16, 6, True), (256, 32, 15, False), (256, 32, 16, True), (512, 13, 40, False),
+    (256, 16, 6, True), (256, 33, 11, False), (256, 33, 12, True), (512, 25, 60, False),
     (1024, 4, 40, False)])
 def test_default_choice(gpu_ctx, n, batch, steps, resident):
     p = Plan(gpu_ctx, n, batch=batch)
