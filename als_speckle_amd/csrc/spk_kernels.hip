@@ -1133,7 +1133,8 @@ __global__ void __launch_bounds__((N / E) * TT)
 }
 
 // ---------------------------------------------------------------------------
-// Resident single-frame iteration block (k_resident).  One cooperative
+// Resident iteration block (k_resident) of one frame, or of several with one
+// schedule.  One cooperative
 // launch of one workgroup per band runs a block of steps; the workgroup of
 // band q owns column band q (column phase) and row band q (row phase) for the
 // whole launch and keeps the frame's modulus (its column band) and support
@@ -1657,9 +1658,9 @@ constexpr int resident_lds_elems() {
 // MANY: several frames, in exchange mode 3 (two wavefronts per SIMD) or, in
 // mode 2, lean (four; twice the frames at once, n <= 512).  With one round of
 // frames mode 3's shorter exchange wins; in rounds the SIMDs' occupancy does:
-// one frame's barriers run under another's transforms.  Its registers are
-// those of 32 spilled values at 512^2; reading modulus and support again in
-// every step instead frees them and takes 4 % longer.  Microseconds per step,
+// one frame's barriers run under another's transforms.  At 512^2 it spills 32
+// registers; with modulus and support read again in every step it spills 10
+// and takes 4 % longer.  Microseconds per step,
 // mode 3 / lean: 512^2 x 4 10.1 / 11.5, x 8 19.0 / 16.5, x 16 36.7 / 32.3;
 // 256^2 x 16 10.3 / 10.3, x 32 19.5 / 15.5, x 64 38.5 / 29.6; 1024^2 x 2 21.5 / 28.9.
 template <int N, int TT, int E, int XM, bool MANY>
@@ -3317,6 +3318,7 @@ template <int N, int TT, int E>
 static hipError_t colpass_nt(int mode, const PassArgs& a, int frames, int zdim,
                              hipStream_t st) {
   dim3 grid(N / TT, frames, zdim), block((N / E) * TT);
+  // four columns per workgroup where the pieces' size counts (k_colpass_pair)
   if constexpr (N >= 2048 && TT == 2 && E == 16) {
     if (mode == 0) {
       launch_pass(k_colpass_pair<N, E>, dim3(N / 4, frames, zdim), block, st, a);
