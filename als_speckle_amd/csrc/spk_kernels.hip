@@ -713,9 +713,9 @@ __global__ void __launch_bounds__((N / E) * TT) k_colpass(PassArgs a) {
 // the tiles of a row pair are 64 contiguous bytes instead of 32.  Bound by
 // those scattered pieces: with 32 bytes the 4096^2 pass took 113 us, 57 of them
 // without its stores and loads, 89 with contiguous stores; 64 bytes 90 us.
-// 2048^2: one frame 23.3 -> 22.8 us, four 78 -> 69, ten 203 -> 185.  1024^2 in
-// tile 2: no gain (16 frames 61.9 / 64.5).  Values, error sums and their order
-// are colpass_item's.  grid (n/4, frames, z)
+// 2048^2: four frames 78 -> 69 us, ten 203 -> 185, one and two no gain
+// (colpass_nt).  1024^2 in tile 2: no gain (16 frames 61.9 / 64.5).  Values,
+// error sums and their order are colpass_item's.  grid (n/4, frames, z)
 // ---------------------------------------------------------------------------
 template <int N, int E>
 __global__ void __launch_bounds__((N / E) * 2) k_colpass_pair(PassArgs a) {
@@ -3318,9 +3318,14 @@ template <int N, int TT, int E>
 static hipError_t colpass_nt(int mode, const PassArgs& a, int frames, int zdim,
                              hipStream_t st) {
   dim3 grid(N / TT, frames, zdim), block((N / E) * TT);
-  // four columns per workgroup where the pieces' size counts (k_colpass_pair)
+  // four columns per workgroup where the pieces' size counts: at 4096^2, and at
+  // 2048^2 from three frames (times projections) on: up to there the frames'
+  // arrays, 100 MB each, stay in the 256 MB of the last cache and the pieces'
+  // size costs less than half as many workgroups do.  Microseconds per iteration at 2048^2, two / four columns: one frame
+  // 49.7 / 49.6, two 83.9 / 85.3, three 120.0 / 119.2, four 173 / 160, ten
+  // 455 / 425; DM, one frame 78.2 / 78.9, two 147 / 141, four 330 / 306.
   if constexpr (N >= 2048 && TT == 2 && E == 16) {
-    if (mode == 0) {
+    if (mode == 0 && (N >= 4096 || frames * zdim >= 3)) {
       launch_pass(k_colpass_pair<N, E>, dim3(N / 4, frames, zdim), block, st, a);
       return hipGetLastError();
     }

@@ -1,0 +1,44 @@
+"""Which launches the library's calls make, and what they do when one fails:
+its host code on a HIP of host functions (emu/fake_hip.cpp), without a GPU."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+@pytest.fixture(scope="module")
+def fake_so(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("fake") / "libfake_hip.so")
+    subprocess.run(["g++", "-O1", "-std=c++17", "-shared", "-fPIC",
+                    os.path.join(HERE, "emu", "fake_hip.cpp"), "-o", so], check=True)
+    return so
+
+
+@pytest.fixture
+def program(fake_so):
+    def run(text):
+        r = subprocess.run([sys.executable, os.path.join(HERE, "emu", "fake_run.py"), fake_so],
+                           input=text, capture_output=True, text=True, timeout=120)
+        assert r.returncode == 0, r.stdout[-2000:] + r.stderr[-2000:]
+        return r.stdout
+    return run
+
+
+def test_column_pass_of_four_columns_where_it_is_faster(program):
+    """At 2048^2 from three columns of a band pair on (frames times projections),
+    at 4096^2 always."""
+    program("""
+for n, batch, step, pair in [(2048, 1, HIO, 0), (2048, 2, HIO, 0), (2048, 1, DM, 0),
+                             (2048, 3, HIO, 1), (2048, 2, DM, 1), (4096, 1, HIO, 1),
+                             (4096, 1, DM, 1), (1024, 4, HIO, 0)]:
+    p = Plan(n, batch, resident=2)
+    ok(p.iterate([step] * 2))
+    got = [(w[1].split("<")[0], int(w[2])) for w in launches() if "colpass" in w[1]]
+    tile = 4 if n == 1024 else 2
+    want = ("k_colpass_pair", n // 4) if pair else ("k_colpass", n // tile)
+    assert got == [want] * 2, (n, batch, step, got)
+    p.close()
+""")
