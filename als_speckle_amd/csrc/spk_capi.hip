@@ -24,11 +24,15 @@ int fail(int code, const std::string& msg) {
   return code;
 }
 
+// (the error is taken off the runtime, where the next call's launch check
+// would find it)
 #define SPK_HIP(call)                                                        \
   do {                                                                       \
     hipError_t e_ = (call);                                                  \
-    if (e_ != hipSuccess)                                                    \
+    if (e_ != hipSuccess) {                                                  \
+      (void)hipGetLastError();                                               \
       return fail(SPK_EHIP, std::string(#call) + ": " + hipGetErrorString(e_)); \
+    }                                                                        \
   } while (0)
 
 #define SPK_REQUIRE(cond, code, msg) \
@@ -1401,7 +1405,6 @@ int iter_step(IterRun& r, int k, int* next) {
     PassArgs ra = base_args(p);
     ra.swr_tab = r.res_fused[k] ? (const SwParam*)r.dptr(r.res_sw_off[k]) : nullptr;
     const int fill = p->rll_fill;
-    p->rll_fill = false;
     if ((rc = prof_arm(p, 2))) return rc;
     double* errp = r.err_trace ? p->errp : nullptr;
     const RStep* tab = (const RStep*)r.dptr(r.res_off[k]);
@@ -1413,6 +1416,7 @@ int iter_step(IterRun& r, int k, int* next) {
       SPK_HIP(launch_resident(p->n, p->tile, p->ept, p->res_xm, ra, tab, r.res_n[k], errp,
                               (long long)B * p->bands, rsync, (int*)(p->pbar + 1), p->rll, fill,
                               B, g, st));
+    p->rll_fill = false;   // not before both its launches are queued
     p->res_launches++;
     p->res_steps += r.res_n[k];
     p->sw_fused_count += r.res_fused[k];

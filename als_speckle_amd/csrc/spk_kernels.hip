@@ -3442,6 +3442,13 @@ static hipError_t tfcol_nt(int kind, const c32* phi, const float* goal, int rows
   return hipGetLastError();
 }
 
+static hipError_t resident_begin(int blocks, unsigned* flags, int words, int* flag, c32* ll,
+                                 int count, int fill, hipStream_t st) {
+  hipLaunchKernelGGL(k_resident_begin, dim3(blocks), dim3(256), 0, st, flags, words, flag,
+                     reinterpret_cast<u32x2*>(ll), count, fill);
+  return hipGetLastError();
+}
+
 // k_resident for several frames: exchange mode 3, or 2 (lean)
 template <int N, int TT, int E>
 static const void* resident_many(int xm) {
@@ -3457,8 +3464,8 @@ static hipError_t resident_nt(int xm, const PassArgs& a, const RStep* steps, int
                               c32* ll, int fill, int frames, int at_once, hipStream_t st) {
   const int words = at_once * (N / TT) * 32, count = xm == 3 ? at_once * 2 * N * N : 0;
   const int blocks = fill && count ? 1024 : std::max(1, words / 256);
-  hipLaunchKernelGGL(k_resident_begin, dim3(blocks), dim3(256), 0, st, flags, words, flag,
-                     reinterpret_cast<u32x2*>(ll), count, fill);
+  const hipError_t begun = resident_begin(blocks, flags, words, flag, ll, count, fill, st);
+  if (begun != hipSuccess) return begun;
   void* args[] = {(void*)&a,     (void*)&steps, (void*)&nsteps, (void*)&errp0, (void*)&errp_step,
                   (void*)&flags, (void*)&flag,  (void*)&ll,     (void*)&frames};
   if (frames > 1 && xm != 3 && !(xm == 2 && N <= kResidentLeanMax)) return hipErrorInvalidValue;
@@ -3485,8 +3492,8 @@ static hipError_t resident_rl_dispatch(int tile, int ept, const c32* tw, c32* u,
                                        unsigned polls, int* flag, c32* ll, hipStream_t st) {
   if constexpr (N >= 64 && N <= 1024) {
     if (tile != 4 || ept != 8) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_resident_begin, dim3(1024), dim3(256), 0, st, nullptr, 0, flag,
-                       reinterpret_cast<u32x2*>(ll), 2 * N * N, 1);
+    const hipError_t begun = resident_begin(1024, nullptr, 0, flag, ll, 2 * N * N, 1, st);
+    if (begun != hipSuccess) return begun;
     void* args[] = {(void*)&tw,     (void*)&u,     (void*)&d,    (void*)&P,  (void*)&Ph,
                     (void*)&iterations, (void*)&inv_nn, (void*)&polls, (void*)&flag, (void*)&ll};
     return hipLaunchCooperativeKernel(reinterpret_cast<const void*>(&k_resident_rl<N, 4, 8>),
@@ -3512,8 +3519,9 @@ template <int N, int TT, int E>
 static hipError_t resident_ipsf_nt(const PassArgs& a, const c32* ipsf, const RStep* steps,
                                    int nsteps, double* errp0, long long errp_step, int* flag,
                                    c32* ll, int fill, hipStream_t st) {
-  hipLaunchKernelGGL(k_resident_begin, dim3(fill ? 1024 : 1), dim3(256), 0, st, nullptr, 0, flag,
-                     reinterpret_cast<u32x2*>(ll), 2 * N * N, fill);
+  const hipError_t begun =
+      resident_begin(fill ? 1024 : 1, nullptr, 0, flag, ll, 2 * N * N, fill, st);
+  if (begun != hipSuccess) return begun;
   void* args[] = {(void*)&a,     (void*)&ipsf,      (void*)&steps, (void*)&nsteps,
                   (void*)&errp0, (void*)&errp_step, (void*)&flag,  (void*)&ll};
   if (g_launch_events[0]) (void)hipEventRecord(g_launch_events[0], st);

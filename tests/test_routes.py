@@ -42,3 +42,21 @@ for n, batch, step, pair in [(2048, 1, HIO, 0), (2048, 2, HIO, 0), (2048, 1, DM,
     assert got == [want] * 2, (n, batch, step, got)
     p.close()
 """)
+
+
+@pytest.mark.parametrize("ipsf", [False, True])
+def test_exchange_buffers_are_emptied_after_a_launch_that_failed(program, ipsf):
+    """The polled exchange takes any value that is not the empty pattern: the
+    launch that empties new buffers is made again when a launch behind it failed."""
+    program("""
+p = Plan(256, ipsf=%r)
+knob("fail_cooperative", 1)
+assert p.iterate([HIO] * 8) == -2
+begin = [w for w in launches() if "begin" in w]
+assert len(begin) == 1 and int(begin[0][-2]) == 2 * 256 * 256 and begin[0][-1] == "1", begin
+for fill in "100":
+    ok(p.iterate([HIO] * 8))
+    words = launches()
+    assert sum(w[0] == "coop" for w in words) == 1
+    assert [w[-1] for w in words if "begin" in w] == [fill], words
+""" % ipsf)
