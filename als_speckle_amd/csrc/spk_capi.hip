@@ -190,6 +190,7 @@ struct spk_plan {
   int resident_min = 2;        // steps of a block that runs resident
   bool res_allowed = true;     // spk_tune.resident != 2
   int xm = 0;
+  int ipsf_fits = -1, rl_fits = -1;   // resident_fits
   int res_xm = 0;              // that of this plan's launches (several frames: 3 or 2)
   // resident launches: the two exchange buffers of mode 3 (n*n values each),
   // then the barrier flags (a 128-byte line per band)
@@ -240,6 +241,18 @@ struct spk_plan {
 };
 
 namespace {
+
+// whether the device holds all workgroups of one frame of a resident form at
+// once; asked when the form is first wanted (cache: -1 until then)
+bool resident_fits(spk_plan* p, ResidentForm form, int* cache) {
+  if (*cache < 0) {
+    int fit = 0;
+    const bool got = resident_frames(p->n, p->tile, p->ept, form, 3, &fit) == hipSuccess;
+    if (!got) (void)hipGetLastError();
+    *cache = got && fit > 0;
+  }
+  return *cache != 0;
+}
 
 int set_device(spk_ctx* ctx) {
   SPK_REQUIRE(ctx, SPK_EINVAL, "null context");
@@ -661,20 +674,23 @@ int spk_plan_create(spk_ctx* ctx, int n, int batch, int shared, const spk_tune* 
   const int res_mode = tune ? tune->resident : 0;
   p->res_allowed = res_mode != 2;
   if (res_mode != 2 && resident_supported(n, tile, ept)) {
-    int fit = 1;
+    int fit = 0;
     // (the occupancy query only where the answer can matter)
     const bool few = batch <= resident_rounds(n) * 2 * resident_fit(n);
     p->res_xm = p->xm;
-    if (batch > 1) {
+    if (batch == 1) {
+      if (resident_frames(n, tile, ept, kResidentOne, p->xm, &fit) != hipSuccess) fit = 0;
+    } else {
       if (p->xm != 3 || !(few || res_mode == 1) ||
-          resident_frames(n, tile, ept, 3, &fit) != hipSuccess)
+          resident_frames(n, tile, ept, kResidentMany, 3, &fit) != hipSuccess)
         fit = 0;
       // more than one round of mode 3: the lean form's
       if (fit && batch > fit && n <= kResidentLeanMax) {
         p->res_xm = 2;
-        if (resident_frames(n, tile, ept, 2, &fit) != hipSuccess) fit = 0;
+        if (resident_frames(n, tile, ept, kResidentMany, 2, &fit) != hipSuccess) fit = 0;
       }
     }
+    (void)hipGetLastError();   // a query that failed is no error of this call
     const int rounds = fit ? (batch + fit - 1) / fit : 0;
     if (rounds && (rounds <= resident_rounds(n) || res_mode == 1)) {
       p->resident = (batch + rounds - 1) / rounds;   // as even as they go
@@ -1176,7 +1192,8 @@ int iter_prepare(spk_plan* p, const spk_step* steps, int nsteps, int per_frame,
   // ends at every shrinkwrap; with a spectrum there is none (the rescaled map
   // is gathered from all over the frame).
   if (blocks && p->resident && (B == 1 || !per_frame) && !p->spec_on && !p->persist &&
-      !p->capturing && (!p->ipsf_on || (B == 1 && p->xm == 3 && p->tile == 4))) {
+      !p->capturing && (!p->ipsf_on || (B == 1 && p->xm == 3 && p->tile == 4 &&
+                                              resident_fits(p, kResidentIpsf, &p->ipsf_fits)))) {
     auto fits = [&](int j) { return !any_dm[j] && !emits[j]; };
     std::vector<RStep> rs;
     std::vector<SwParam> sp;
@@ -2044,7 +2061,8 @@ int spk_coherence_rl(spk_plan* p, const float* est, int rows, int cols, const fl
   // the updates in one launch where the resident form is built (W and w hold
   // its exchange), otherwise as launches
   const bool one = iterations > 0 && p->res_allowed && p->xm == 3 && tile == 4 && !p->capturing &&
-                   resident_supported(n, tile, p->ept);
+                   resident_supported(n, tile, p->ept) &&
+                   resident_fits(p, kResidentRl, &p->rl_fits);
   if (one)
     SPK_HIP(launch_resident_rl(n, tile, p->ept, p->tw, u, d, P, Ph, iterations, inv_nn, p->polls,
                                (int*)(p->pbar + 1), W, st));

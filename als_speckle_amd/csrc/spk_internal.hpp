@@ -205,10 +205,13 @@ hipError_t launch_resident(int n, int tile, int ept, int xm, const PassArgs& a,
                            const RStep* steps, int nsteps, double* errp0, long long errp_step,
                            unsigned* flags, int* flag, c32* ll, int fill, int frames, int at_once,
                            hipStream_t st);
-// frames that one launch of several holds at once on the current device, in
-// exchange mode 3 or (n <= kResidentLeanMax) 2
+// frames whose workgroups the current device holds at once, by form: of one
+// frame in any exchange mode, of several in mode 3 or (n <= kResidentLeanMax) 2,
+// k_resident_ipsf and k_resident_rl.  A form runs where this is at least 1:
+// its workgroups wait for each other.
 constexpr int kResidentLeanMax = 512;
-hipError_t resident_frames(int n, int tile, int ept, int xm, int* out);
+enum ResidentForm { kResidentOne, kResidentMany, kResidentIpsf, kResidentRl };
+hipError_t resident_frames(int n, int tile, int ept, ResidentForm form, int xm, int* out);
 // the same with a partially coherent projection by the tiled ipsf, in tile 4
 // and exchange mode 3 (k_resident_ipsf); fused shrinkwraps are not part of it
 hipError_t launch_resident_ipsf(int n, int tile, int ept, const PassArgs& a, const c32* ipsf,

@@ -3449,31 +3449,42 @@ static hipError_t resident_begin(int blocks, unsigned* flags, int words, int* fl
   return hipGetLastError();
 }
 
-// k_resident for several frames: exchange mode 3, or 2 (lean)
+// the kernel of a resident form and exchange mode, null where it is not built
 template <int N, int TT, int E>
-static const void* resident_many(int xm) {
-  if constexpr (N <= kResidentLeanMax) {
-    if (xm == 2) return reinterpret_cast<const void*>(&k_resident<N, TT, E, 2, true>);
+static const void* resident_kernel(ResidentForm form, int xm) {
+  switch (form) {
+    case kResidentOne:
+      return xm == 1   ? reinterpret_cast<const void*>(&k_resident<N, TT, E, 1, false>)
+             : xm == 2 ? reinterpret_cast<const void*>(&k_resident<N, TT, E, 2, false>)
+             : xm == 3 ? reinterpret_cast<const void*>(&k_resident<N, TT, E, 3, false>)
+                       : reinterpret_cast<const void*>(&k_resident<N, TT, E, 0, false>);
+    case kResidentMany:
+      if constexpr (N <= kResidentLeanMax) {
+        if (xm == 2) return reinterpret_cast<const void*>(&k_resident<N, TT, E, 2, true>);
+      }
+      return xm == 3 ? reinterpret_cast<const void*>(&k_resident<N, TT, E, 3, true>) : nullptr;
+    case kResidentIpsf:
+      if constexpr (TT == 4) return reinterpret_cast<const void*>(&k_resident_ipsf<N, TT, E>);
+      return nullptr;
+    case kResidentRl:
+      if constexpr (TT == 4) return reinterpret_cast<const void*>(&k_resident_rl<N, TT, E>);
+      return nullptr;
   }
-  return reinterpret_cast<const void*>(&k_resident<N, TT, E, 3, true>);
+  return nullptr;
 }
 
 template <int N, int TT, int E>
 static hipError_t resident_nt(int xm, const PassArgs& a, const RStep* steps, int nsteps,
                               double* errp0, long long errp_step, unsigned* flags, int* flag,
                               c32* ll, int fill, int frames, int at_once, hipStream_t st) {
+  const void* fn = resident_kernel<N, TT, E>(frames > 1 ? kResidentMany : kResidentOne, xm);
+  if (!fn) return hipErrorInvalidValue;
   const int words = at_once * (N / TT) * 32, count = xm == 3 ? at_once * 2 * N * N : 0;
   const int blocks = fill && count ? 1024 : std::max(1, words / 256);
   const hipError_t begun = resident_begin(blocks, flags, words, flag, ll, count, fill, st);
   if (begun != hipSuccess) return begun;
   void* args[] = {(void*)&a,     (void*)&steps, (void*)&nsteps, (void*)&errp0, (void*)&errp_step,
                   (void*)&flags, (void*)&flag,  (void*)&ll,     (void*)&frames};
-  if (frames > 1 && xm != 3 && !(xm == 2 && N <= kResidentLeanMax)) return hipErrorInvalidValue;
-  const void* fn = frames > 1 ? resident_many<N, TT, E>(xm)
-                   : xm == 1 ? reinterpret_cast<const void*>(&k_resident<N, TT, E, 1, false>)
-                   : xm == 2 ? reinterpret_cast<const void*>(&k_resident<N, TT, E, 2, false>)
-                   : xm == 3 ? reinterpret_cast<const void*>(&k_resident<N, TT, E, 3, false>)
-                             : reinterpret_cast<const void*>(&k_resident<N, TT, E, 0, false>);
   if (g_launch_events[0]) {
     (void)hipEventRecord(g_launch_events[0], st);
   }
@@ -3496,18 +3507,19 @@ static hipError_t resident_rl_dispatch(int tile, int ept, const c32* tw, c32* u,
     if (begun != hipSuccess) return begun;
     void* args[] = {(void*)&tw,     (void*)&u,     (void*)&d,    (void*)&P,  (void*)&Ph,
                     (void*)&iterations, (void*)&inv_nn, (void*)&polls, (void*)&flag, (void*)&ll};
-    return hipLaunchCooperativeKernel(reinterpret_cast<const void*>(&k_resident_rl<N, 4, 8>),
-                                      dim3(N / 4), dim3((N / 8) * 4), args, 0, st);
+    return hipLaunchCooperativeKernel(resident_kernel<N, 4, 8>(kResidentRl, 3), dim3(N / 4),
+                                      dim3((N / 8) * 4), args, 0, st);
   }
   return hipErrorInvalidValue;
 }
 
-// frames that one launch of several holds at once on the current device
+// frames whose workgroups the current device holds at once
 template <int N, int TT, int E>
-static hipError_t resident_frames_nt(int xm, int* out) {
+static hipError_t resident_frames_nt(ResidentForm form, int xm, int* out) {
+  const void* fn = resident_kernel<N, TT, E>(form, xm);
+  if (!fn) return hipErrorInvalidValue;
   int occ = 0, dev = 0, cus = 0;
-  hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
-      &occ, resident_many<N, TT, E>(xm), (N / E) * TT, 0);
+  hipError_t e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&occ, fn, (N / E) * TT, 0);
   if (e == hipSuccess) e = hipGetDevice(&dev);
   if (e == hipSuccess)
     e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
@@ -3526,8 +3538,7 @@ static hipError_t resident_ipsf_nt(const PassArgs& a, const c32* ipsf, const RSt
                   (void*)&errp0, (void*)&errp_step, (void*)&flag,  (void*)&ll};
   if (g_launch_events[0]) (void)hipEventRecord(g_launch_events[0], st);
   hipError_t e = hipLaunchCooperativeKernel(
-      reinterpret_cast<const void*>(&k_resident_ipsf<N, TT, E>), dim3(N / TT), dim3((N / E) * TT),
-      args, 0, st);
+      resident_kernel<N, TT, E>(kResidentIpsf, 3), dim3(N / TT), dim3((N / E) * TT), args, 0, st);
   if (g_launch_events[0]) {
     (void)hipEventRecord(g_launch_events[1], st);
     g_launch_events[0] = g_launch_events[1] = nullptr;
@@ -3558,11 +3569,12 @@ static hipError_t resident_dispatch(int tile, int ept, int xm, const PassArgs& a
 }
 
 template <int N>
-static hipError_t resident_frames_dispatch(int tile, int ept, int xm, int* out) {
+static hipError_t resident_frames_dispatch(int tile, int ept, ResidentForm form, int xm,
+                                           int* out) {
   if constexpr (N >= 64 && N <= 1024) {
-    if (tile == 4 && ept == 8) return resident_frames_nt<N, 4, 8>(xm, out);
+    if (tile == 4 && ept == 8) return resident_frames_nt<N, 4, 8>(form, xm, out);
     if constexpr (N >= 256 && N <= 512) {
-      if (tile == 2 && ept == 8) return resident_frames_nt<N, 2, 8>(xm, out);
+      if (tile == 2 && ept == 8) return resident_frames_nt<N, 2, 8>(form, xm, out);
     }
   }
   return hipErrorInvalidValue;
@@ -3647,7 +3659,7 @@ constexpr bool shape_ok() {
                           int nsteps, double* errp0, long long errp_step, unsigned* bar,    \
                           int* flag, c32* ll, int fill, int frames, int at_once,                 \
                           hipStream_t st);                                                  \
-  hipError_t resident_frames_##n(int tile, int ept, int xm, int* out);                              \
+  hipError_t resident_frames_##n(int tile, int ept, ResidentForm form, int xm, int* out);   \
   hipError_t resident_rl_##n(int tile, int ept, const c32* tw, c32* u, const float* d,      \
                              const c32* P, const c32* Ph, int iterations, float inv_nn,     \
                              unsigned polls, int* flag, c32* ll, hipStream_t st);           \
@@ -3762,8 +3774,8 @@ constexpr bool shape_ok() {
     return resident_dispatch<n>(tile, ept, xm, a, steps, nsteps, errp0, errp_step, bar,     \
                                 flag, ll, fill, frames, at_once, st);                            \
   }                                                                                         \
-  hipError_t resident_frames_##n(int tile, int ept, int xm, int* out) {                             \
-    return resident_frames_dispatch<n>(tile, ept, xm, out);                                     \
+  hipError_t resident_frames_##n(int tile, int ept, ResidentForm form, int xm, int* out) {  \
+    return resident_frames_dispatch<n>(tile, ept, form, xm, out);                           \
   }                                                                                         \
   hipError_t resident_rl_##n(int tile, int ept, const c32* tw, c32* u, const float* d,      \
                              const c32* P, const c32* Ph, int iterations, float inv_nn,     \
@@ -3865,8 +3877,8 @@ hipError_t launch_resident_rl(int n, int tile, int ept, const c32* tw, c32* u, c
   SPK_SIZE_SWITCH(resident_rl, tile, ept, tw, u, d, P, Ph, iterations, inv_nn, polls, flag, ll, st)
 }
 
-hipError_t resident_frames(int n, int tile, int ept, int xm, int* out) {
-  SPK_SIZE_SWITCH(resident_frames, tile, ept, xm, out)
+hipError_t resident_frames(int n, int tile, int ept, ResidentForm form, int xm, int* out) {
+  SPK_SIZE_SWITCH(resident_frames, tile, ept, form, xm, out)
 }
 
 hipError_t launch_resident_ipsf(int n, int tile, int ept, const PassArgs& a, const c32* ipsf,

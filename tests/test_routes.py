@@ -60,3 +60,28 @@ for fill in "100":
     assert sum(w[0] == "coop" for w in words) == 1
     assert [w[-1] for w in words if "begin" in w] == [fill], words
 """ % ipsf)
+
+
+def test_a_device_too_small_for_a_resident_launch_runs_the_passes(program):
+    """A resident launch needs all its workgroups on the device at once: 256 at
+    1024^2, 64 at 256^2 (a partition of the device has fewer compute units)."""
+    program("""
+for cus, n, fits in [(64, 1024, False), (255, 1024, False), (256, 1024, True), (64, 256, True),
+                     (63, 256, False), (8, 64, False)]:
+    knob("cus", cus)
+    for resident in (0, 1):
+        for ipsf in (False, True):
+            p = Plan(n, ipsf=ipsf, resident=resident)
+            ok(p.iterate([HIO] * 8))
+            words = launches()
+            assert sum(w[0] == "coop" for w in words) == fits, (cus, n, ipsf, words)
+            assert sum("rowpass" in w[1] for w in words) == (0 if fits else 8)
+            p.close()
+        p = Plan(n, resident=resident)
+        launches()
+        ok(p.coherence(2))
+        words = launches()
+        assert sum(w[0] == "coop" for w in words) == fits, (cus, n, words)
+        assert sum("colpass" in w[1] for w in words) == (3 if fits else 11)
+        p.close()
+""")
