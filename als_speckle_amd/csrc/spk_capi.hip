@@ -185,15 +185,16 @@ struct spk_plan {
   int pgrid = 0;
   // shrinkwraps fused into the passes where possible (spk_tune.sw_separate = 0)
   bool sw_fuse = true;
-  // resident single-frame launches (k_resident) and their exchange mode
+  // resident launches (k_resident, k_resident_ipsf) and their exchange mode
   int resident = 0;            // frames at once, 0: one launch per pass
   int resident_min = 2;        // steps of a block that runs resident
   bool res_allowed = true;     // spk_tune.resident != 2
   int xm = 0;
   int ipsf_fits = -1, rl_fits = -1;   // resident_fits
   int res_xm = 0;              // that of this plan's launches (several frames: 3 or 2)
-  // resident launches: the two exchange buffers of mode 3 (n*n values each),
-  // then the barrier flags (a 128-byte line per band)
+  // resident launches, one allocation: for each frame at once the two exchange
+  // buffers of mode 3 (n*n values each), then the barrier flags of each (a
+  // 128-byte line per band)
   c32* rll = nullptr;
   bool rll_fill = true;   // new, or left unread by a launch that gave up
   unsigned polls = 1u << 18;   // polls of a grid-barrier wait before it gives up
@@ -252,6 +253,16 @@ bool resident_fits(spk_plan* p, ResidentForm form, int* cache) {
     *cache = got && fit > 0;
   }
   return *cache != 0;
+}
+
+// values in the exchange buffers of mode 3, of the frames that a launch runs at once
+size_t exchange_values(const spk_plan* p) {
+  return p->res_xm == 3 ? (size_t)p->resident * 2 * p->nn() : 0;
+}
+// the resident launches' memory, allocated for the first block that can use it;
+// where there is none left the block runs one launch per pass
+bool resident_memory(spk_plan* p) {
+  return p->rll || dalloc(&p->rll, exchange_values(p) + (size_t)p->resident * p->bands * 16) == SPK_OK;
 }
 
 int set_device(spk_ctx* ctx) {
@@ -1230,7 +1241,7 @@ int iter_prepare(spk_plan* p, const spk_step* steps, int nsteps, int per_frame,
         rs.push_back(rsj);
       }
       // an ipsf step saves more: four launches per pass, from 16 us at 64^2
-      if ((int)rs.size() >= (p->ipsf_on ? 2 : p->resident_min)) {
+      if ((int)rs.size() >= (p->ipsf_on ? 2 : p->resident_min) && resident_memory(p)) {
         res_end[k] = k1;
         r.res_n[k] = (int)rs.size();
         r.res_fused[k] = fused;
@@ -1413,12 +1424,8 @@ int iter_step(IterRun& r, int k, int* next) {
   *next = k + 1;
   if (r.res_end[k]) {
     const int k1 = r.res_end[k];
-    // one allocation: the exchange buffers of mode 3, then the barrier flags,
-    // for the frames that a launch runs at once
     const int g = p->resident;
-    const size_t ll = p->res_xm == 3 ? (size_t)g * 2 * p->nn() : 0;
-    if (!p->rll && (rc = dalloc(&p->rll, ll + (size_t)g * p->bands * 16))) return rc;
-    unsigned* rsync = reinterpret_cast<unsigned*>(p->rll + ll);
+    unsigned* rsync = reinterpret_cast<unsigned*>(p->rll + exchange_values(p));
     PassArgs ra = base_args(p);
     ra.swr_tab = r.res_fused[k] ? (const SwParam*)r.dptr(r.res_sw_off[k]) : nullptr;
     const int fill = p->rll_fill;

@@ -85,3 +85,24 @@ for cus, n, fits in [(64, 1024, False), (255, 1024, False), (256, 1024, True), (
         assert sum("colpass" in w[1] for w in words) == (3 if fits else 11)
         p.close()
 """)
+
+
+@pytest.mark.parametrize("n,batch", [(256, 4), (1024, 1), (64, 300)])
+def test_without_memory_for_the_exchange_buffers_the_passes_run(program, n, batch):
+    """A plan that fits the device is not refused for what only its resident form
+    would need, and takes that form once there is room."""
+    program("""
+knob("occupancy", 8 if %d == 64 else 1)
+p = Plan(%d, %d)
+ok(p.iterate([HIO] * p.batch, per_frame=1))   # the step tables' buffers
+launches()
+knob("malloc_limit", fake.fake_live())
+ok(p.iterate([HIO] * 40))
+words = launches()
+assert not any(w[0] == "coop" or "begin" in w for w in words), words
+assert sum("rowpass" in w[1] for w in words) == 40
+knob("malloc_limit", 0)
+ok(p.iterate([HIO] * 40))
+words = launches()
+assert sum(w[0] == "coop" for w in words) == 1 and not any("rowpass" in w[1] for w in words)
+""" % (n, n, batch))
