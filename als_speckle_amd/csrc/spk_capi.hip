@@ -265,6 +265,15 @@ bool resident_memory(spk_plan* p) {
   return p->rll || dalloc(&p->rll, exchange_values(p) + (size_t)p->resident * p->bands * 16) == SPK_OK;
 }
 
+// whether the caller records the stream into a graph of its own (a cooperative
+// launch is left out of it; a stream that cannot be asked counts as recorded)
+bool stream_recorded(hipStream_t st) {
+  hipStreamCaptureStatus s = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &s) == hipSuccess) return s != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();
+  return true;
+}
+
 int set_device(spk_ctx* ctx) {
   SPK_REQUIRE(ctx, SPK_EINVAL, "null context");
   SPK_HIP(hipSetDevice(ctx->device));
@@ -1204,7 +1213,8 @@ int iter_prepare(spk_plan* p, const spk_step* steps, int nsteps, int per_frame,
   // is gathered from all over the frame).
   if (blocks && p->resident && (B == 1 || !per_frame) && !p->spec_on && !p->persist &&
       !p->capturing && (!p->ipsf_on || (B == 1 && p->xm == 3 && p->tile == 4 &&
-                                              resident_fits(p, kResidentIpsf, &p->ipsf_fits)))) {
+                        resident_fits(p, kResidentIpsf, &p->ipsf_fits))) &&
+      !stream_recorded(p->ctx->stream)) {
     auto fits = [&](int j) { return !any_dm[j] && !emits[j]; };
     std::vector<RStep> rs;
     std::vector<SwParam> sp;
@@ -2068,7 +2078,7 @@ int spk_coherence_rl(spk_plan* p, const float* est, int rows, int cols, const fl
   // the updates in one launch where the resident form is built (W and w hold
   // its exchange), otherwise as launches
   const bool one = iterations > 0 && p->res_allowed && p->xm == 3 && tile == 4 && !p->capturing &&
-                   resident_supported(n, tile, p->ept) &&
+                   resident_supported(n, tile, p->ept) && !stream_recorded(st) &&
                    resident_fits(p, kResidentRl, &p->rl_fits);
   if (one)
     SPK_HIP(launch_resident_rl(n, tile, p->ept, p->tw, u, d, P, Ph, iterations, inv_nn, p->polls,

@@ -106,3 +106,16 @@ ok(p.iterate([HIO] * 40))
 words = launches()
 assert sum(w[0] == "coop" for w in words) == 1 and not any("rowpass" in w[1] for w in words)
 """ % (n, n, batch))
+
+
+def test_launches_in_a_callers_capture_are_plain(program):
+    program("""
+p, many = Plan(256), Plan(256, 4)
+ok(p.coherence(2)), ok(many.iterate([HIO] * 8))
+assert sum(w[0] == "coop" for w in launches()) == 2
+knob("capturing", 1)
+ok(p.coherence(2)), ok(many.iterate([HIO] * 8))
+words = launches()
+assert not any(w[0] == "coop" for w in words)
+assert sum("k_colpass" in w[1] for w in words) == 11 + 8
+""")
