@@ -66,7 +66,7 @@ int default_ept(int n, int tile, int batch) {
 }
 
 // Resident launches of several frames (uniform schedules): in exchange mode 3
-// a launch holds 2^20 / n^2 frames at once (2^19 at 64^2); where those are not
+// a launch holds 2^20 / n^2 frames at once (half of that at 64^2); where those are not
 // all and n <= kResidentLeanMax, the lean form holds twice as many (k_resident)
 // and takes the rest in rounds.  They pay up to four rounds, three from 512 up;
 // microseconds per step of all frames on MI355X, one launch per pass / resident:
@@ -77,8 +77,9 @@ int default_ept(int n, int tile, int batch) {
 //   40.6 / 32.3, x 24 54.4 / 47.7, x 28 61.6 / 60.0 (four rounds of 7), x 40
 //   82.7 / 78.6, x 64 125 / 128;  1024^2 x 2 30.1 / 21.5, x 3 36.6 / 32.1.
 int resident_rounds(int n) { return n <= 256 ? 4 : 3; }
-// frames at once by the sizes alone (a 256-CU device): mode 3, lean
-int resident_fit(int n) { return std::max(1, (1 << 20) / (n * n)); }
+// frames at once in mode 3 by the sizes alone (256 CUs of eight wavefronts; a
+// band of 64^2 is half of one)
+int resident_fit(int n) { return std::max(1, (n == 64 ? 1 << 19 : 1 << 20) / (n * n)); }
 // Steps from which a block runs resident by default: a cooperative launch
 // takes about 20 us more than a plain one and the frames' state goes in and
 // out once per round.  Microseconds of a block, per pass / resident: 4 / 8

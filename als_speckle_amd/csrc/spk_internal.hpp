@@ -124,7 +124,7 @@ constexpr int group_tile(int n) {
 }
 constexpr int kGroupEpt = 8;
 
-// One step of a resident single-frame iteration block (k_resident).
+// One step of a resident iteration block (k_resident).
 struct RStep {
   Coef c;          // kActive, kNoOut, kSwRow, kSwFin; coefficients of the update
   int err;         // write this step's error partials
@@ -188,18 +188,17 @@ hipError_t launch_com_partial(const c32* data, int frames, int rows, int cols, d
                               int nblk, hipStream_t st);
 hipError_t launch_roll_sum(const c32* data, int frames, int rows, int cols, const int* shift,
                            c32* out, hipStream_t st);
-// resident single-frame iteration block: one cooperative launch of n/tile
-// workgroups runs nsteps steps with the frame's modulus, support and iterate
-// in registers (k_resident); xm: exchange mode of Phi (0 plain + fences,
-// 1 device-scope + fences, 2 device-scope, no fences, 3 values polled
-// themselves in the two n*n buffers of ll; fill: empty them first, a new
-// pair); `frames` frames of the plan, `at_once` of them at a time (one frame:
-// any exchange mode; several: mode 3, or 2 up to kResidentLeanMax; flags and,
-// in mode 3, ll for each of at_once);
-// errp0[kidx *
-// errp_step + band] gets the error partials of the steps with err set;
-// flags: n/tile * 32 words of barrier flags (zeroed by the launcher); flag:
-// this launch's give-up flag, then the sticky one
+// resident iteration block: one cooperative launch runs nsteps steps of
+// `frames` frames, `at_once` of them at a time by n/tile workgroups each, with
+// a frame's modulus, support and iterate in registers (k_resident).  xm:
+// exchange mode of Phi (0 plain + fences, 1 device-scope + fences, 2
+// device-scope, no fences, 3 values polled themselves); one frame: any,
+// several: mode 3, or 2 up to kResidentLeanMax.  ll: mode 3's two n*n buffers
+// for each of at_once frames; fill: empty them first, they are new or of
+// unknown contents.  errp0[kidx * errp_step + band] gets the error partials of
+// the steps with err set.  flags: n/tile * 32 words of barrier flags for each
+// of at_once frames (zeroed by the launcher); flag: this launch's give-up
+// flag, then the sticky one
 bool resident_supported(int n, int tile, int ept);
 hipError_t launch_resident(int n, int tile, int ept, int xm, const PassArgs& a,
                            const RStep* steps, int nsteps, double* errp0, long long errp_step,

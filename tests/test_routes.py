@@ -119,3 +119,31 @@ words = launches()
 assert not any(w[0] == "coop" for w in words)
 assert sum("k_colpass" in w[1] for w in words) == 11 + 8
 """)
+
+
+def test_plan_bytes_count_the_exchange_that_a_plan_takes(program):
+    """spk_plan_bytes against what a plan and its blocks allocate, at the batches
+    where the resident form changes.  The occupancies are those of a 256-CU
+    device: workgroups per compute unit at 64^2, 128^2, 256^2, 512^2, 1024^2."""
+    program("""
+for n, occupancy in [(64, 8), (128, 8), (256, 4), (512, 2), (1024, 1)]:
+    knob("occupancy", occupancy)
+    fit = 256 * occupancy // (n // 4)
+    for batch in sorted({1, fit - 1, fit, fit + 1, 2 * fit, 2 * fit + 1, 6 * fit, 8 * fit, 8 * fit + 1}):
+        if batch < 1 or batch * n * n > 1 << 23:
+            continue
+        before = fake.fake_live()
+        p = Plan(n, batch)
+        plan = fake.fake_live() - before
+        ok(p.iterate([HIO] * 120))
+        taken = fake.fake_live() - before - plan      # exchange, flags; step tables (64 KB)
+        if any(w[0] == "coop" for w in launches()):
+            taken -= 65536
+        size = ctypes.c_size_t()
+        ok(lib.spk_plan_bytes(n, batch, 1, 0, ctypes.byref(size)))
+        counted = size.value - plan - 65536
+        # flags are counted for the most bands (tile 2); nothing else may differ
+        flags = min(batch, 2 * fit) * (n // 2) * 128
+        assert 0 <= counted - taken <= flags, (n, batch, counted, taken)
+        p.close()
+""")
