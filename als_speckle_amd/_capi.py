@@ -55,6 +55,7 @@ SIGNATURES = {
     "spk_plan_create": (c_int, [c_void_p, c_int, c_int, c_int, POINTER(SpkTune), POINTER(c_void_p)]),
     "spk_plan_destroy": (c_int, [c_void_p]),
     "spk_plan_check": (c_int, [c_void_p]),
+    "spk_plan_set_barrier_polls": (c_int, [c_void_p, c_int]),
     "spk_plan_info": (c_int, [c_void_p, POINTER(c_int), POINTER(c_int), POINTER(c_int)]),
     "spk_plan_sw_counts": (c_int, [c_void_p, POINTER(ctypes.c_longlong),
                                    POINTER(ctypes.c_longlong)]),

@@ -198,7 +198,7 @@ struct spk_plan {
   // 128-byte line per band)
   c32* rll = nullptr;
   bool rll_fill = true;   // new, or left unread by a launch that gave up
-  unsigned polls = 1u << 18;   // polls of a grid-barrier wait before it gives up
+  unsigned polls = 0;          // polls of a wait for other workgroups before it gives up
   long long res_launches = 0, res_steps = 0;
   long long sw_fused_count = 0, sw_separate_count = 0;
   unsigned* pbar = nullptr;
@@ -720,7 +720,7 @@ int spk_plan_create(spk_ctx* ctx, int n, int batch, int shared, const spk_tune* 
       p->resident_min = asked ? 2 : resident_min_steps(n, rounds);
     }
   }
-  p->polls = (tune && tune->barrier_polls > 0) ? (unsigned)tune->barrier_polls : (1u << 18);
+  (void)spk_plan_set_barrier_polls(p, tune ? tune->barrier_polls : 0);
   p->sw_fuse = !(tune && tune->sw_separate > 0);
   const size_t nn = (size_t)n * n;
   const size_t fms = shared ? 1 : (size_t)batch;
@@ -787,6 +787,12 @@ int spk_plan_resident_counts(const spk_plan* p, long long* launches, long long* 
   return SPK_OK;
 }
 
+int spk_plan_set_barrier_polls(spk_plan* p, int polls) {
+  SPK_REQUIRE(p, SPK_EINVAL, "null plan");
+  p->polls = polls > 0 ? (unsigned)polls : 1u << 18;
+  return SPK_OK;
+}
+
 int spk_plan_check(spk_plan* p) {
   SPK_REQUIRE(p, SPK_EINVAL, "null plan");
   int rc = set_device(p->ctx);
@@ -798,8 +804,8 @@ int spk_plan_check(spk_plan* p) {
   if (h[2]) {
     SPK_HIP(hipMemset(p->pbar + 2, 0, sizeof(unsigned)));
     p->rll_fill = true;
-    return fail(SPK_EHIP, "a grid barrier of a resident or persistent launch gave up "
-                          "waiting; results of that launch are invalid");
+    return fail(SPK_EHIP, "a wait of a resident or persistent launch gave up; results of that "
+                          "launch are invalid");
   }
   return SPK_OK;
 }

@@ -200,7 +200,8 @@ class Plan:
         ``_capi.STEP_DTYPE`` array (step-major, frames fastest with per_frame).
 
         Returns a (nsteps, batch) float64 device tensor of modulus errors, or
-        None.  With per_frame, ``steps`` has nsteps * batch entries.
+        None.  With per_frame, ``steps`` has nsteps * batch entries.  Only
+        queues work: ``check`` tells whether a resident launch gave up waiting.
         """
         tab = _capi.step_table(steps)
         nsteps = tab.size // (self.batch if per_frame else 1)
@@ -222,7 +223,7 @@ class Plan:
         return fu.value, se.value
 
     def resident_counts(self) -> tuple[int, int]:
-        """(launches, steps) of the resident single-frame launches so far."""
+        """(launches, steps) of ``iterate``'s resident launches so far."""
         la, st = ctypes.c_longlong(), ctypes.c_longlong()
         check(self.lib.spk_plan_resident_counts(self.handle, byref(la), byref(st)))
         return la.value, st.value
@@ -301,7 +302,9 @@ class Plan:
 
     def coherence_rl(self, estimate: torch.Tensor, modulus: torch.Tensor, iterations: int,
                      semantics: str = "numpy", is_fourier: bool = False) -> torch.Tensor:
-        """Richardson-Lucy ipsf (n x n complex64, not centre-shifted) of one frame."""
+        """Richardson-Lucy ipsf (n x n complex64, not centre-shifted) of one frame.
+        Only queues work: ``check`` tells whether the updates' resident launch
+        gave up waiting (the ipsf is then invalid)."""
         r, c = estimate.shape
         _expect(estimate, torch.complex64, (r, c), self.ctx.device, "estimate")
         _expect(modulus, torch.float32, (self.n, self.n), self.ctx.device, "modulus")
@@ -360,9 +363,14 @@ class Plan:
         check(self.lib.spk_set_spectrum(self.handle, r.ctypes.data, w.ctypes.data, r.size))
 
     def check(self) -> None:
-        """Wait for queued work; raise if a grid barrier of a resident or
-        persistent launch gave up waiting (SpkError, the flag is cleared)."""
+        """Wait for queued work; raise if a wait of a resident launch (``iterate``,
+        ``coherence_rl``) or a persistent block gave up (SpkError, the flag is
+        cleared)."""
         check(self.lib.spk_plan_check(self.handle))
+
+    def set_barrier_polls(self, polls: int) -> None:
+        """The ``barrier_polls`` of later launches (0: library default)."""
+        check(self.lib.spk_plan_set_barrier_polls(self.handle, int(polls)))
 
     def close(self) -> None:
         if getattr(self, "handle", None):

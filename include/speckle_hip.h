@@ -79,8 +79,11 @@ typedef struct spk_tune {
                          it pays (the default: not for blocks of a few steps,
                          many frames), 1: where built, 2: never.  The
                          workgroups of a launch wait for each other: it is a
-                         cooperative launch (spk_plan_check reports a wait
-                         that gave up)                                       */
+                         cooperative launch, taken where the device holds
+                         them all at once.  Cooperative launches of a
+                         process's streams run one after the other; beside
+                         one of another process on the same device a wait
+                         can give up (spk_plan_check reports it)             */
   int32_t exchange;   /* resident launches: how Phi crosses between workgroups,
                          1 plain + barrier with device-scope fences, 2
                          device-scope accesses + fences, 3 device-scope
@@ -121,11 +124,15 @@ int spk_plan_info(const spk_plan* plan, int* tile, int* ept, int* persist);
  * passes and as stand-alone kernels.  No reference counterpart. */
 int spk_plan_sw_counts(const spk_plan* plan, long long* fused, long long* separate);
 
-/* Waits for the plan's queued work and reports whether a grid barrier of a
- * resident launch or a persistent iteration block gave up waiting (SPK_EHIP;
- * the flag is then cleared).  No counterpart in the reference, whose
- * kernels each end with a blocking wait (gpu.py:349). */
+/* Waits for the plan's queued work and reports whether a wait of a resident
+ * launch (of spk_iterate or spk_coherence_rl) or of a persistent iteration
+ * block gave up (SPK_EHIP; the flag is then cleared).  The calls themselves
+ * only queue work and return SPK_OK: a program that fetches their results
+ * checks here first.  No counterpart in the reference, whose kernels each end
+ * with a blocking wait (gpu.py:349). */
 int spk_plan_check(spk_plan* plan);
+/* spk_tune.barrier_polls of the plan's later launches; 0 = default. */
+int spk_plan_set_barrier_polls(spk_plan* plan, int polls);
 
 /* -------------------------------------------------------------------------
  * Plans.  A plan holds `batch` frames of n x n (n a power of two, as pyfft
@@ -202,6 +209,9 @@ int spk_set_spectrum(spk_plan* plan, const float* rescales, const float* weights
  * err_trace: device pointer to nsteps * batch doubles (may be NULL):
  * err_trace[k * batch + f] = sqrt(sum(|F psi_k| - m)^2 / sum m^2) for the
  * iterate psi_k entering step k, accumulated in FP64.
+ * By default runs of steps of one frame, and with per_frame == 0 of several,
+ * are resident launches (spk_tune.resident): spk_plan_check tells whether one
+ * gave up waiting, its results are then invalid.
  * ---------------------------------------------------------------------- */
 int spk_iterate(spk_plan* plan, const spk_step* steps, int nsteps,
                 int per_frame, double* err_trace);
@@ -333,7 +343,10 @@ int spk_rftf_stack(spk_plan* plan, const float* stack_c64, int frames, int rows,
  * `iterations` updates u *= ifft2(fft2(d / ifft2(fft2(u) P)) Ph) from the
  * start Gaussian; ipsf = fft2(u) (real part with SPK_SEM_NUMPY, the CPU
  * branch) / |ipsf(0,0)|, n x n c64 row-major, not centre-shifted.
- * is_fourier: the estimate is a Fourier-space array (the GPU branch). */
+ * is_fourier: the estimate is a Fourier-space array (the GPU branch).
+ * 64^2..1024^2 in tile 4 with spk_tune.resident != 2: the updates are one
+ * resident launch (plain launches in a caller's stream capture);
+ * spk_plan_check tells whether it gave up waiting, ipsf is then invalid. */
 int spk_coherence_rl(spk_plan* plan, const float* estimate_c64, int rows, int cols,
                      const float* modulus, int iterations, int semantics, int is_fourier,
                      float* ipsf_c64);

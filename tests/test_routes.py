@@ -147,3 +147,16 @@ for n, occupancy in [(64, 8), (128, 8), (256, 4), (512, 2), (1024, 1)]:
         assert 0 <= counted - taken <= flags, (n, batch, counted, taken)
         p.close()
 """)
+
+
+def test_exchange_buffers_are_emptied_after_a_reported_give_up(program):
+    program("""
+p = Plan(256)
+fills = []
+for gave_up in (0, 1, 0):
+    ok(p.iterate([HIO] * 8))
+    fills += [w[-1] for w in launches() if "begin" in w]
+    knob("sticky", gave_up)
+    assert lib.spk_plan_check(p.h) == -2 * gave_up
+assert fills == ["1", "0", "1"], fills
+""")
