@@ -922,7 +922,7 @@ int spk_get_psi(spk_plan* p, int frame, float* out) {
   int f0, nf;
   if ((rc = frame_range(p, frame, true, &f0, &nf))) return rc;
   SPK_HIP(launch_unpack_c64(p->n, p->tile, (c32*)out, p->psi + (size_t)f0 * p->nn(), 1.0f, nf,
-                            p->ctx->stream));
+                            p->ctx->stream, p->pbar + 2));
   return SPK_OK;
 }
 
@@ -1539,7 +1539,7 @@ int iter_finish(IterRun& r) {
   spk_plan* p = r.p;
   if (r.err_trace) {
     SPK_HIP(launch_err_finalize(p->errp, r.nsteps, r.B, p->bands, p->summ2, r.err_trace,
-                                (const int*)r.dptr(r.act_off), p->ctx->stream));
+                                (const int*)r.dptr(r.act_off), p->pbar + 2, p->ctx->stream));
   }
   p->phib_g = r.fr;
   return SPK_OK;
@@ -1754,7 +1754,7 @@ static int copy_roi_frames(spk_plan* p, int f0, int nf, float* dst, int slots, i
               SPK_EINVAL, "ROI outside the frame");
   c32* d = (c32*)dst + (size_t)slot * rows * cols;
   SPK_HIP(launch_copy_roi(p->n, p->tile, p->psi + (size_t)f0 * p->nn(), d, r0, c0, rows, cols, nf,
-                          p->ctx->stream));
+                          p->pbar + 2, p->ctx->stream));
   return SPK_OK;
 }
 
@@ -2107,7 +2107,7 @@ int spk_coherence_rl(spk_plan* p, const float* est, int rows, int cols, const fl
   if ((rc = fft2_tiled(p, u, u, cb, false))) return rc;
   SPK_HIP(launch_coh(9, n, tile, u, nullptr, nullptr, nullptr, nullptr, part, 0, 0,
                      semantics == SPK_SEM_NUMPY ? 1.0 : 0.0, 0, st));
-  SPK_HIP(launch_unpack_c64(n, tile, (c32*)ipsf, u, 1.0f, 1, st));
+  SPK_HIP(launch_unpack_c64(n, tile, (c32*)ipsf, u, 1.0f, 1, st, p->pbar + 2));
   return SPK_OK;
 }
 

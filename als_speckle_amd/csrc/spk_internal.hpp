@@ -233,8 +233,11 @@ hipError_t launch_rowfft(int n, int tile, int ept, int mode, const c32* in, c32*
 hipError_t launch_pack_c64(int n, int tile, c32* dst, const c32* src,
                            const float* sup, long long sstride, int frames,
                            hipStream_t st);
+// gave_up: a plan's sticky give-up flag; while it is set the output is NaN (as
+// launch_err_finalize's and launch_copy_roi's).  Null: none
 hipError_t launch_unpack_c64(int n, int tile, c32* dst, const c32* src,
-                             float scale, int frames, hipStream_t st);
+                             float scale, int frames, hipStream_t st,
+                             const unsigned* gave_up = nullptr);
 hipError_t launch_pack_f32(int n, int tile, float* dst, const float* src,
                            int frames, hipStream_t st);
 hipError_t launch_unpack_f32(int n, int tile, float* dst, const float* src,
@@ -247,7 +250,7 @@ hipError_t launch_sumsq(int n, const float* mod, long long mstride,
                         hipStream_t st);
 hipError_t launch_err_finalize(const double* errp, int nsteps, int frames,
                                int bands, const double* summ2, double* trace,
-                               const int* active, hipStream_t st);
+                               const int* active, const unsigned* gave_up, hipStream_t st);
 // frames: fmap[0..frames) with parameters tab[0..frames), or (fmap null)
 // the range frame0.. with p0 (tab null) / tab
 // rmax: the largest blur radius among the frames (<= 47)
@@ -257,7 +260,8 @@ hipError_t launch_shrinkwrap(int n, int tile, const c32* psi, float* sup,
                              const int* fmap, int frame0, int frames, int rmax,
                              hipStream_t st);
 hipError_t launch_copy_roi(int n, int tile, const c32* psi, c32* dst, int r0,
-                           int c0, int rows, int cols, int frames, hipStream_t st);
+                           int c0, int rows, int cols, int frames, const unsigned* gave_up,
+                           hipStream_t st);
 // nblk <= 64
 hipError_t launch_align(c32* data, int frames, long long per_frame,
                         double* partial, int nblk, hipStream_t st);

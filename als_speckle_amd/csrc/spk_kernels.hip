@@ -2401,14 +2401,21 @@ __global__ void __launch_bounds__(256) k_pack_c64(c32* dst, const c32* src, int 
   dst[fo + p] = v;
 }
 
+// What leaves a plan (iterate, regions, traces, ipsf) is NaN while its sticky
+// give-up flag is set: a launch whose workgroups stopped waiting for each other
+// left no valid values.
+__device__ __forceinline__ c32 or_nan(c32 v, const unsigned* gave_up) {
+  return gave_up && *gave_up ? c32{NAN, NAN} : v;
+}
+
 template <int TT>
 __global__ void __launch_bounds__(256) k_unpack_c64(c32* dst, const c32* src, int n,
-                                                    float scl) {
+                                                    float scl, const unsigned* gave_up) {
   const int p = blockIdx.x * 256 + threadIdx.x;
   const size_t fo = (size_t)blockIdx.y * n * n;
   int r, c;
   tile_rc<TT>(n, p, r, c);
-  dst[fo + (size_t)r * n + c] = scale(src[fo + p], scl);
+  dst[fo + (size_t)r * n + c] = or_nan(scale(src[fo + p], scl), gave_up);
 }
 
 template <int TT>
@@ -2487,11 +2494,12 @@ __device__ __forceinline__ void neumaier_add(double& s, double& c, double x) {
 static __global__ void __launch_bounds__(256) k_err_finalize(const double* errp, int nsteps,
                                                              int frames, int bands,
                                                              const double* summ2, double* trace,
-                                                             const int* active) {
+                                                             const int* active,
+                                                             const unsigned* gave_up) {
   const int i = (int)((blockIdx.x * 256u + threadIdx.x) >> 6), lane = threadIdx.x & 63;
   if (i >= nsteps * frames) return;  // whole wavefronts
   const int f = i % frames;
-  if (active && !active[i]) {
+  if ((active && !active[i]) || *gave_up) {
     if (lane == 0) trace[i] = nan("");
     return;
   }
@@ -2629,12 +2637,13 @@ static __global__ void __launch_bounds__(256) k_sw_threshold(float* sup, long lo
 // ---------------------------------------------------------------------------
 template <int TT>
 __global__ void __launch_bounds__(256) k_copy_roi(const c32* psi, c32* dst, int n, int r0,
-                                                  int c0, int rows, int cols) {
+                                                  int c0, int rows, int cols,
+                                                  const unsigned* gave_up) {
   const int k = blockIdx.x * 256 + threadIdx.x;
   if (k >= rows * cols) return;
   const int j = k / cols, i = k % cols;
   dst[(size_t)blockIdx.y * rows * cols + k] =
-      psi[(size_t)blockIdx.y * n * n + tpos<TT>(n, r0 + j, c0 + i)];
+      or_nan(psi[(size_t)blockIdx.y * n * n + tpos<TT>(n, r0 + j, c0 + i)], gave_up);
 }
 
 // ---------------------------------------------------------------------------
@@ -3940,14 +3949,17 @@ hipError_t launch_pack_c64(int n, int tile, c32* dst, const c32* src, const floa
 }
 
 hipError_t launch_unpack_c64(int n, int tile, c32* dst, const c32* src, float scale,
-                             int frames, hipStream_t st) {
+                             int frames, hipStream_t st, const unsigned* gave_up) {
   dim3 grid((unsigned)((size_t)n * n / 256), frames);
   if (tile == 8)
-    hipLaunchKernelGGL(k_unpack_c64<8>, grid, dim3(256), 0, st, dst, src, n, scale);
+    hipLaunchKernelGGL(k_unpack_c64<8>, grid, dim3(256), 0, st, dst, src, n, scale,
+                       gave_up);
   else if (tile == 2)
-    hipLaunchKernelGGL(k_unpack_c64<2>, grid, dim3(256), 0, st, dst, src, n, scale);
+    hipLaunchKernelGGL(k_unpack_c64<2>, grid, dim3(256), 0, st, dst, src, n, scale,
+                       gave_up);
   else
-    hipLaunchKernelGGL(k_unpack_c64<4>, grid, dim3(256), 0, st, dst, src, n, scale);
+    hipLaunchKernelGGL(k_unpack_c64<4>, grid, dim3(256), 0, st, dst, src, n, scale,
+                       gave_up);
   return hipGetLastError();
 }
 
@@ -3999,23 +4011,27 @@ hipError_t launch_sumsq(int n, const float* mod, long long mstride, double* part
 
 hipError_t launch_err_finalize(const double* errp, int nsteps, int frames, int bands,
                                const double* summ2, double* trace, const int* active,
-                               hipStream_t st) {
+                               const unsigned* gave_up, hipStream_t st) {
   const int total = nsteps * frames;  // one wavefront each, four per workgroup
   hipLaunchKernelGGL(k_err_finalize, dim3((total + 3) / 4), dim3(256), 0, st, errp,
-                     nsteps, frames, bands, summ2, trace, active);
+                     nsteps, frames, bands, summ2, trace, active, gave_up);
   return hipGetLastError();
 }
 
 hipError_t launch_copy_roi(int n, int tile, const c32* psi, c32* dst, int r0, int c0,
-                           int rows, int cols, int frames, hipStream_t st) {
+                           int rows, int cols, int frames, const unsigned* gave_up,
+                           hipStream_t st) {
   const int total = rows * cols;
   dim3 grid((total + 255) / 256, frames);
   if (tile == 8)
-    hipLaunchKernelGGL(k_copy_roi<8>, grid, dim3(256), 0, st, psi, dst, n, r0, c0, rows, cols);
+    hipLaunchKernelGGL(k_copy_roi<8>, grid, dim3(256), 0, st, psi, dst, n, r0, c0, rows, cols,
+                       gave_up);
   else if (tile == 2)
-    hipLaunchKernelGGL(k_copy_roi<2>, grid, dim3(256), 0, st, psi, dst, n, r0, c0, rows, cols);
+    hipLaunchKernelGGL(k_copy_roi<2>, grid, dim3(256), 0, st, psi, dst, n, r0, c0, rows, cols,
+                       gave_up);
   else
-    hipLaunchKernelGGL(k_copy_roi<4>, grid, dim3(256), 0, st, psi, dst, n, r0, c0, rows, cols);
+    hipLaunchKernelGGL(k_copy_roi<4>, grid, dim3(256), 0, st, psi, dst, n, r0, c0, rows, cols,
+                       gave_up);
   return hipGetLastError();
 }
 

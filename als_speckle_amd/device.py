@@ -201,7 +201,8 @@ class Plan:
 
         Returns a (nsteps, batch) float64 device tensor of modulus errors, or
         None.  With per_frame, ``steps`` has nsteps * batch entries.  Only
-        queues work: ``check`` tells whether a resident launch gave up waiting.
+        queues work: ``check`` tells whether a resident launch gave up waiting
+        (its results are then NaN).
         """
         tab = _capi.step_table(steps)
         nsteps = tab.size // (self.batch if per_frame else 1)
@@ -304,7 +305,7 @@ class Plan:
                      semantics: str = "numpy", is_fourier: bool = False) -> torch.Tensor:
         """Richardson-Lucy ipsf (n x n complex64, not centre-shifted) of one frame.
         Only queues work: ``check`` tells whether the updates' resident launch
-        gave up waiting (the ipsf is then invalid)."""
+        gave up waiting (the ipsf is then NaN)."""
         r, c = estimate.shape
         _expect(estimate, torch.complex64, (r, c), self.ctx.device, "estimate")
         _expect(modulus, torch.float32, (self.n, self.n), self.ctx.device, "modulus")

@@ -127,8 +127,9 @@ int spk_plan_sw_counts(const spk_plan* plan, long long* fused, long long* separa
 /* Waits for the plan's queued work and reports whether a wait of a resident
  * launch (of spk_iterate or spk_coherence_rl) or of a persistent iteration
  * block gave up (SPK_EHIP; the flag is then cleared).  The calls themselves
- * only queue work and return SPK_OK: a program that fetches their results
- * checks here first.  No counterpart in the reference, whose kernels each end
+ * only queue work and return SPK_OK; from the wait that gave up to this report
+ * what the plan gives out (spk_get_psi, spk_copy_roi, error traces, the ipsf of
+ * spk_coherence_rl) is NaN.  No counterpart in the reference, whose kernels each end
  * with a blocking wait (gpu.py:349). */
 int spk_plan_check(spk_plan* plan);
 /* spk_tune.barrier_polls of the plan's later launches; 0 = default. */
@@ -211,7 +212,7 @@ int spk_set_spectrum(spk_plan* plan, const float* rescales, const float* weights
  * iterate psi_k entering step k, accumulated in FP64.
  * By default runs of steps of one frame, and with per_frame == 0 of several,
  * are resident launches (spk_tune.resident): spk_plan_check tells whether one
- * gave up waiting, its results are then invalid.
+ * gave up waiting, its results are then NaN.
  * ---------------------------------------------------------------------- */
 int spk_iterate(spk_plan* plan, const spk_step* steps, int nsteps,
                 int per_frame, double* err_trace);
@@ -346,7 +347,7 @@ int spk_rftf_stack(spk_plan* plan, const float* stack_c64, int frames, int rows,
  * is_fourier: the estimate is a Fourier-space array (the GPU branch).
  * 64^2..1024^2 in tile 4 with spk_tune.resident != 2: the updates are one
  * resident launch (plain launches in a caller's stream capture);
- * spk_plan_check tells whether it gave up waiting, ipsf is then invalid. */
+ * spk_plan_check tells whether it gave up waiting, ipsf is then NaN. */
 int spk_coherence_rl(spk_plan* plan, const float* estimate_c64, int rows, int cols,
                      const float* modulus, int iterations, int semantics, int is_fourier,
                      float* ipsf_c64);

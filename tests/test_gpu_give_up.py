@@ -1,8 +1,8 @@
 """A resident launch that gave up waiting leaves values in the exchange buffers
 that nobody took.  The plan's next launch must not take them: after the report
 (spk_plan_check asks for emptied buffers) and without it (the launch before
-each resident one sees the flag) it gives the per-pass result, bitwise.  The
-give-up is forced from the host by a poll limit of 1, back to the default after
+each resident one sees the flag) it gives the per-pass result, bitwise.  Up to
+the report everything that leaves the plan is NaN.  The give-up is forced from the host by a poll limit of 1, back to the default after
 it; every kernel ends as always."""
 import pytest
 import torch
@@ -51,17 +51,22 @@ def test_next_launch_after_a_give_up(gpu_ctx, n, batch, ipsf, reported):
     p = plan(gpu_ctx, n, batch, ipsf)
     p.set_barrier_polls(1)
     p.set_psi(crand(shape, 9))
-    p.iterate([HIO] * 100)
+    lost = p.iterate([HIO] * 100)
+    roi = torch.zeros((batch, 9, 11), dtype=torch.complex64, device="cuda")
+    p.copy_roi_all(roi, 0, 3, 5, 9, 11)
+    assert all(x.isnan().all() for x in (lost, p.get_psi(), roi))
     if reported:
         give_up(p)
     p.set_barrier_polls(0)
     p.set_psi(crand(shape, 7))
     got = p.iterate([HIO] * 12)
     assert p.resident_counts() == (2, 112) and ref.resident_counts() == (0, 0)
-    assert torch.equal(got, trace)
-    assert torch.equal(torch.view_as_real(p.get_psi()), torch.view_as_real(ref.get_psi()))
     if not reported:
+        assert got.isnan().all() and p.get_psi().isnan().all()
         give_up(p)
+    else:
+        assert torch.equal(got, trace)
+    assert torch.equal(torch.view_as_real(p.get_psi()), torch.view_as_real(ref.get_psi()))
     p.check()
     p.close(), ref.close()
 
@@ -71,7 +76,7 @@ def test_coherence_updates_report_and_recover(gpu_ctx):
     est, mod = crand((300, 211), 1), rand((n, n), 3) + 0.1
     p, ref = Plan(gpu_ctx, n), Plan(gpu_ctx, n, resident=2)
     p.set_barrier_polls(1)
-    p.coherence_rl(est, mod, 10)
+    assert p.coherence_rl(est, mod, 10).isnan().all()
     give_up(p)
     p.set_barrier_polls(0)
     got = p.coherence_rl(est, mod, 2)
