@@ -90,19 +90,23 @@ class phasing_batch:
         self._seeded = True
 
     def iterate(self, iterations, order=None, beta=0.8, semantics="numpy", error_trace=True):
-        """All trials advance ``iterations`` iterations together."""
+        """All trials advance ``iterations`` iterations together.
+
+        Queues the work and returns.  Should a launch of it give up waiting for
+        its workgroups, the results are NaN and the next call that fetches
+        some (``get_error_trace``, ``get``) raises SpkError.
+        """
         assert self._seeded, "seed() before iterate()"
         sem = _capi.SEM_CODES[semantics]
         steps = [(_capi.ALG_CODES[a], sem, beta, 0.0, 0.0)
                  for a in expand_order(order, iterations)]
-        before = self._plan.resident_counts()[0]
         self._trace = self._plan.iterate(steps, error_trace=error_trace) if steps else None
-        if steps and (self._plan.persist or self._plan.resident_counts()[0] != before):
-            self._plan.check()   # raises if a launch gave up waiting for its workgroups
+        if self._plan.persist and steps:
+            self._plan.check()   # raises if a persistent block's grid barrier gave up
 
     def get_error_trace(self):
         """(iterations, trials) FP64 modulus errors of the last ``iterate``."""
-        return None if self._trace is None else self._trace.cpu().numpy()
+        return None if self._trace is None else self.get(self._trace)
 
     def roi_stack(self) -> torch.Tensor:
         """(trials, rows, cols) device tensor of every trial's ROI (the savebuffer)."""
@@ -121,4 +125,9 @@ class phasing_batch:
         return stack, self.ctx.stack_mean(stack)
 
     def get(self, x):
-        return x.detach().cpu().numpy() if isinstance(x, torch.Tensor) else x
+        if not isinstance(x, torch.Tensor):
+            return x
+        out = x.detach().cpu().numpy()
+        if self._plan is not None:
+            self._plan.check()   # raises if a launch gave up waiting for its workgroups
+        return out

@@ -4,11 +4,13 @@ that nobody took.  The plan's next launch must not take them: after the report
 each resident one sees the flag) it gives the per-pass result, bitwise.  Up to
 the report everything that leaves the plan is NaN.  The give-up is forced from the host by a poll limit of 1, back to the default after
 it; every kernel ends as always."""
+import numpy as np
 import pytest
 import torch
 
 from als_speckle_amd import _capi
 from als_speckle_amd._capi import SpkError
+from als_speckle_amd.batch import phasing_batch
 from als_speckle_amd.device import Plan
 
 pytestmark = pytest.mark.gpu
@@ -83,3 +85,26 @@ def test_coherence_updates_report_and_recover(gpu_ctx):
     p.check()
     assert torch.equal(torch.view_as_real(got), torch.view_as_real(ref.coherence_rl(est, mod, 2)))
     p.close(), ref.close()
+
+
+def test_batched_trials_queue_their_blocks_and_report_where_results_are_fetched(gpu_ctx,
+                                                                                monkeypatch):
+    n, checks = 256, []
+    check = Plan.check
+    monkeypatch.setattr(Plan, "check", lambda self: (checks.append(1), check(self))[1])
+    b = phasing_batch(3, gpu_info=gpu_ctx)
+    sup = np.zeros((n, n), np.float32)
+    sup[90:150, 80:170] = 1
+    b.load((n * rand((n, n), 1)).cpu().numpy(), sup)
+    b.seed(guesses=crand((3, n, n), 3))
+    b.iterate(20)
+    stack, mean = b.aligned_average()
+    assert b._plan.resident_counts()[0] == 1 and not checks
+    assert np.isfinite(b.get_error_trace()).all() and np.isfinite(b.get(mean)).all()
+    b._plan.set_barrier_polls(1)
+    for fetch in (b.get_error_trace, lambda: b.get(b.roi_stack())):
+        b.iterate(100)
+        with pytest.raises(SpkError):
+            fetch()
+    b.iterate(100)
+    assert b.aligned_average()[1].isnan().all()
