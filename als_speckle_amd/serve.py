@@ -199,8 +199,8 @@ class _Chunk:
     def __init__(self, cls, cid, slots):
         self.cls, self.cid, self.slots = cls, cid, slots
         self.n = cls.n
-        # per-pass launches: the size classes run on concurrent streams, and a
-        # resident launch (cooperative, the whole device) must not overlap another
+        # per-pass launches: the size classes run on concurrent streams, where
+        # resident launches (cooperative) would run one after the other
         self.plan = Plan(cls.ctx, cls.n, batch=slots, shared=False, tile=cls.tile, ept=cls.ept,
                          resident=2)
         self.free = list(range(slots))
@@ -291,7 +291,7 @@ class _Class:
         if autotune:
             from .tune import autotune as tune_fn
             with torch.cuda.stream(self.stream):
-                r = tune_fn(self.ctx, n, chunk_slots, shared=False)
+                r = tune_fn(self.ctx, n, chunk_slots, shared=False, resident=2)
             self.tile, self.ept = r.tile, r.ept
         self.chunks = []
         self.next_id = 0

@@ -63,9 +63,10 @@ def _key(ctx, n, batch, shared):
     return f"{name}|n={n}|batch={batch}|shared={int(shared)}"
 
 
-def _time_candidate(ctx, n, batch, shared, tile, ept, persist, iters, m, s, g):
+def _time_candidate(ctx, n, batch, shared, tile, ept, persist, iters, m, s, g, resident):
     hio = (_capi.HIO, _capi.SEM_CODES["numpy"], 0.8, 0.0, 0.0)
-    plan = Plan(ctx, n, batch=batch, shared=shared, tile=tile, ept=ept, persist=persist)
+    plan = Plan(ctx, n, batch=batch, shared=shared, tile=tile, ept=ept, persist=persist,
+                resident=resident)
     try:
         plan.set_modulus(m)
         plan.set_support(s)
@@ -87,14 +88,18 @@ def _time_candidate(ctx, n, batch, shared, tile, ept, persist, iters, m, s, g):
 
 
 def autotune(ctx: Context, n: int, batch: int = 1, shared: bool = True, iters: int = 20,
-             persist: bool = False, cache_path: str | None = None) -> TuneResult:
+             persist: bool = False, cache_path: str | None = None,
+             resident: int = 0) -> TuneResult:
     """Fastest (tile, ept, persist) for `batch` resident n x n frames; the
-    persistent launch mode is a candidate only with persist=True.
+    persistent launch mode is a candidate only with persist=True.  resident: as
+    the plans that will take the shape (2: one launch per pass).
 
     Times `iters` HIO iterations per candidate (best of 3) on a synthetic
     frame; allocates one plan at a time.  The result is cached.
     """
     key = _key(ctx, n, batch, shared) + ("|persist" if persist else "")
+    if resident:
+        key += f"|resident={int(resident)}"
     if key in _cache:
         return _cache[key]
     if cache_path and os.path.exists(cache_path):
@@ -113,7 +118,8 @@ def autotune(ctx: Context, n: int, batch: int = 1, shared: bool = True, iters: i
     g = torch.from_numpy((rng.random(gshape) + 1j * rng.random(gshape)).astype(np.complex64)).to(dev)
     table = []
     for tile, ept, pers in candidates(n, persist):
-        us = _time_candidate(ctx, n, batch, shared, tile, ept, pers, iters, m, s, g) * 1e6
+        us = _time_candidate(ctx, n, batch, shared, tile, ept, pers, iters, m, s, g,
+                             resident) * 1e6
         table.append({"tile": tile, "ept": ept, "persist": pers, "us_per_iter": round(us, 3)})
     best = min(table, key=lambda r: r["us_per_iter"])
     res = TuneResult(tile=best["tile"], ept=best["ept"], persist=best["persist"],
