@@ -310,14 +310,6 @@ SPK_HD int mcol_pos(int band, int b, int t, int i) {
   constexpr int T = N / E;
   return band * N * TT + (t + i * T) * TT + b;
 }
-// row pass: element i of thread t on row b of row-band `band`, in the
-// column-band-major layout (where the row pass writes Phi)
-template <int N, int TT, int E = ept<N, TT>()>
-SPK_HD int cbrow_pos(int band, int b, int t, int i) {
-  constexpr int T = N / E;
-  const int col = t + i * T;
-  return (col / TT) * N * TT + (band * TT + b) * TT + (col % TT);
-}
 
 // Phi's column-band-major copy in the dual layout: bands of at least four
 // columns, so that the row pass of two rows writes 64-byte pieces (4096^2: row
@@ -334,6 +326,22 @@ template <int N, int TT, int E = ept<N, TT>()>
 SPK_HD int dual_col_pos(int band, int b, int t, int i) {
   constexpr int T = N / E, W = TT > 4 ? TT : 4;
   return mcb_pos<W>(N, t + i * T, band * TT + b);
+}
+
+// column pass of four columns (tile 2, bands 2q and 2q + 1): its columns 2b and
+// 2b + 1 of row r as one access, in units of the pair: in the tiled layout,
+// the dual layout's four-column bands and the column-band-major modulus
+template <int N>
+SPK_HD int pair_tile_pos(int q, int b, int r) {
+  return ((r / 2) * (N / 2) + 2 * q + b) * 2 + r % 2;
+}
+template <int N>
+SPK_HD int pair_dual_pos(int q, int b, int r) {
+  return (q * N + r) * 2 + b;
+}
+template <int N>
+SPK_HD int pair_mod_pos(int q, int b, int r) {
+  return (2 * q + b) * N + r;
 }
 
 // LDS slot of element p of transform b (TT transforms per workgroup,

@@ -65,7 +65,7 @@ int fft2_tiled_tw(int inverse, const c32* in, c32* out, const TW& tw) {
     for (int tid = 0; tid < T * TT; ++tid)
       for (int i = 0; i < E; ++i) {
         if constexpr (dual_layout<N>())
-          colband[cbrow_pos<N, TT, E>(band, tid % TT, tid / TT, i)] = x[tid][i];
+          colband[dual_row_pos<N, TT, E>(band, tid % TT, tid / TT, i)] = x[tid][i];
         else
           tiled[row_pos<N, TT, E>(band, tid % TT, tid / TT, i)] = x[tid][i];
       }
@@ -75,7 +75,7 @@ int fft2_tiled_tw(int inverse, const c32* in, c32* out, const TW& tw) {
   for (int band = 0; band < N / TT; ++band) {
     for (int tid = 0; tid < T * TT; ++tid)
       for (int i = 0; i < E; ++i)
-        x[tid][i] = dual_layout<N>() ? colband[mcol_pos<N, TT, E>(band, tid % TT, tid / TT, i)]
+        x[tid][i] = dual_layout<N>() ? colband[dual_col_pos<N, TT, E>(band, tid % TT, tid / TT, i)]
                                      : tiled[col_pos<N, TT, E>(band, tid % TT, tid / TT, i)];
     if (inverse) emu_stages<N, TT, E, true, 0>(x, lds.data(), tw);
     else emu_stages<N, TT, E, false, 0>(x, lds.data(), tw);
