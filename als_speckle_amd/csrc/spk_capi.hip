@@ -181,7 +181,7 @@ struct spk_plan {
   // persistent iteration blocks (k_persist): on/off, co-resident grid size
   // (0 = not queried yet), barrier counter [0], give-up flag of the running
   // launch [1] (cleared with the counter before each launch) and the sticky
-  // give-up flag [2] that spk_plan_check reports and clears
+  // give-up flag [2] that spk_plan_check reports and clears; [3] stays 0
   int persist = 0;
   int pgrid = 0;
   // shrinkwraps fused into the passes where possible (spk_tune.sw_separate = 0)
@@ -1795,7 +1795,7 @@ int spk_fft2(spk_plan* p, const float* in, float* out, int count, int inverse) {
   a.c.flags = kActive;
   SPK_HIP(launch_colpass(p->n, p->tile, p->ept, inverse ? 3 : 2, a, count, 1, st));
   const float scl = inverse ? (float)(1.0 / ((double)p->n * p->n)) : 1.0f;
-  SPK_HIP(launch_unpack_c64(p->n, p->tile, (c32*)out, tiled, scl, count, st));
+  SPK_HIP(launch_unpack_c64(p->n, p->tile, (c32*)out, tiled, scl, count, st, p->pbar + 3));
   return SPK_OK;
 }
 

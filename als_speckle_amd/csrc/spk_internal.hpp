@@ -233,11 +233,11 @@ hipError_t launch_rowfft(int n, int tile, int ept, int mode, const c32* in, c32*
 hipError_t launch_pack_c64(int n, int tile, c32* dst, const c32* src,
                            const float* sup, long long sstride, int frames,
                            hipStream_t st);
-// gave_up: a plan's sticky give-up flag; while it is set the output is NaN (as
-// launch_err_finalize's and launch_copy_roi's).  Null: none
+// gave_up: a plan's sticky give-up flag, or a word that stays 0; while it is set
+// the output is NaN (as launch_err_finalize's and launch_copy_roi's)
 hipError_t launch_unpack_c64(int n, int tile, c32* dst, const c32* src,
                              float scale, int frames, hipStream_t st,
-                             const unsigned* gave_up = nullptr);
+                             const unsigned* gave_up);
 hipError_t launch_pack_f32(int n, int tile, float* dst, const float* src,
                            int frames, hipStream_t st);
 hipError_t launch_unpack_f32(int n, int tile, float* dst, const float* src,

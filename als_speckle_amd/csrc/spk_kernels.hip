@@ -2161,18 +2161,20 @@ __global__ void __launch_bounds__(256) k_pack_c64(c32* dst, const c32* src, int 
 // What leaves a plan (iterate, regions, traces, ipsf) is NaN while its sticky
 // give-up flag is set: a launch whose workgroups stopped waiting for each other
 // left no valid values.
-__device__ __forceinline__ c32 or_nan(c32 v, const unsigned* gave_up) {
-  return gave_up && *gave_up ? c32{NAN, NAN} : v;
+__device__ __forceinline__ c32 or_nan(c32 v, unsigned gave_up) {
+  return gave_up ? c32{NAN, NAN} : v;
 }
 
 template <int TT>
-__global__ void __launch_bounds__(256) k_unpack_c64(c32* dst, const c32* src, int n,
-                                                    float scl, const unsigned* gave_up) {
+__global__ void __launch_bounds__(256) k_unpack_c64(c32* __restrict__ dst,
+                                                    const c32* __restrict__ src, int n, float scl,
+                                                    const unsigned* __restrict__ gave_up) {
+  const unsigned bad = *gave_up;   // scalar, under the load of the value
   const int p = blockIdx.x * 256 + threadIdx.x;
   const size_t fo = (size_t)blockIdx.y * n * n;
   int r, c;
   tile_rc<TT>(n, p, r, c);
-  dst[fo + (size_t)r * n + c] = or_nan(scale(src[fo + p], scl), gave_up);
+  dst[fo + (size_t)r * n + c] = or_nan(scale(src[fo + p], scl), bad);
 }
 
 template <int TT>
@@ -2250,17 +2252,20 @@ __device__ __forceinline__ void neumaier_add(double& s, double& c, double x) {
 // the result does not depend on the launch shape.
 static __global__ void __launch_bounds__(256) k_err_finalize(const double* errp, int nsteps,
                                                              int frames, int bands,
-                                                             const double* summ2, double* trace,
+                                                             const double* summ2,
+                                                             double* __restrict__ trace,
                                                              const int* active,
-                                                             const unsigned* gave_up) {
+                                                             const unsigned* __restrict__ gave_up) {
   const int i = (int)((blockIdx.x * 256u + threadIdx.x) >> 6), lane = threadIdx.x & 63;
   if (i >= nsteps * frames) return;  // whole wavefronts
   const int f = i % frames;
-  if ((active && !active[i]) || *gave_up) {
+  if (active && !active[i]) {
     if (lane == 0) trace[i] = nan("");
     return;
   }
   const double* v = errp + (size_t)i * bands;
+  // (a vector load beside the partials': a scalar one is waited for on its own)
+  const unsigned bad = __hip_atomic_load(gave_up, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
   double s = 0.0, c = 0.0;
   for (int b = lane; b < bands; b += 64) neumaier_add(s, c, v[b]);
   const double mine = s + c;
@@ -2269,7 +2274,7 @@ static __global__ void __launch_bounds__(256) k_err_finalize(const double* errp,
     const double x = __shfl(mine, l, 64);
     neumaier_add(S, C, x);
   }
-  if (lane == 0) trace[i] = sqrt((S + C) / summ2[f]);
+  if (lane == 0) trace[i] = bad ? nan("") : sqrt((S + C) / summ2[f]);
 }
 
 // ---------------------------------------------------------------------------
@@ -2393,14 +2398,16 @@ static __global__ void __launch_bounds__(256) k_sw_threshold(float* sup, long lo
 // apart), 206 us of kernels; one takes 13 us.
 // ---------------------------------------------------------------------------
 template <int TT>
-__global__ void __launch_bounds__(256) k_copy_roi(const c32* psi, c32* dst, int n, int r0,
-                                                  int c0, int rows, int cols,
-                                                  const unsigned* gave_up) {
+__global__ void __launch_bounds__(256) k_copy_roi(const c32* __restrict__ psi,
+                                                  c32* __restrict__ dst, int n, int r0, int c0,
+                                                  int rows, int cols,
+                                                  const unsigned* __restrict__ gave_up) {
+  const unsigned bad = *gave_up;
   const int k = blockIdx.x * 256 + threadIdx.x;
   if (k >= rows * cols) return;
   const int j = k / cols, i = k % cols;
   dst[(size_t)blockIdx.y * rows * cols + k] =
-      or_nan(psi[(size_t)blockIdx.y * n * n + tpos<TT>(n, r0 + j, c0 + i)], gave_up);
+      or_nan(psi[(size_t)blockIdx.y * n * n + tpos<TT>(n, r0 + j, c0 + i)], bad);
 }
 
 // ---------------------------------------------------------------------------
