@@ -187,9 +187,10 @@ struct spk_plan {
   // shrinkwraps fused into the passes where possible (spk_tune.sw_separate = 0)
   bool sw_fuse = true;
   // resident launches (k_resident, k_resident_ipsf) and their exchange mode
-  int resident = 0;            // frames at once, 0: one launch per pass
+  int res_mode = 0;            // spk_tune.resident
+  bool res_asked = false;      // the form or its exchange was asked for
+  int resident = -1;           // frames at once, 0: one launch per pass, -1: see resident_form
   int resident_min = 2;        // steps of a block that runs resident
-  bool res_allowed = true;     // spk_tune.resident != 2
   int xm = 0;
   int ipsf_fits = -1, rl_fits = -1;   // resident_fits
   int res_xm = 0;              // that of this plan's launches (several frames: 3 or 2)
@@ -256,6 +257,44 @@ bool resident_fits(spk_plan* p, ResidentForm form, int* cache) {
   return *cache != 0;
 }
 
+// Whether the plan's blocks run resident, decided with the first one (the
+// occupancy query loads the size's kernels).  By default where the form is
+// built and pays: one frame of 64^2 to 1024^2 takes about half the time of one
+// launch per pass on MI355X, several see resident_rounds; the exchange of Phi
+// by polled values is the default (the barrier forms are slower, the fenced
+// ones most).
+bool resident_form(spk_plan* p) {
+  if (p->resident >= 0) return p->resident > 0;
+  p->resident = 0;
+  const int n = p->n, batch = p->batch;
+  if (p->res_mode == 2 || !resident_supported(n, p->tile, p->ept)) return false;
+  auto frames = [&](ResidentForm form, int xm) {
+    int fit = 0;
+    if (resident_frames(n, p->tile, p->ept, form, xm, &fit) == hipSuccess) return fit;
+    (void)hipGetLastError();
+    return 0;
+  };
+  int fit = 0;
+  p->res_xm = p->xm;
+  if (batch == 1) {
+    fit = frames(kResidentOne, p->xm);
+  } else if (p->xm == 3 &&
+             (p->res_mode == 1 || batch <= resident_rounds(n) * 2 * resident_fit(n))) {
+    fit = frames(kResidentMany, 3);
+    // more than one round of mode 3: the lean form's
+    if (fit && batch > fit && n <= kResidentLeanMax) {
+      p->res_xm = 2;
+      fit = frames(kResidentMany, 2);
+    }
+  }
+  const int rounds = fit ? (batch + fit - 1) / fit : 0;
+  if (rounds && (rounds <= resident_rounds(n) || p->res_mode == 1)) {
+    p->resident = (batch + rounds - 1) / rounds;   // as even as they go
+    // a caller that asks for the form or its exchange gets it for any block
+    p->resident_min = p->res_asked ? 2 : resident_min_steps(n, rounds);
+  }
+  return p->resident > 0;
+}
 // values in the exchange buffers of mode 3, of the frames that a launch runs at once
 size_t exchange_values(const spk_plan* p) {
   return p->res_xm == 3 ? (size_t)p->resident * 2 * p->nn() : 0;
@@ -687,39 +726,9 @@ int spk_plan_create(spk_ctx* ctx, int n, int batch, int shared, const spk_tune* 
   p->bands = n / tile;
   p->persist = (tune && tune->persist > 0) ? 1 : 0;
   p->phib_g.assign(batch, 0.0f);
-  // resident launches by default where they are built and pay: one frame of
-  // 64^2 to 1024^2 takes about half the time of one launch per pass on
-  // MI355X, several see resident_rounds; the exchange of Phi by polled values
-  // is the default (the barrier forms are slower, the fenced ones most)
   p->xm = (tune && tune->exchange >= 1 && tune->exchange <= 4) ? tune->exchange - 1 : 3;
-  const int res_mode = tune ? tune->resident : 0;
-  p->res_allowed = res_mode != 2;
-  if (res_mode != 2 && resident_supported(n, tile, ept)) {
-    int fit = 0;
-    // (the occupancy query only where the answer can matter)
-    const bool few = batch <= resident_rounds(n) * 2 * resident_fit(n);
-    p->res_xm = p->xm;
-    if (batch == 1) {
-      if (resident_frames(n, tile, ept, kResidentOne, p->xm, &fit) != hipSuccess) fit = 0;
-    } else {
-      if (p->xm != 3 || !(few || res_mode == 1) ||
-          resident_frames(n, tile, ept, kResidentMany, 3, &fit) != hipSuccess)
-        fit = 0;
-      // more than one round of mode 3: the lean form's
-      if (fit && batch > fit && n <= kResidentLeanMax) {
-        p->res_xm = 2;
-        if (resident_frames(n, tile, ept, kResidentMany, 2, &fit) != hipSuccess) fit = 0;
-      }
-    }
-    (void)hipGetLastError();   // a query that failed is no error of this call
-    const int rounds = fit ? (batch + fit - 1) / fit : 0;
-    if (rounds && (rounds <= resident_rounds(n) || res_mode == 1)) {
-      p->resident = (batch + rounds - 1) / rounds;   // as even as they go
-      // a caller that asks for the form or its exchange gets it for any block
-      const bool asked = res_mode == 1 || (tune && tune->exchange > 0);
-      p->resident_min = asked ? 2 : resident_min_steps(n, rounds);
-    }
-  }
+  p->res_mode = tune ? tune->resident : 0;
+  p->res_asked = p->res_mode == 1 || (tune && tune->exchange > 0);
   (void)spk_plan_set_barrier_polls(p, tune ? tune->barrier_polls : 0);
   p->sw_fuse = !(tune && tune->sw_separate > 0);
   const size_t nn = (size_t)n * n;
@@ -1218,11 +1227,13 @@ int iter_prepare(spk_plan* p, const spk_step* steps, int nsteps, int per_frame,
   // With an ipsf the block is k_resident_ipsf's (tile 4, exchange mode 3), and
   // ends at every shrinkwrap; with a spectrum there is none (the rescaled map
   // is gathered from all over the frame).
-  if (blocks && p->resident && (B == 1 || !per_frame) && !p->spec_on && !p->persist &&
-      !p->capturing && (!p->ipsf_on || (B == 1 && p->xm == 3 && p->tile == 4 &&
-                        resident_fits(p, kResidentIpsf, &p->ipsf_fits))) &&
-      !stream_recorded(p->ctx->stream)) {
-    auto fits = [&](int j) { return !any_dm[j] && !emits[j]; };
+  auto fits = [&](int j) { return !any_dm[j] && !emits[j]; };
+  bool any_fits = false;
+  for (int k = 0; k < nsteps; ++k) any_fits |= fits(k);
+  if (blocks && any_fits && (B == 1 || !per_frame) && !p->spec_on && !p->persist &&
+      !p->capturing && p->resident != 0 && !stream_recorded(p->ctx->stream) && resident_form(p) &&
+      (!p->ipsf_on || (B == 1 && p->xm == 3 && p->tile == 4 &&
+                       resident_fits(p, kResidentIpsf, &p->ipsf_fits)))) {
     std::vector<RStep> rs;
     std::vector<SwParam> sp;
     for (int k = 0; k < nsteps;) {
@@ -1337,7 +1348,6 @@ int iter_prepare(spk_plan* p, const spk_step* steps, int nsteps, int per_frame,
   r.block_end.assign(nsteps, 0);
   r.block_off.assign(nsteps, 0);
   if (blocks && p->persist && !p->ipsf_on && !p->spec_on) {
-    auto fits = [&](int j) { return !any_dm[j] && !emits[j]; };
     for (int k = 0; k < nsteps;) {
       if (!fits(k)) { ++k; continue; }
       int k1 = k;
@@ -2084,7 +2094,7 @@ int spk_coherence_rl(spk_plan* p, const float* est, int rows, int cols, const fl
   SPK_HIP(launch_coh(7, n, tile, nullptr, nullptr, u, nullptr, nullptr, nullptr, 0, 0, w0, w0, st));
   // the updates in one launch where the resident form is built (W and w hold
   // its exchange), otherwise as launches
-  const bool one = iterations > 0 && p->res_allowed && p->xm == 3 && tile == 4 && !p->capturing &&
+  const bool one = iterations > 0 && p->res_mode != 2 && p->xm == 3 && tile == 4 && !p->capturing &&
                    resident_supported(n, tile, p->ept) && !stream_recorded(st) &&
                    resident_fits(p, kResidentRl, &p->rl_fits);
   if (one)

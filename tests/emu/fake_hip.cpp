@@ -44,6 +44,7 @@ int launch(const char* how, const void* f, Dim g, Dim b, void** args) {
 
 extern "C" {
 void fake_set(const char* name, long long v) { knob[name] = v; }
+long long fake_get(const char* name) { return knob[name]; }
 const char* fake_log() { return log_text.c_str(); }
 void fake_clear() { log_text.clear(); }
 unsigned long long fake_live() { return live; }
@@ -118,6 +119,7 @@ int hipMemsetAsync(void* d, int v, size_t n, void*) { std::memset(d, v, n); retu
 int hipGetSymbolAddress(void** p, const void*) { static char sym[1 << 20]; *p = sym; return 0; }
 
 int hipOccupancyMaxActiveBlocksPerMultiprocessor(int* n, const void* f, int, size_t) {
+  ++knob["queries"];
   *n = (int)(names[f].find(",2,true>") != std::string::npos ? 2 * knob["occupancy"]
                                                              : knob["occupancy"]);
   return 0;

@@ -10,6 +10,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.dirname(os.path.abspath(__file__)
 fake = ctypes.CDLL(sys.argv[1], ctypes.RTLD_GLOBAL)
 fake.fake_log.restype = ctypes.c_char_p
 fake.fake_live.restype = ctypes.c_ulonglong
+fake.fake_get.restype = ctypes.c_longlong
 spec = importlib.util.spec_from_file_location(
     "_capi", os.path.join(ROOT, "als_speckle_amd", "_capi.py"))
 capi = importlib.util.module_from_spec(spec)

@@ -160,3 +160,21 @@ for gave_up in (0, 1, 0):
     assert lib.spk_plan_check(p.h) == -2 * gave_up
 assert fills == ["1", "0", "1"], fills
 """)
+
+
+def test_a_plan_asks_for_occupancies_with_its_first_block(program):
+    """The first question about a size's kernels loads them (5 ms): a plan that
+    runs no block of steps does not ask, one that does asks once."""
+    program("""
+for n, batch in [(1024, 1), (256, 4), (256, 20), (4096, 1)]:
+    knob("queries", 0)
+    p = Plan(n, batch)
+    ok(p.iterate([DM]))
+    assert fake.fake_get(b"queries") == 0, (n, batch)
+    ok(p.iterate([HIO] * 20))
+    asked = fake.fake_get(b"queries")
+    assert (asked > 0) == (n < 2048)
+    ok(p.iterate([HIO] * 20))
+    assert fake.fake_get(b"queries") == asked
+    p.close()
+""")
