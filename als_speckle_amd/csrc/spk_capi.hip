@@ -234,8 +234,8 @@ struct spk_plan {
   // Start of the plan's k-th array in its allocation.  A pass streams several
   // arrays at the same index; allocations are aligned far beyond the memory
   // channels' interleave, so at 4096^2 the streams' accesses meet in the same
-  // channels: 1 KB from one array to the next takes an iteration from 228 to
-  // 218 us (two frames 538 to 522; 256 bytes: no change; more: no further
+  // channels: 1 KB from one array to the next takes an iteration from 226 to
+  // 216 us (two frames 538 to 522; 256 bytes: no change; more: no further
   // gain).  At 2048^2 and below it changes nothing (49.2 us either way).
   size_t skew(int k) const { return dual() ? (size_t)k * 1024 : 0; }
   c32* phi_in() const { return dual() ? phic : phi; }    // column pass input

@@ -313,9 +313,11 @@ SPK_HD int mcol_pos(int band, int b, int t, int i) {
 
 // Phi's column-band-major copy in the dual layout: bands of at least four
 // columns, so that the row pass of two rows writes 64-byte pieces (4096^2: row
-// pass 158 -> 127 us with 64-byte instead of 32-byte pieces; the column pass of
-// two columns reads half of each piece and its neighbour, on the same XCD, the
-// other half from the L2).  Row pass: row b of row-band `band`, column t + i T.
+// pass 158 -> 127 us with 64-byte instead of 32-byte pieces; a column pass of
+// two columns, which the steps with a shrinkwrap, an ipsf or a spectrum run,
+// reads half of each piece and its neighbour, on the same XCD, the other half
+// from the L2: with a shrinkwrap 200 -> 205-210 us, which its row passes win back,
+// 418 -> 416 us per iteration; with an ipsf 646 -> 560).  Row pass: row b of row-band `band`, column t + i T.
 template <int N, int TT, int E = ept<N, TT>()>
 SPK_HD int dual_row_pos(int band, int b, int t, int i) {
   constexpr int T = N / E, W = TT > 4 ? TT : 4;

@@ -437,7 +437,7 @@ class phasing:
                 print("  iteration %s" % stop)
                 sys.stdout.flush()
         if self._plan.resident_counts()[0] != resident_before:
-            # resident launches wait at grid barriers: raise if one gave up
+            # a resident launch's workgroups wait for each other: raise if one gave up
             # (the reference's iterate blocks on its kernels, gpu.py:349)
             self._plan.check()
         if error_trace and traces:
